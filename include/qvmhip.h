@@ -261,6 +261,13 @@ QVMHIP_API int qvmhip_copy(qvmhip_state *dst, const qvmhip_state *src);
 /* dst += src elementwise, same n/dtype: the running sum of the Kraus-list
  * evolution of a density matrix (map-into sum #'+, src/apply-gate.lisp:76-96). */
 QVMHIP_API int qvmhip_accumulate(qvmhip_state *dst, const qvmhip_state *src);
+/* rho -> sum_j K_j rho K_j^H on qubits[0..k-1] (< nq, nat-tuple order) of
+ * the density matrix vec(rho) held row-major in a 2*nq-qubit state: the Kraus
+ * loop of apply-gate-to-state on density states (src/apply-gate.lisp:66-99) as
+ * one sweep with the map's superoperator.  K: `count` 2^k x 2^k matrices,
+ * 1 <= k <= 3; count = 1 is a unitary gate (src/apply-gate.lisp:40-65). */
+QVMHIP_API int qvmhip_density_apply_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, uint32_t k,
+                                          const uint32_t *qubits);
 /* For a 2*nq-qubit state holding vec(rho) row-major (rho[i][j] at i*2^nq + j):
  * out[i] = Re rho[i][i], i < 2^nq.  density-matrix-state-measurement-
  * probabilities (src/state-representation.lisp:268-286) and the diagonal of

@@ -28,6 +28,7 @@ SOURCES = {
     "tile.hip": ["-ffp-contract=off"],
     "reduce.hip": ["-ffp-contract=off"],
     "fused.hip": [],
+    "channel.hip": ["-ffp-contract=off"],
     "program.hip": [],
     "mlp.hip": [],
     "batch.hip": [],

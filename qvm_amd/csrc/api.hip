@@ -26,7 +26,6 @@ using namespace qvmhip;
 
 namespace {
 
-constexpr size_t kMatSlot = 128 * 1024;
 constexpr size_t kStageBytes = size_t(64) << 20;
 
 uint64_t scratch_bytes(uint32_t n) {
@@ -250,9 +249,25 @@ int qvmhip_apply_fused(qvmhip_state *s, const double *U, uint32_t k, const uint3
     if (!U || !finite_matrix(U, k)) return fail(QVMHIP_EINVAL, "matrix is null or not finite");
     // upload to the matrix slot's second half (first half: ops / dense)
     const size_t bytes = sizeof(double) * 2 * (size_t(1) << (2 * k));
-    void *dst = (char *)s->mat + kMatSlot / 2;
+    void *dst = (char *)s->mat + kFusedMatOffset;
     QH_CHECK(hipMemcpyAsync(dst, U, bytes, hipMemcpyHostToDevice, s->stream));
     return launch_fused_dense(s, dst, k, qubits);
+}
+
+int qvmhip_density_apply_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, uint32_t k,
+                               const uint32_t *qubits) {
+    if (!s) return fail(QVMHIP_EINVAL, "null state");
+    if (2 * nq != s->n) return fail(QVMHIP_EINVAL, "a density state of nq qubits has 2*nq qubits");
+    if (k < 1 || k > 3 || k > nq) return fail(QVMHIP_EINVAL, "Kraus operators act on 1..3 qubits of the density state");
+    int rc = check_qubits(s, k, qubits);
+    if (rc) return rc;
+    for (uint32_t i = 0; i < k; ++i)
+        if (qubits[i] >= nq) return fail(QVMHIP_EINVAL, "qubit out of range for the density state");
+    if (!K || count < 1) return fail(QVMHIP_EINVAL, "no Kraus operators");
+    for (uint32_t j = 0; j < count; ++j)
+        if (!finite_matrix(K + j * (size_t(2) << (2 * k)), k)) return fail(QVMHIP_EINVAL, "matrix is not finite");
+    DeviceScope ds(s->device);
+    return launch_kraus(s, nq, K, count, k, qubits);
 }
 
 int qvmhip_apply_tile_pass(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, uint32_t nops,

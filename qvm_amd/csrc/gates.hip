@@ -1117,6 +1117,10 @@ int launch_gate(qvmhip_state *s, const double *U, uint32_t k, const uint32_t *qu
     return run_split<float>(s, gs);
 }
 
+bool gate_is_dense(const double *U, uint32_t k, const uint32_t *qubits) {
+    return split_gate(reinterpret_cast<const cd *>(U), k, qubits, true).kind == 1;
+}
+
 int launch_diagonal(qvmhip_state *s, const double *d, uint32_t k, const uint32_t *qubits) {
     const uint32_t D = 1u << k;
     std::vector<cd> U((size_t)D * D, cd(0, 0));

@@ -23,6 +23,8 @@ constexpr int kRedBlocks = 2048;    // partial sums of one reduction launch
 constexpr int kChunkLog2 = 8;       // sampling chunk: 256 amplitudes
 // A dispatch holds at most 2^32 work-items; sweep kernels cap their grid at
 // 2^22 workgroups and grid-stride over the rest (34-qubit states).
+constexpr size_t kMatSlot = 128 * 1024;           // device matrix slot of a state
+constexpr size_t kFusedMatOffset = kMatSlot / 2;  // its second half: matrices of fused blocks
 constexpr uint64_t kMaxGrid = uint64_t(1) << 22;
 
 // Workgroups of a dispatch go to the 8 XCDs round robin: workgroup b runs on
@@ -229,6 +231,9 @@ inline void prof_end(qvmhip_state *s) {
 
 // Launch helpers implemented in the kernel files.
 int launch_gate(qvmhip_state *s, const double *U, uint32_t k, const uint32_t *qubits, int force_dense);
+bool gate_is_dense(const double *U, uint32_t k, const uint32_t *qubits);  // neither diagonal nor a permutation
+// sum_j K_j rho K_j^H on the density matrix of nq qubits held in s, 1 <= k <= 3
+int launch_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, uint32_t k, const uint32_t *qubits);
 int launch_diagonal(qvmhip_state *s, const double *d, uint32_t k, const uint32_t *qubits);
 int launch_permutation(qvmhip_state *s, const uint32_t *perm, uint32_t k, const uint32_t *qubits);
 int launch_fill_zero_state(qvmhip_state *s);

@@ -5,11 +5,13 @@ methods of the state protocol: an n-qubit density matrix rho is held as
 vec(rho), row-major (rho[i][j] at index i * 2^n + j), in a 2n-qubit engine
 state, so every operation is one of the pure-state kernels:
 
-    gate U on qubits q          U* on q, then U on the ghosts q + n
+    gate U on qubits q          U* on q and U on the ghosts q + n
                                 (vec(A rho B) = (A (x) B^T) vec(rho),
                                 src/apply-gate.lisp:40-65)
-    Kraus list {K_j}            sum_j (K_j (x) K_j*) vec(rho): a pristine copy,
-                                a device running sum (qvmhip_accumulate)
+    Kraus list {K_j}            sum_j (K_j (x) K_j*) vec(rho): one sweep with the
+                                map's superoperator (qvmhip_density_apply_kraus,
+                                up to 3 qubits), else a pristine copy and a
+                                device running sum (qvmhip_accumulate)
                                 (src/apply-gate.lisp:66-99)
     measurement probabilities   the diagonal Re rho[i][i] (qvmhip_density_diagonal,
                                 src/state-representation.lisp:268-286)
@@ -150,6 +152,12 @@ class DensityQVM:
         """rho -> sum_j K_j rho K_j^H on the Quil-ordered qubits."""
         ops = [np.asarray(k, dtype=np.complex128) for k in kraus_ops]
         if not ops:
+            return
+        k = len(quil_qubits)
+        if 1 <= k <= (2 if len(ops) == 1 else 3):
+            # one sweep with the map's superoperator.  A 3-qubit unitary stays
+            # two sweeps: its 64x64 superoperator is bound by the matrix cores
+            self.state.density_apply_kraus(self.number_of_qubits, np.stack(ops), G.nat_tuple(*quil_qubits))
             return
         if len(ops) == 1:
             self._apply_single(ops[0], quil_qubits)

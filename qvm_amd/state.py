@@ -273,6 +273,17 @@ class HipPureState:
         """self += other, elementwise."""
         N.check(N.lib().qvmhip_accumulate(self._h, other._h))
 
+    def density_apply_kraus(self, nq: int, kraus_ops, qubits) -> None:
+        """rho -> sum_j K_j rho K_j^H on ``qubits`` (nat-tuple order) of the
+        nq-qubit density matrix this 2*nq-qubit state holds, in one sweep."""
+        q = N.u32arr(qubits)
+        k = len(q)
+        K = N.cmat(kraus_ops)
+        if K.shape[1:] != (1 << k, 1 << k):
+            raise ValueError(f"matrix shape {K.shape[1:]} does not match {k} qubits")
+        N.check(N.lib().qvmhip_density_apply_kraus(self._h, int(nq), N.dptr(K.view(np.float64)), len(K), k,
+                                                   N.u32ptr(q)))
+
     def density_diagonal(self, nq: int) -> np.ndarray:
         """Re rho[i][i] of the density matrix this 2*nq-qubit state holds
         as vec(rho), row-major."""
