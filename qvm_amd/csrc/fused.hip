@@ -513,7 +513,8 @@ int run_fused(qvmhip_state *s, const void *mat_dev, const uint32_t *qubits) {
     // the 30-qubit layered + QFT circuits in k = 4 / 5 blocks took 1176 /
     // 830 ms against 1119 / 786 ms cached.
     const uint32_t line_bits = sizeof(T) == 8 ? 3u : 4u;
-    bool ntm = sizeof(T) == 8;
+    const bool stream = stream_accesses(s);
+    bool ntm = sizeof(T) == 8 && stream;
     for (int b = 2; b < K; ++b)
         if (pos[b] < line_bits) ntm = false;
     int ncu = 0;
@@ -526,8 +527,12 @@ int run_fused(qvmhip_state *s, const void *mat_dev, const uint32_t *qubits) {
             const uint64_t ncb = g.ngroups / 32;
             const uint32_t grid2 = (uint32_t)std::min<uint64_t>((ncb + 3) / 4, (uint64_t)per_cu_rows2 * (uint64_t)ncu);
             prof_begin(s, QVMHIP_K_FUSED);
-            hipLaunchKernelGGL((k_fused_rows2<T, K, true>), dim3(grid2), dim3(256), 0, s->stream,
-                               (vec2_t<T> *)s->amps, (const double *)mat_dev, g, off);
+            if (stream)
+                hipLaunchKernelGGL((k_fused_rows2<T, K, true>), dim3(grid2), dim3(256), 0, s->stream,
+                                   (vec2_t<T> *)s->amps, (const double *)mat_dev, g, off);
+            else
+                hipLaunchKernelGGL((k_fused_rows2<T, K, false>), dim3(grid2), dim3(256), 0, s->stream,
+                                   (vec2_t<T> *)s->amps, (const double *)mat_dev, g, off);
             prof_end(s);
             QH_LAUNCH_CHECK();
             return QVMHIP_OK;
@@ -545,7 +550,7 @@ int run_fused(qvmhip_state *s, const void *mat_dev, const uint32_t *qubits) {
         if (g.ngroups >= 64 && pos[0] >= line_bits) {
             static std::atomic<int> rows_cache{0};
             const int per_cu_rows = resident_per_cu(rows_cache, k_fused_rows<T, K, false>);
-            const bool nt_rows = sizeof(T) == 8;
+            const bool nt_rows = sizeof(T) == 8 && stream;
             const uint64_t ncb = g.ngroups / 64;
             const uint32_t grid_rows =
                 (uint32_t)std::min<uint64_t>((ncb + 3) / 4, (uint64_t)per_cu_rows * (uint64_t)ncu);

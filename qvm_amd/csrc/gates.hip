@@ -68,6 +68,35 @@ struct SparseArgs {
 
 // ---------------------------------------------------------------------------
 // Kernels.
+//
+// NTM (all sweep kernels): the amplitudes are loaded and stored non-temporal.
+// The host asks for it when the state is too large to stay in the Infinity
+// Cache (stream_accesses); a gate on a smaller state finds it there.
+
+// two FP32 amplitudes as one 16-byte access
+typedef float F4 __attribute__((ext_vector_type(4)));
+
+// Stores a whole line's share where only some lanes change their amplitude.
+// A plain store of a value the thread has just loaded from there would be
+// dropped by the compiler, and the partial lines that are left write at half
+// the rate (SWAP and CNOT below bit 6 at 2^24 FP64 amplitudes: 163 us against 84).
+template <bool NTM, typename V>
+__device__ __forceinline__ void stg_whole(V *p, V x) {
+    if constexpr (!NTM) asm volatile("" : "+v"(x.x), "+v"(x.y));
+    stg<NTM>(p, x);
+}
+
+template <bool NTM>
+__device__ __forceinline__ F4 ld4(const F4 *p) {
+    if constexpr (NTM) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+
+template <bool NTM>
+__device__ __forceinline__ void st4(F4 *p, const F4 &v) {
+    if constexpr (NTM) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
 
 // Dense k-qubit operator, k <= 3, one complement group per thread, GPT groups
 // per thread kept in flight.  Consecutive threads take consecutive groups, so
@@ -146,18 +175,18 @@ __device__ __forceinline__ vec2_t<T> dense1_row(const vec2_t<T> &lo, const vec2_
 
 // q < 6: the partner (index i ^ 2^q) is in the same wavefront; a lane shuffle
 // brings it.  len is a multiple of kBlock, so every lane of every wave is live.
-template <typename T>
+template <typename T, bool NTM>
 __global__ __launch_bounds__(kBlock) void k_dense1_lane(vec2_t<T> *__restrict__ psi, uint64_t len, uint32_t q,
                                                         const Dense1Coef<T> u) {
     using V = vec2_t<T>;
     const uint64_t step = (uint64_t)gridDim.x * kBlock;
     for (uint64_t i = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x; i < len; i += step) {
-        const V x = ldg<true>(&psi[i]);
+        const V x = ldg<NTM>(&psi[i]);
         V p;
         p.x = __shfl_xor(x.x, 1 << q, 64);
         p.y = __shfl_xor(x.y, 1 << q, 64);
         const uint32_t r = (uint32_t)(i >> q) & 1u;
-        stg<true>(&psi[i], dense1_row<T>(r ? p : x, r ? x : p, r, u));
+        stg<NTM>(&psi[i], dense1_row<T>(r ? p : x, r ? x : p, r, u));
     }
 }
 
@@ -166,13 +195,13 @@ __global__ __launch_bounds__(kBlock) void k_dense1_lane(vec2_t<T> *__restrict__ 
 // sweep slower).  Element j holds amplitudes 2j and 2j + 1: for q = 0 they
 // are the pair; otherwise each pairs with the same half of lane j ^ 2^(q-1).
 // n4 (elements) is a multiple of kBlock, so every lane of every wave is live.
+template <bool NTM>
 __global__ __launch_bounds__(kBlock) void k_dense1_lane2_f32(float2 *__restrict__ psi, uint64_t n4, uint32_t q,
                                                              const Dense1Coef<float> u) {
-    typedef float F4 __attribute__((ext_vector_type(4)));
     F4 *p4 = reinterpret_cast<F4 *>(psi);
     const uint64_t step = (uint64_t)gridDim.x * kBlock;
     for (uint64_t j = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x; j < n4; j += step) {
-        const F4 v = __builtin_nontemporal_load(&p4[j]);
+        const F4 v = ld4<NTM>(&p4[j]);
         const float2 a0 = make_float2(v.x, v.y), a1 = make_float2(v.z, v.w);
         float2 y0, y1;
         if (q == 0) {
@@ -194,7 +223,7 @@ __global__ __launch_bounds__(kBlock) void k_dense1_lane2_f32(float2 *__restrict_
         o.y = y0.y;
         o.z = y1.x;
         o.w = y1.y;
-        __builtin_nontemporal_store(o, &p4[j]);
+        st4<NTM>(&p4[j], o);
     }
 }
 
@@ -202,7 +231,7 @@ __global__ __launch_bounds__(kBlock) void k_dense1_lane2_f32(float2 *__restrict_
 // 2 load 64 lower members each (contiguous), waves 1 and 3 the matching upper
 // members, and the partners are exchanged through LDS.  npairs is a multiple
 // of 128.
-template <typename T>
+template <typename T, bool NTM>
 __global__ __launch_bounds__(kBlock) void k_dense1_xchg(vec2_t<T> *__restrict__ psi, uint64_t npairs, uint32_t q,
                                                         const Dense1Coef<T> u) {
     using V = vec2_t<T>;
@@ -212,12 +241,12 @@ __global__ __launch_bounds__(kBlock) void k_dense1_xchg(vec2_t<T> *__restrict__ 
     for (uint64_t c = xcd_block(blockIdx.x, gridDim.x); c < nchunk; c += gridDim.x) {
         const uint64_t pair = c * 128 + ((t >> 7) << 6) + (t & 63u);
         const uint64_t a = insert_zero(pair, q) | ((uint64_t)h << q);
-        const V x = ldg<true>(&psi[a]);
+        const V x = ldg<NTM>(&psi[a]);
         sm[t] = x;
         __syncthreads();
         const V p = sm[t ^ 64u];
         __syncthreads();  // sm is rewritten by the next chunk
-        stg<true>(&psi[a], dense1_row<T>(h ? p : x, h ? x : p, h, u));
+        stg<NTM>(&psi[a], dense1_row<T>(h ? p : x, h ? x : p, h, u));
     }
 }
 
@@ -300,23 +329,22 @@ __device__ __forceinline__ void diag_entry(const DiagFullArgs<T> &a, uint64_t i,
 
 // FP32: two amplitudes per thread as one 16-byte access (the FP64 kernel's
 // one-per-lane form would make 512 B wavefront accesses).  len is even.
-template <int KT>
+template <bool NTM, int KT>
 __global__ __launch_bounds__(kBlock) void k_diag_full_f32x2(float2 *__restrict__ psi, const DiagFullArgs<float> a) {
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    f4 *p4 = (f4 *)psi;
+    F4 *p4 = (F4 *)psi;
     const uint64_t n2 = a.len / 2;
     const uint64_t step = (uint64_t)gridDim.x * kBlock;
     for (uint64_t k = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x; k < n2; k += step) {
-        const f4 x = __builtin_nontemporal_load(&p4[k]);
+        const F4 x = ld4<NTM>(&p4[k]);
         float m0r, m0i, m1r, m1i;
         diag_entry<float, KT>(a, 2 * k, m0r, m0i);
         diag_entry<float, KT>(a, 2 * k + 1, m1r, m1i);
-        f4 y;
+        F4 y;
         y.x = x.x * m0r - x.y * m0i;
         y.y = x.x * m0i + x.y * m0r;
         y.z = x.z * m1r - x.w * m1i;
         y.w = x.z * m1i + x.w * m1r;
-        __builtin_nontemporal_store(y, &p4[k]);
+        st4<NTM>(&p4[k], y);
     }
 }
 
@@ -424,20 +452,20 @@ __global__ __launch_bounds__(kBlock) void k_perm(vec2_t<T> *__restrict__ psi,
 // controls are set; the others are written back unchanged, which keeps every
 // store a full contiguous run (the pair-per-group form touches half of every
 // line when the bits are this low).
-template <typename T>
+template <typename T, bool NTM>
 __global__ __launch_bounds__(kBlock) void k_perm_lane(vec2_t<T> *__restrict__ psi, uint64_t len, uint32_t tmask,
                                                       uint32_t o0, uint32_t o1, uint32_t ctrl, uint32_t masked) {
     using V = vec2_t<T>;
     const uint32_t flip = o0 ^ o1;
     const uint64_t step = (uint64_t)gridDim.x * kBlock;
     for (uint64_t i = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x; i < len; i += step) {
-        const V x = ldg<true>(&psi[i]);
+        const V x = ldg<NTM>(&psi[i]);
         V p;
         p.x = __shfl_xor(x.x, (int)flip, 64);
         p.y = __shfl_xor(x.y, (int)flip, 64);
         const uint32_t lo = (uint32_t)i & 63u;
         const bool moved = ((lo & tmask) == o0 || (lo & tmask) == o1) && (lo & ctrl) == ctrl;
-        if (moved || !masked) stg<true>(&psi[i], moved ? p : x);
+        if (moved || !masked) stg_whole<NTM>(&psi[i], moved ? p : x);
     }
 }
 
@@ -450,7 +478,7 @@ __global__ __launch_bounds__(kBlock) void k_perm_lane(vec2_t<T> *__restrict__ ps
 // ngroups is a multiple of 128.  Measured at n = 30 against the pair form
 // (k_perm): CNOT(q, q + 7) for q = 6, 8, 12, 15, 20, 22 2.54-2.89 ms against
 // 2.59-3.01, SWAP(q, 29 - q) for q = 8, 12 2.58 / 2.62 against 2.77 / 2.80.
-template <typename T>
+template <typename T, bool NTM>
 __global__ __launch_bounds__(kBlock) void k_perm_xchg(vec2_t<T> *__restrict__ psi, const GroupSpec g, uint64_t e0,
                                                       uint64_t e1) {
     using V = vec2_t<T>;
@@ -460,11 +488,11 @@ __global__ __launch_bounds__(kBlock) void k_perm_xchg(vec2_t<T> *__restrict__ ps
     for (uint64_t c = xcd_block(blockIdx.x, gridDim.x); c < nchunk; c += gridDim.x) {
         const uint64_t grp = c * 128 + ((t >> 7) << 6) + (t & 63u);
         const uint64_t a = group_base(g, grp) | (h ? e1 : e0);
-        sm[t] = ldg<true>(&psi[a]);
+        sm[t] = ldg<NTM>(&psi[a]);
         __syncthreads();
         const V p = sm[t ^ 64u];
         __syncthreads();  // sm is rewritten by the next chunk
-        stg<true>(&psi[a], p);
+        stg<NTM>(&psi[a], p);
     }
 }
 
@@ -482,16 +510,16 @@ __global__ __launch_bounds__(kBlock) void k_perm_xchg(vec2_t<T> *__restrict__ ps
 // per lane as one 16-byte access (element j holds amplitudes 2j, 2j + 1); the
 // partner of amplitude 2j + e is in lane j ^ (flip >> 1), in the other half
 // when flip has bit 0.  n4 (elements) is a multiple of kBlock.
+template <bool NTM>
 __global__ __launch_bounds__(kBlock) void k_perm_lane2_f32(float2 *__restrict__ psi, uint64_t n4, uint32_t tmask,
                                                            uint32_t o0, uint32_t o1, uint32_t ctrl) {
-    typedef float F4 __attribute__((ext_vector_type(4)));
     F4 *p4 = reinterpret_cast<F4 *>(psi);
     const uint32_t flip = o0 ^ o1;
     const int d = (int)(flip >> 1);
     const bool odd = (flip & 1u) != 0;
     const uint64_t step = (uint64_t)gridDim.x * kBlock;
     for (uint64_t j = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x; j < n4; j += step) {
-        const F4 v = __builtin_nontemporal_load(&p4[j]);
+        const F4 v = ld4<NTM>(&p4[j]);
         const float s0x = __shfl_xor(v.x, d, 64), s0y = __shfl_xor(v.y, d, 64);
         const float s1x = __shfl_xor(v.z, d, 64), s1y = __shfl_xor(v.w, d, 64);
         const uint32_t lo0 = (uint32_t)(j << 1) & 127u, lo1 = lo0 | 1u;
@@ -506,7 +534,7 @@ __global__ __launch_bounds__(kBlock) void k_perm_lane2_f32(float2 *__restrict__ 
             o.z = odd ? s0x : s1x;
             o.w = odd ? s0y : s1y;
         }
-        __builtin_nontemporal_store(o, &p4[j]);
+        st4<NTM>(&p4[j], o);
     }
 }
 
@@ -517,7 +545,7 @@ __global__ __launch_bounds__(kBlock) void k_perm_lane2_f32(float2 *__restrict__ 
 // caller sets it when they form 64-byte halves of each line (in-line bit 2
 // only; n = 30: CPHASE(29, 2) 2.57 -> 2.11 ms), since 16- and 32-byte pieces
 // wrote slower than whole lines (CPHASE(9, 0) 2.61 -> 4.26 ms).
-template <typename T>
+template <typename T, bool NTM>
 __global__ __launch_bounds__(kBlock) void k_diag_line(vec2_t<T> *__restrict__ psi, const GroupSpec hg,
                                                       uint64_t count, uint64_t h0, uint32_t lmask, uint32_t l0,
                                                       T dr, T di, uint32_t masked) {
@@ -525,14 +553,14 @@ __global__ __launch_bounds__(kBlock) void k_diag_line(vec2_t<T> *__restrict__ ps
     const uint64_t step = (uint64_t)gridDim.x * kBlock;
     for (uint64_t j = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x; j < count; j += step) {
         const uint64_t i = group_base(hg, j) | h0;
-        const V x = ldg<true>(&psi[i]);
+        const V x = ldg<NTM>(&psi[i]);
         V y = x;
         const bool hit = ((uint32_t)i & lmask) == l0;
         if (hit) {
             y.x = x.x * dr - x.y * di;
             y.y = x.x * di + x.y * dr;
         }
-        if (hit || !masked) stg<true>(&psi[i], y);
+        if (hit || !masked) stg_whole<NTM>(&psi[i], y);
     }
 }
 
@@ -542,21 +570,21 @@ __global__ __launch_bounds__(kBlock) void k_diag_line(vec2_t<T> *__restrict__ ps
 // off2 the entry's offset in pairs), each thread one pair, non-temporal (the
 // caller uses it for runs of >= 128 B); the products are those of
 // k_diag_sparse.
+template <bool NTM>
 __global__ __launch_bounds__(kBlock) void k_diag_sparse2_f32(float2 *__restrict__ psi, const GroupSpec g2,
                                                              uint64_t off2, float dr, float di) {
-    typedef float F4 __attribute__((ext_vector_type(4)));
     F4 *p4 = reinterpret_cast<F4 *>(psi);
     const uint64_t step = (uint64_t)gridDim.x * kBlock;
     for (uint64_t i = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x; i < g2.ngroups;
          i += step) {
         const uint64_t e = group_base(g2, i) | off2;
-        const F4 v = __builtin_nontemporal_load(&p4[e]);
+        const F4 v = ld4<NTM>(&p4[e]);
         F4 y;
         y.x = v.x * dr - v.y * di;
         y.y = v.x * di + v.y * dr;
         y.z = v.z * dr - v.w * di;
         y.w = v.z * di + v.w * dr;
-        __builtin_nontemporal_store(y, &p4[e]);
+        st4<NTM>(&p4[e], y);
     }
 }
 
@@ -565,7 +593,7 @@ __global__ __launch_bounds__(kBlock) void k_diag_sparse2_f32(float2 *__restrict_
 // moving amplitude at in-line position l of line A (upper bits h0) pairs with
 // position l ^ (l0 ^ l1) of line B (upper bits h1): a lane shuffle.  With
 // h0 == h1 both entries lie in the same lines.
-template <typename T>
+template <typename T, bool NTM>
 __global__ __launch_bounds__(kBlock) void k_perm_line(vec2_t<T> *__restrict__ psi, const GroupSpec hg,
                                                       uint64_t count, uint64_t h0, uint64_t h1, uint32_t lmask,
                                                       uint32_t l0, uint32_t l1) {
@@ -576,8 +604,8 @@ __global__ __launch_bounds__(kBlock) void k_perm_line(vec2_t<T> *__restrict__ ps
     for (uint64_t j = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x; j < count; j += step) {
         const uint64_t g = group_base(hg, j);
         const uint64_t ia = g | h0, ib = g | h1;
-        const V xa = ldg<true>(&psi[ia]);
-        const V xb = two ? ldg<true>(&psi[ib]) : xa;
+        const V xa = ldg<NTM>(&psi[ia]);
+        const V xb = two ? ldg<NTM>(&psi[ib]) : xa;
         V pa, pb;
         pa.x = __shfl_xor(xa.x, d, 64);
         pa.y = __shfl_xor(xa.y, d, 64);
@@ -585,10 +613,10 @@ __global__ __launch_bounds__(kBlock) void k_perm_line(vec2_t<T> *__restrict__ ps
         pb.y = __shfl_xor(xb.y, d, 64);
         const uint32_t ls = (uint32_t)ia & lmask;
         if (two) {
-            stg<true>(&psi[ia], ls == l0 ? pb : xa);
-            stg<true>(&psi[ib], ls == l1 ? pa : xb);
+            stg_whole<NTM>(&psi[ia], ls == l0 ? pb : xa);
+            stg_whole<NTM>(&psi[ib], ls == l1 ? pa : xb);
         } else {
-            stg<true>(&psi[ia], (ls == l0 || ls == l1) ? pa : xa);
+            stg_whole<NTM>(&psi[ia], (ls == l0 || ls == l1) ? pa : xa);
         }
     }
 }
@@ -779,6 +807,19 @@ bool long_runs(const GroupSpec &g, size_t amp_bytes) {
     return qmin >= 16 || ((uint64_t(1) << qmin) * amp_bytes >= 128);
 }
 
+// Launches KERNEL<..., NTM, ...> for the run-time flag nt: QH_LAUNCH_NT(nt,
+// (KERNEL<T, NTM>), grid, stream, args...).
+#define QH_LAUNCH_NT(nt, KERNEL, grid, stream, ...)                                              \
+    do {                                                                                         \
+        if (nt) {                                                                                \
+            constexpr bool NTM = true;                                                           \
+            hipLaunchKernelGGL(KERNEL, grid, dim3(kBlock), 0, stream, __VA_ARGS__);              \
+        } else {                                                                                 \
+            constexpr bool NTM = false;                                                          \
+            hipLaunchKernelGGL(KERNEL, grid, dim3(kBlock), 0, stream, __VA_ARGS__);              \
+        }                                                                                        \
+    } while (0)
+
 template <typename T, int KT>
 int run_dense_small(qvmhip_state *s, const GateSplit &gs) {
     constexpr int D = 1 << KT;
@@ -807,11 +848,11 @@ int run_dense_small(qvmhip_state *s, const GateSplit &gs) {
             const uint32_t q = gs.tq[0];
             prof_begin(s, KT);
             if (q < 6)
-                hipLaunchKernelGGL((k_dense1_lane<T>), dim3(grid_for(s->len, kBlock)), dim3(kBlock), 0, s->stream,
-                                   (vec2_t<T> *)s->amps, s->len, q, u);
+                QH_LAUNCH_NT(stream_accesses(s), (k_dense1_lane<T, NTM>), dim3(grid_for(s->len, kBlock)), s->stream,
+                             (vec2_t<T> *)s->amps, s->len, q, u);
             else
-                hipLaunchKernelGGL((k_dense1_xchg<T>), dim3(grid_for(s->len / 2, 128)), dim3(kBlock), 0, s->stream,
-                                   (vec2_t<T> *)s->amps, s->len / 2, q, u);
+                QH_LAUNCH_NT(stream_accesses(s), (k_dense1_xchg<T, NTM>), dim3(grid_for(s->len / 2, 128)), s->stream,
+                             (vec2_t<T> *)s->amps, s->len / 2, q, u);
             prof_end(s);
             QH_LAUNCH_CHECK();
             return QVMHIP_OK;
@@ -825,8 +866,8 @@ int run_dense_small(qvmhip_state *s, const GateSplit &gs) {
                 u.ui[i] = (float)gs.V[i].imag();
             }
             prof_begin(s, KT);
-            hipLaunchKernelGGL(k_dense1_lane2_f32, dim3(grid_for(s->len / 2, kBlock)), dim3(kBlock), 0, s->stream,
-                               (float2 *)s->amps, s->len / 2, gs.tq[0], u);
+            QH_LAUNCH_NT(stream_accesses(s), (k_dense1_lane2_f32<NTM>), dim3(grid_for(s->len / 2, kBlock)), s->stream,
+                         (float2 *)s->amps, s->len / 2, gs.tq[0], u);
             prof_end(s);
             QH_LAUNCH_CHECK();
             return QVMHIP_OK;
@@ -834,10 +875,8 @@ int run_dense_small(qvmhip_state *s, const GateSplit &gs) {
     }
     const dim3 grid(grid_for(a.g.ngroups, (uint64_t)kBlock * GPT));
     prof_begin(s, KT);
-    if (long_runs(a.g, s->amp_bytes))
-        hipLaunchKernelGGL((k_dense<T, KT, GPT, true>), grid, dim3(kBlock), 0, s->stream, (vec2_t<T> *)s->amps, a);
-    else
-        hipLaunchKernelGGL((k_dense<T, KT, GPT, false>), grid, dim3(kBlock), 0, s->stream, (vec2_t<T> *)s->amps, a);
+    QH_LAUNCH_NT(stream_accesses(s) && long_runs(a.g, s->amp_bytes), (k_dense<T, KT, GPT, NTM>), grid, s->stream,
+                 (vec2_t<T> *)s->amps, a);
     prof_end(s);
     QH_LAUNCH_CHECK();
     return QVMHIP_OK;
@@ -874,6 +913,7 @@ int run_dense_big(qvmhip_state *s, const GateSplit &gs) {
 template <typename T>
 int run_diag(qvmhip_state *s, const GateSplit &gs) {
     const uint32_t Dr = 1u << gs.kt;
+    const bool nt = stream_accesses(s);
     std::vector<uint32_t> ent;
     for (uint32_t j = 0; j < Dr; ++j)
         if (!exactly(gs.V[(size_t)j * Dr + j], 1.0, 0.0)) ent.push_back(j);
@@ -897,10 +937,10 @@ int run_diag(qvmhip_state *s, const GateSplit &gs) {
                 const dim3 g2(grid_for(a.len / 2, (uint64_t)kBlock));
                 prof_begin(s, QVMHIP_K_DIAG_FULL);
                 switch (gs.kt) {
-                    case 1: hipLaunchKernelGGL((k_diag_full_f32x2<1>), g2, dim3(kBlock), 0, s->stream, psi, a); break;
-                    case 2: hipLaunchKernelGGL((k_diag_full_f32x2<2>), g2, dim3(kBlock), 0, s->stream, psi, a); break;
-                    case 3: hipLaunchKernelGGL((k_diag_full_f32x2<3>), g2, dim3(kBlock), 0, s->stream, psi, a); break;
-                    default: hipLaunchKernelGGL((k_diag_full_f32x2<0>), g2, dim3(kBlock), 0, s->stream, psi, a);
+                    case 1: QH_LAUNCH_NT(nt, (k_diag_full_f32x2<NTM, 1>), g2, s->stream, psi, a); break;
+                    case 2: QH_LAUNCH_NT(nt, (k_diag_full_f32x2<NTM, 2>), g2, s->stream, psi, a); break;
+                    case 3: QH_LAUNCH_NT(nt, (k_diag_full_f32x2<NTM, 3>), g2, s->stream, psi, a); break;
+                    default: QH_LAUNCH_NT(nt, (k_diag_full_f32x2<NTM, 0>), g2, s->stream, psi, a);
                 }
                 prof_end(s);
                 QH_LAUNCH_CHECK();
@@ -910,10 +950,10 @@ int run_diag(qvmhip_state *s, const GateSplit &gs) {
         const dim3 grid(grid_for(a.len, (uint64_t)kBlock));
         prof_begin(s, QVMHIP_K_DIAG_FULL);
         switch (gs.kt) {
-            case 1: hipLaunchKernelGGL((k_diag_full<T, true, 1>), grid, dim3(kBlock), 0, s->stream, psi, a); break;
-            case 2: hipLaunchKernelGGL((k_diag_full<T, true, 2>), grid, dim3(kBlock), 0, s->stream, psi, a); break;
-            case 3: hipLaunchKernelGGL((k_diag_full<T, true, 3>), grid, dim3(kBlock), 0, s->stream, psi, a); break;
-            default: hipLaunchKernelGGL((k_diag_full<T, true, 0>), grid, dim3(kBlock), 0, s->stream, psi, a);
+            case 1: QH_LAUNCH_NT(nt, (k_diag_full<T, NTM, 1>), grid, s->stream, psi, a); break;
+            case 2: QH_LAUNCH_NT(nt, (k_diag_full<T, NTM, 2>), grid, s->stream, psi, a); break;
+            case 3: QH_LAUNCH_NT(nt, (k_diag_full<T, NTM, 3>), grid, s->stream, psi, a); break;
+            default: QH_LAUNCH_NT(nt, (k_diag_full<T, NTM, 0>), grid, s->stream, psi, a);
         }
         prof_end(s);
         QH_LAUNCH_CHECK();
@@ -940,9 +980,9 @@ int run_diag(qvmhip_state *s, const GateSplit &gs) {
         if (ls.hg.ngroups % kBlock == 0) {
             const uint64_t e0 = a.off[0] | a.g.ctrl_mask;
             prof_begin(s, QVMHIP_K_DIAG_SPARSE);
-            hipLaunchKernelGGL((k_diag_line<T>), dim3(grid_for(ls.hg.ngroups, kBlock)), dim3(kBlock), 0, s->stream,
-                               psi, ls.hg, ls.hg.ngroups, e0 & ls.hmask, ls.lmask, (uint32_t)e0 & ls.lmask, a.dr[0],
-                               a.di[0], (ls.lmask & 3u) == 0 ? 1u : 0u);
+            QH_LAUNCH_NT(nt, (k_diag_line<T, NTM>), dim3(grid_for(ls.hg.ngroups, kBlock)), s->stream, psi, ls.hg,
+                         ls.hg.ngroups, e0 & ls.hmask, ls.lmask, (uint32_t)e0 & ls.lmask, a.dr[0], a.di[0],
+                         (ls.lmask & 3u) == 0 ? 1u : 0u);
             prof_end(s);
             QH_LAUNCH_CHECK();
             return QVMHIP_OK;
@@ -958,20 +998,17 @@ int run_diag(qvmhip_state *s, const GateSplit &gs) {
         g2.ctrl_mask >>= 1;
         g2.ngroups >>= 1;
         prof_begin(s, QVMHIP_K_DIAG_SPARSE);
-        hipLaunchKernelGGL(k_diag_sparse2_f32, dim3(grid_for(g2.ngroups, (uint64_t)kBlock)), dim3(kBlock), 0,
-                           s->stream, (float2 *)s->amps, g2, a.off[0] >> 1, (float)a.dr[0], (float)a.di[0]);
+        QH_LAUNCH_NT(nt, (k_diag_sparse2_f32<NTM>), dim3(grid_for(g2.ngroups, (uint64_t)kBlock)), s->stream,
+                     (float2 *)s->amps, g2, a.off[0] >> 1, (float)a.dr[0], (float)a.di[0]);
         prof_end(s);
         QH_LAUNCH_CHECK();
         return QVMHIP_OK;
     }
     prof_begin(s, QVMHIP_K_DIAG_SPARSE);
-    if (a.nent == 1) {
-        if (lr) hipLaunchKernelGGL((k_diag_sparse<T, GPT, true, true>), grid, dim3(kBlock), 0, s->stream, psi, a);
-        else hipLaunchKernelGGL((k_diag_sparse<T, GPT, false, true>), grid, dim3(kBlock), 0, s->stream, psi, a);
-    } else {
-        if (lr) hipLaunchKernelGGL((k_diag_sparse<T, GPT, true, false>), grid, dim3(kBlock), 0, s->stream, psi, a);
-        else hipLaunchKernelGGL((k_diag_sparse<T, GPT, false, false>), grid, dim3(kBlock), 0, s->stream, psi, a);
-    }
+    if (a.nent == 1)
+        QH_LAUNCH_NT(nt && lr, (k_diag_sparse<T, GPT, NTM, true>), grid, s->stream, psi, a);
+    else
+        QH_LAUNCH_NT(nt && lr, (k_diag_sparse<T, GPT, NTM, false>), grid, s->stream, psi, a);
     prof_end(s);
     QH_LAUNCH_CHECK();
     return QVMHIP_OK;
@@ -980,6 +1017,7 @@ int run_diag(qvmhip_state *s, const GateSplit &gs) {
 template <typename T>
 int run_perm(qvmhip_state *s, const GateSplit &gs) {
     const uint32_t Dr = 1u << gs.kt;
+    const bool nt = stream_accesses(s);
     SparseArgs<T> a;
     std::memset(&a, 0, sizeof(a));
     make_group_spec(a.g, gs, s->n);
@@ -1007,9 +1045,8 @@ int run_perm(qvmhip_state *s, const GateSplit &gs) {
         uint32_t tmask = 0;
         for (uint32_t t = 0; t < gs.kt; ++t) tmask |= 1u << gs.tq[t];
         prof_begin(s, QVMHIP_K_PERM);
-        hipLaunchKernelGGL(k_perm_lane2_f32, dim3(grid_for(s->len / 2, kBlock)), dim3(kBlock), 0, s->stream,
-                           (float2 *)s->amps, s->len / 2, tmask, (uint32_t)a.off[0], (uint32_t)a.off[1],
-                           (uint32_t)a.g.ctrl_mask);
+        QH_LAUNCH_NT(nt, (k_perm_lane2_f32<NTM>), dim3(grid_for(s->len / 2, kBlock)), s->stream, (float2 *)s->amps,
+                     s->len / 2, tmask, (uint32_t)a.off[0], (uint32_t)a.off[1], (uint32_t)a.g.ctrl_mask);
         prof_end(s);
         QH_LAUNCH_CHECK();
         return QVMHIP_OK;
@@ -1027,9 +1064,8 @@ int run_perm(qvmhip_state *s, const GateSplit &gs) {
         // FP64 with every bit >= 2: the moved amplitudes are 64-byte halves
         // of lines, and only they are stored (as in k_diag_line)
         const uint32_t masked = (sizeof(T) == 8 && ((tmask | (uint32_t)a.g.ctrl_mask) & 3u) == 0) ? 1u : 0u;
-        hipLaunchKernelGGL((k_perm_lane<T>), dim3(grid_for(s->len, kBlock)), dim3(kBlock), 0, s->stream,
-                           (vec2_t<T> *)s->amps, s->len, tmask, (uint32_t)a.off[0], (uint32_t)a.off[1],
-                           (uint32_t)a.g.ctrl_mask, masked);
+        QH_LAUNCH_NT(nt, (k_perm_lane<T, NTM>), dim3(grid_for(s->len, kBlock)), s->stream, (vec2_t<T> *)s->amps,
+                     s->len, tmask, (uint32_t)a.off[0], (uint32_t)a.off[1], (uint32_t)a.g.ctrl_mask, masked);
         prof_end(s);
         QH_LAUNCH_CHECK();
         return QVMHIP_OK;
@@ -1040,8 +1076,8 @@ int run_perm(qvmhip_state *s, const GateSplit &gs) {
     V2Ptr<T> psi = (vec2_t<T> *)s->amps;
     if (sizeof(T) == 8 && a.nent == 2 && a.g.nsorted && a.g.sorted[0] >= 6 && a.g.ngroups % 128 == 0) {
         prof_begin(s, QVMHIP_K_PERM);
-        hipLaunchKernelGGL((k_perm_xchg<T>), dim3(grid_for(a.g.ngroups, 128)), dim3(kBlock), 0, s->stream,
-                           (vec2_t<T> *)s->amps, a.g, a.off[0], a.off[1]);
+        QH_LAUNCH_NT(nt, (k_perm_xchg<T, NTM>), dim3(grid_for(a.g.ngroups, 128)), s->stream, (vec2_t<T> *)s->amps,
+                     a.g, a.off[0], a.off[1]);
         prof_end(s);
         QH_LAUNCH_CHECK();
         return QVMHIP_OK;
@@ -1053,22 +1089,19 @@ int run_perm(qvmhip_state *s, const GateSplit &gs) {
         if (ls.hg.ngroups % kBlock == 0) {
             const uint64_t e0 = a.off[0] | a.g.ctrl_mask, e1 = a.off[1] | a.g.ctrl_mask;
             prof_begin(s, QVMHIP_K_PERM);
-            hipLaunchKernelGGL((k_perm_line<T>), dim3(grid_for(ls.hg.ngroups, kBlock)), dim3(kBlock), 0, s->stream,
-                               psi, ls.hg, ls.hg.ngroups, e0 & ls.hmask, e1 & ls.hmask, ls.lmask,
-                               (uint32_t)e0 & ls.lmask, (uint32_t)e1 & ls.lmask);
+            QH_LAUNCH_NT(nt, (k_perm_line<T, NTM>), dim3(grid_for(ls.hg.ngroups, kBlock)), s->stream, psi, ls.hg,
+                         ls.hg.ngroups, e0 & ls.hmask, e1 & ls.hmask, ls.lmask, (uint32_t)e0 & ls.lmask,
+                         (uint32_t)e1 & ls.lmask);
             prof_end(s);
             QH_LAUNCH_CHECK();
             return QVMHIP_OK;
         }
     }
     prof_begin(s, QVMHIP_K_PERM);
-    if (a.nent == 2) {
-        if (lr) hipLaunchKernelGGL((k_perm<T, GPT, true, true>), grid, dim3(kBlock), 0, s->stream, psi, a);
-        else hipLaunchKernelGGL((k_perm<T, GPT, false, true>), grid, dim3(kBlock), 0, s->stream, psi, a);
-    } else {
-        if (lr) hipLaunchKernelGGL((k_perm<T, GPT, true, false>), grid, dim3(kBlock), 0, s->stream, psi, a);
-        else hipLaunchKernelGGL((k_perm<T, GPT, false, false>), grid, dim3(kBlock), 0, s->stream, psi, a);
-    }
+    if (a.nent == 2)
+        QH_LAUNCH_NT(nt && lr, (k_perm<T, GPT, NTM, true>), grid, s->stream, psi, a);
+    else
+        QH_LAUNCH_NT(nt && lr, (k_perm<T, GPT, NTM, false>), grid, s->stream, psi, a);
     prof_end(s);
     QH_LAUNCH_CHECK();
     return QVMHIP_OK;

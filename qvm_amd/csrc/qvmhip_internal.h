@@ -206,6 +206,17 @@ struct qvmhip_state {
 };
 
 namespace qvmhip {
+// Whether the sweeps of a state use non-temporal accesses.  Up to 256 MiB
+// the state stays in the Infinity Cache from one gate to the next and the
+// cached forms find it there; the non-temporal ones go to HBM.  Measured per
+// gate (us, non-temporal / cached; FP64 RX(12), CNOT(9, 13), CZ(8, 14)):
+// 2^22 amplitudes 22.8 / 19.0, 13.7 / 9.9, 9.2 / 8.0; 2^24 (256 MiB)
+// 81.3 / 62.3, 55.9 / 34.1, 26.7 / 22.2; past it the cached forms thrash: RX 2^25
+// 160 / 175, 2^28 1319 / 1420.  FP32 crosses over at the same size in bytes
+// (RX(12): 2^25 82.8 / 65.2, 2^26 162 / 177).
+constexpr uint64_t kStreamBytes = uint64_t(256) << 20;
+inline bool stream_accesses(const qvmhip_state *s) { return s->len * s->amp_bytes > kStreamBytes; }
+
 // Live per-launch timing.  prof_begin/prof_end bracket one kernel launch
 // with HIP events on the state's stream when profiling is on.
 inline hipEvent_t prof_event(qvmhip_state *s) {
