@@ -180,6 +180,14 @@ QVMHIP_API int qvmhip_norm(qvmhip_state *s, double *out);
  * norm, as the stochastic Kraus evolution accumulates it
  * (src/apply-gate.lisp:16-39). */
 QVMHIP_API int qvmhip_total_probability(qvmhip_state *s, double *out);
+/* The stochastic Kraus evolution of a pure state (src/apply-gate.lisp:16-39)
+ * with the caller's uniform r: the state becomes K_j psi / |K_j psi| for the
+ * first j whose running sum of |K_j psi|^2 reaches r, the last one when none
+ * does; *index = j.  K: `count` 2^k x 2^k matrices, k = 1 or 2.  A chosen
+ * operator that annihilates the state returns QVMHIP_ERANGE with the state
+ * unchanged. */
+QVMHIP_API int qvmhip_apply_kraus_choice(qvmhip_state *s, const double *K, uint32_t count, uint32_t k,
+                                         const uint32_t *qubits, double r, uint32_t *index);
 /* normalize-wavefunction: src/wavefunction.lisp:349-364 (length <= 0:
  * compute the norm first). */
 QVMHIP_API int qvmhip_normalize(qvmhip_state *s, double length);

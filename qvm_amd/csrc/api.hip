@@ -270,6 +270,16 @@ int qvmhip_density_apply_kraus(qvmhip_state *s, uint32_t nq, const double *K, ui
     return launch_kraus(s, nq, K, count, k, qubits);
 }
 
+int qvmhip_apply_kraus_choice(qvmhip_state *s, const double *K, uint32_t count, uint32_t k, const uint32_t *qubits,
+                              double r, uint32_t *index) {
+    int rc = check_qubits(s, k, qubits);
+    if (rc) return rc;
+    if (k > 2) return fail(QVMHIP_EINVAL, "the Kraus choice takes 1- and 2-qubit operators");
+    if (!K || !index || count < 1) return fail(QVMHIP_EINVAL, "null argument or no Kraus operators");
+    DeviceScope ds(s->device);
+    return launch_kraus_choice(s, K, count, k, qubits, r, index);
+}
+
 int qvmhip_apply_tile_pass(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, uint32_t nops,
                            const qvmhip_tile_op *ops) {
     if (!s) return fail(QVMHIP_EINVAL, "null state");

@@ -1,6 +1,8 @@
 // channel.hip -- noise channels (Kraus maps): the superoperator of a
-// density-matrix gate in one sweep.
+// density-matrix gate in one sweep, and the stochastic choice of one Kraus
+// operator on a pure state in one read and one gate sweep.
 //
+// Density matrices.
 // A density matrix rho is held as vec(rho), row-major, in a 2*nq-qubit state:
 // column bits 0..nq-1, row bits nq..2*nq-1 (src/density-qvm.lisp).  A Kraus map
 // rho -> sum_j K_j rho K_j^H on k qubits is then one linear map on the 2k index
@@ -12,8 +14,19 @@
 // copies; as one superoperator it is one read and one write of the state
 // whatever m is.  A 12-qubit noisy circuit (2^24 amplitudes, 94 gates with 1,
 // 2 or 4 operators) went from 80.2 to 8.05 ms, 85 us or 6.3 TB/s per gate.
+//
+// Pure states.  One operator of the map is chosen by inverse-transform
+// sampling over p_j = |K_j psi|^2 (src/apply-gate.lisp:16-39).  Trying the operators
+// one after another on a copy moves, per operator tried, a copied state (32
+// bytes per amplitude), a gate sweep (32) and a norm (16), then a norm and a
+// scale sweep (48).  k_kraus_norms reads the state once for up to four
+// operators: every group's products K_j x are formed in registers and only
+// their squares are kept.  The chosen operator, divided by sqrt(p_j), is then
+// one ordinary gate in place: 48 bytes per amplitude in all.
+#include <algorithm>
 #include <cmath>
 #include <complex>
+#include <cstring>
 #include <vector>
 
 #include "qvmhip_internal.h"
@@ -59,6 +72,143 @@ int launch_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, 
     void *dst = (char *)s->mat + kFusedMatOffset;
     QH_CHECK(hipMemcpyAsync(dst, m, S.size() * sizeof(cd), hipMemcpyHostToDevice, s->stream));
     return launch_fused_dense(s, dst, 2 * k, q);
+}
+
+// Operators per read: every one adds 2^k complex products per amplitude.  Four
+// 1-qubit or two 2-qubit operators stay under the time of the read (2^24 FP64
+// amplitudes: 4 x 18 or 2 x 30 FP64 operations per amplitude, about 30 us of
+// issue against 45 us).
+constexpr int kraus_per_read(int k) { return k == 1 ? 4 : 2; }
+constexpr int kNormBlocks = 1024;  // partials of kNormBlocks * 4 sums fit the state's reduction scratch
+static_assert(kNormBlocks * 4 <= kRedBlocks * 2, "reduction scratch");
+
+template <typename T, int K>
+struct KrausArgs {
+    static constexpr int D = 1 << K, C = kraus_per_read(K);
+    GroupSpec g;
+    uint64_t off[D];
+    T ur[C * D * D];
+    T ui[C * D * D];
+};
+
+// partial[C * block + j] = the block's share of sum |K_j x|^2, in FP64; the
+// products are rounded in T and summed left to right, as the gate kernels do.
+// Bound by the read; UN groups per thread are in flight.
+template <typename T, int K>
+__global__ __launch_bounds__(kBlock) void k_kraus_norms(const vec2_t<T> *__restrict__ psi, const KrausArgs<T, K> a,
+                                                        double *__restrict__ partial) {
+    constexpr int D = 1 << K, C = kraus_per_read(K), UN = K == 1 ? 4 : 2, NW = kBlock / 64;
+    using V = vec2_t<T>;
+    __shared__ double sm[C][NW];
+    double acc[C];
+#pragma unroll
+    for (int j = 0; j < C; ++j) acc[j] = 0.0;
+    const uint64_t step = (uint64_t)gridDim.x * kBlock;
+    for (uint64_t i0 = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i0 < a.g.ngroups; i0 += UN * step) {
+        V x[UN][D];
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+            const uint64_t i = i0 + u * step;
+            const uint64_t base = group_base(a.g, i < a.g.ngroups ? i : i0);
+#pragma unroll
+            for (int d = 0; d < D; ++d) x[u][d] = psi[base + a.off[d]];
+        }
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+            if (i0 + u * step >= a.g.ngroups) break;
+#pragma unroll
+            for (int j = 0; j < C; ++j)
+#pragma unroll
+                for (int r = 0; r < D; ++r) {
+                    T yr = T(0), yi = T(0);
+#pragma unroll
+                    for (int c = 0; c < D; ++c) {
+                        const T mr = a.ur[(j * D + r) * D + c], mi = a.ui[(j * D + r) * D + c];
+                        const T pr = x[u][c].x * mr - x[u][c].y * mi;
+                        const T pi = x[u][c].x * mi + x[u][c].y * mr;
+                        yr = c ? yr + pr : pr;
+                        yi = c ? yi + pi : pi;
+                    }
+                    acc[j] += (double)yr * (double)yr + (double)yi * (double)yi;
+                }
+        }
+    }
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+        double v = acc[j];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+        if (lane == 0) sm[j][wid] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < C) {
+        double t = 0.0;
+        for (int w = 0; w < NW; ++w) t += sm[threadIdx.x][w];
+        partial[C * blockIdx.x + threadIdx.x] = t;
+    }
+}
+
+// out[j] = |K_j psi|^2 for the first `count` (at most kraus_per_read(K)) operators.
+template <typename T, int K>
+static int kraus_norms(qvmhip_state *s, const cd *ops, uint32_t count, const uint32_t *qubits, double *out) {
+    constexpr int D = 1 << K, C = kraus_per_read(K);
+    KrausArgs<T, K> a;
+    std::memset(&a, 0, sizeof(a));
+    a.g.nsorted = K;
+    for (int b = 0; b < K; ++b) a.g.sorted[b] = qubits[b];
+    std::sort(a.g.sorted, a.g.sorted + K);
+    a.g.ngroups = uint64_t(1) << (s->n - K);
+    for (int d = 0; d < D; ++d)
+        for (int b = 0; b < K; ++b)
+            if ((d >> b) & 1) a.off[d] |= uint64_t(1) << qubits[b];
+    for (uint32_t e = 0; e < count * D * D; ++e) {
+        a.ur[e] = (T)ops[e].real();
+        a.ui[e] = (T)ops[e].imag();
+    }
+    const uint32_t grid = (uint32_t)std::min<uint64_t>((a.g.ngroups + kBlock - 1) / kBlock, kNormBlocks);
+    hipLaunchKernelGGL((k_kraus_norms<T, K>), dim3(grid), dim3(kBlock), 0, s->stream, (const vec2_t<T> *)s->amps, a,
+                       s->red);
+    QH_LAUNCH_CHECK();
+    return sums_to_host(s, (int)grid, C, out, (int)count);
+}
+
+int launch_kraus_choice(qvmhip_state *s, const double *K, uint32_t count, uint32_t k, const uint32_t *qubits, double r,
+                        uint32_t *index) {
+    const size_t DD = size_t(1) << (2 * k);
+    const cd *ops = reinterpret_cast<const cd *>(K);
+    const uint32_t per = (uint32_t)kraus_per_read((int)k);
+    double sum = 0.0, p = 0.0;
+    uint32_t chosen = count - 1;
+    bool found = false;
+    for (uint32_t j0 = 0; j0 < count && !found; j0 += per) {
+        const uint32_t c = std::min(per, count - j0);
+        double pj[4];
+        int rc;
+        if (s->dtype == QVMHIP_F64)
+            rc = k == 1 ? kraus_norms<double, 1>(s, ops + j0 * DD, c, qubits, pj)
+                        : kraus_norms<double, 2>(s, ops + j0 * DD, c, qubits, pj);
+        else
+            rc = k == 1 ? kraus_norms<float, 1>(s, ops + j0 * DD, c, qubits, pj)
+                        : kraus_norms<float, 2>(s, ops + j0 * DD, c, qubits, pj);
+        if (rc) return rc;
+        for (uint32_t j = 0; j < c && !found; ++j) {
+            // operators past the chosen one are never looked at
+            const double *m = K + 2 * (j0 + j) * DD;
+            if (!std::all_of(m, m + 2 * DD, [](double v) { return std::isfinite(v); }))
+                return fail(QVMHIP_EINVAL, "matrix is not finite");
+            p = pj[j];
+            sum += p;
+            chosen = j0 + j;
+            found = sum >= r;
+        }
+    }
+    const double len = std::sqrt(p);
+    if (!(len > 0) || !std::isfinite(len)) return fail(QVMHIP_ERANGE, "cannot normalize a zero/non-finite state");
+    std::vector<cd> U(ops + chosen * DD, ops + (chosen + 1) * DD);
+    for (cd &z : U) z *= 1.0 / len;
+    *index = chosen;
+    return launch_gate(s, reinterpret_cast<const double *>(U.data()), k, qubits, 0);
 }
 
 }  // namespace qvmhip

@@ -245,6 +245,13 @@ int launch_gate(qvmhip_state *s, const double *U, uint32_t k, const uint32_t *qu
 bool gate_is_dense(const double *U, uint32_t k, const uint32_t *qubits);  // neither diagonal nor a permutation
 // sum_j K_j rho K_j^H on the density matrix of nq qubits held in s, 1 <= k <= 3
 int launch_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, uint32_t k, const uint32_t *qubits);
+// psi -> K_j psi / |K_j psi| for the first j whose running sum of |K_j psi|^2
+// reaches r (the last one when none does); 1 <= k <= 2
+int launch_kraus_choice(qvmhip_state *s, const double *K, uint32_t count, uint32_t k, const uint32_t *qubits, double r,
+                        uint32_t *index);
+// adds the `n` partials in s->red (`width` interleaved sums) and waits: the
+// first `count` sums go to out
+int sums_to_host(qvmhip_state *s, int n, int width, double *out, int count);
 int launch_diagonal(qvmhip_state *s, const double *d, uint32_t k, const uint32_t *qubits);
 int launch_permutation(qvmhip_state *s, const uint32_t *perm, uint32_t k, const uint32_t *qubits);
 int launch_fill_zero_state(qvmhip_state *s);

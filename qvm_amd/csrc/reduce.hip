@@ -706,6 +706,16 @@ int reduce_probability(qvmhip_state *s, int mode, uint32_t q, double *out_dev) {
     return QVMHIP_OK;
 }
 
+int sums_to_host(qvmhip_state *s, int n, int width, double *out, int count) {
+    double *dev = s->red + kRedBlocks * 2;
+    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(kBlock), 0, s->stream, s->red, n, width, dev);
+    QH_LAUNCH_CHECK();
+    QH_CHECK(hipMemcpyAsync(s->host, dev, sizeof(double) * width, hipMemcpyDeviceToHost, s->stream));
+    QH_CHECK(hipStreamSynchronize(s->stream));
+    std::copy(s->host, s->host + count, out);
+    return QVMHIP_OK;
+}
+
 int reduce_norm2(qvmhip_state *s, double *out_dev) { return reduce_probability(s, 0, 0, out_dev); }
 
 int launch_force_measure(qvmhip_state *s, uint32_t q, int bit, double inv_norm, int compiled_form) {

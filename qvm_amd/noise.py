@@ -11,11 +11,11 @@ Mirrors the reference's noisy-qvm (src/noisy-qvm.lisp) for pure states:
     check_kraus_ops / check_povm  src/channel-qvm.lisp:109-135, 197-206
     perturb_measurement           src/channel-qvm.lisp:185-195
 
-The Kraus choice needs a second statevector of the same size (the trial
-amplitudes): each candidate K_j is applied to a device copy of the state and
-the running sum of its total probability is compared with one uniform draw;
-the chosen trial buffer is swapped in and renormalised.  Every step is an
-engine kernel (copy, gate application, reduction, scale).
+The Kraus choice of a 1- or 2-qubit map is one engine call: the running sum of
+|K_j psi|^2 is compared with one uniform draw and the chosen operator is
+applied in place, renormalised.  Wider maps need a second statevector of the
+same size (the trial amplitudes): each candidate K_j is applied to a device
+copy of the state, and the chosen trial buffer is swapped in.
 """
 from __future__ import annotations
 
@@ -92,10 +92,14 @@ def perturb_measurement(actual: int, p00: float, p01: float, p10: float, p11: fl
 def evolve_pure_state_stochastically(state: HipPureState, trial: HipPureState, kraus_ops, quil_qubits,
                                      r: float) -> int:
     """Apply one Kraus operator of the map, chosen by inverse-transform
-    sampling with the draw r: for j = 1, 2, ... the trial buffer is set to
-    K_j psi and p_j = |K_j psi|^2 added to a running sum until the sum
-    reaches r; the last trial buffer becomes the state, renormalised.
-    Returns the index j chosen."""
+    sampling with the draw r: p_j = |K_j psi|^2 is added to a running sum until
+    the sum reaches r; K_j psi, renormalised, becomes the state.  Maps on 1 or
+    2 qubits read the state once for the p_j and apply the chosen operator in
+    place; wider ones set the trial buffer to each K_j psi in turn.  Returns
+    the index j chosen."""
+    if 1 <= len(quil_qubits) <= 2 and len(kraus_ops):
+        ops = np.stack([np.asarray(k, dtype=np.complex128) for k in kraus_ops])
+        return state.apply_kraus_choice(ops, G.nat_tuple(*quil_qubits), r)
     summed = 0.0
     chosen = -1
     for j, K in enumerate(kraus_ops):

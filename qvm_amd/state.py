@@ -135,6 +135,20 @@ class HipPureState:
         N.check(N.lib().qvmhip_total_probability(self._h, C.byref(out)))
         return out.value
 
+    def apply_kraus_choice(self, kraus_ops, qubits, r: float) -> int:
+        """The state becomes K_j psi / |K_j psi|, j the first operator whose
+        running sum of |K_j psi|^2 reaches r (``qubits`` in nat-tuple order, 1
+        or 2 of them).  Returns j."""
+        q = N.u32arr(qubits)
+        k = len(q)
+        K = N.cmat(kraus_ops)
+        if K.shape[1:] != (1 << k, 1 << k):
+            raise ValueError(f"matrix shape {K.shape[1:]} does not match {k} qubits")
+        out = C.c_uint32()
+        N.check(N.lib().qvmhip_apply_kraus_choice(self._h, N.dptr(K.view(np.float64)), len(K), k, N.u32ptr(q),
+                                                  float(r), C.byref(out)))
+        return out.value
+
     def normalize(self, length: float = 0.0) -> None:
         N.check(N.lib().qvmhip_normalize(self._h, float(length)))
 
