@@ -25,7 +25,9 @@ ARCH = "gfx950"
 SOURCES = {
     "api.hip": [],
     "gates.hip": ["-ffp-contract=off"],
-    "tile.hip": ["-ffp-contract=off"],
+    # every branch of the tile kernels' op loop is uniform: left unstructured,
+    # an op's arm goes straight back to the loop and the block stays in place
+    "tile.hip": ["-ffp-contract=off", "-mllvm", "-structurizecfg-skip-uniform-regions=true"],
     "reduce.hip": ["-ffp-contract=off"],
     "fused.hip": [],
     "channel.hip": ["-ffp-contract=off"],

@@ -294,7 +294,7 @@ int qvmhip_apply_tile_pass(qvmhip_state *s, uint32_t m, const uint32_t *tile_qub
     if (!rc) rc = check_tile_globals(s->n, m, tile_qubits, nops, ops);
     if (rc) return rc;
     if (nops == 0) return QVMHIP_OK;
-    return launch_tile_pass(s, m, tile_qubits, nops, ops, 0);
+    return launch_tile_pass(s, m, tile_qubits, nops, ops);
 }
 
 int qvmhip_tile_schedule(int dtype, uint32_t flags, uint32_t m, uint32_t nops, const qvmhip_tile_op *ops,

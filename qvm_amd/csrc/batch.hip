@@ -28,7 +28,6 @@ struct BItem {
     uint32_t k = 0;            // tile m or gate width
     uint32_t qubits[16] = {0};
     size_t op_off = 0;         // tile ops in blob
-    uint32_t nops = 0;
     bool cut = false;          // tile ops hold CUT_PHASE ops
     std::vector<double> U;     // gate matrix (k <= 3)
 };
@@ -351,11 +350,9 @@ int qvmhip_batch_add_tile_pass(qvmhip_batch *b, uint32_t inst, uint32_t m, const
     it.kind = kItemTile;
     it.k = m;
     std::copy(tile_qubits, tile_qubits + m, it.qubits);
-    std::vector<qvmhip_tile_op> sched;
-    schedule_tile_ops(b->dtype, (b->flags & QVMHIP_FLAG_FMA_TILES) != 0, m, ops, nops, sched);
-    it.nops = (uint32_t)sched.size();
-    it.cut = tile_ops_have_cut(sched.data(), sched.size());
-    it.op_off = push(b->blob, sched.data(), sizeof(qvmhip_tile_op) * sched.size());
+    const TileCode code = compile_tile_ops(b->dtype, (b->flags & QVMHIP_FLAG_FMA_TILES) != 0, m, ops, nops);
+    it.cut = code.cut;
+    it.op_off = push(b->blob, code.bytes.data(), code.bytes.size());
     b->prog[inst].push_back(std::move(it));
     return QVMHIP_OK;
 }
@@ -475,7 +472,7 @@ int qvmhip_batch_finalize(qvmhip_batch *b, int use_graph) {
                 bl.zero = bl.zero || from_zero || zero_mask != 0;
                 const uint64_t nb = build_tile_entry(
                     ent.data(), b->dtype, (b->flags & QVMHIP_FLAG_FMA_TILES) != 0, b->nq[i], it.k, it.qubits,
-                    b->offset[i], blocks, it.op_off, it.nops, kTilesPerBlock, from_zero, zero_mask);
+                    b->offset[i], blocks, it.op_off, kTilesPerBlock, from_zero, zero_mask);
                 b->entries.insert(b->entries.end(), ent.begin(), ent.end());
                 b->blkmap.insert(b->blkmap.end(), (size_t)nb, local);
                 blocks += nb;

@@ -271,13 +271,16 @@ int launch_sample_search(hipStream_t st, int dtype, const void *amps, uint64_t l
                          const double *u, uint64_t nshots, int rule_ge, uint64_t *out, double eps,
                          uint8_t *near_flags, unsigned long long *near_count);
 int collapse_to_basis(qvmhip_state *s, const uint64_t *index_dev);
-// ops_on_device = 0: public ops on the host (scheduled here); 1: an already
-// scheduled program on the device.
-// cut: an already scheduled program holds CUT_PHASE ops (for host ops the
-// scheduler's output decides).
+// A tile pass's op list as the kernels run it (any host or device memory).
+struct TileCode {
+    std::vector<char> bytes;
+    bool cut = false;  // holds CUT_PHASE ops
+};
+TileCode compile_tile_ops(int dtype, bool fma, uint32_t m, const qvmhip_tile_op *ops, uint32_t nops);
+// public ops on the host / a compiled list on the device
 int launch_tile_pass(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, uint32_t nops,
-                     const qvmhip_tile_op *ops_dev_or_host, int ops_on_device, bool cut = false);
-bool tile_ops_have_cut(const qvmhip_tile_op *ops, size_t n);
+                     const qvmhip_tile_op *ops);
+int launch_tile_code(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, const void *code_dev, bool cut);
 int launch_fused_dense(qvmhip_state *s, const void *mat_dev, uint32_t k, const uint32_t *qubits);
 int expectation_zz(qvmhip_state *s, const uint32_t *edges, uint32_t nedges, double *out);
 int inner_product(qvmhip_state *a, qvmhip_state *b, double *re, double *im);
@@ -328,8 +331,8 @@ size_t tile_entry_bytes();
 // tiles_per_block tiles.  zero_mask: state qubits untouched before this pass
 // of a run that starts from |0...0> (blocks with one of them set are zero).
 uint64_t build_tile_entry(void *entry, int dtype, bool fma, uint32_t n, uint32_t m, const uint32_t *tq,
-                          uint64_t amp_offset, uint64_t block_start, uint64_t op_off, uint32_t nops,
-                          uint32_t tiles_per_block, bool from_zero, uint64_t zero_mask);
+                          uint64_t amp_offset, uint64_t block_start, uint64_t op_off, uint32_t tiles_per_block,
+                          bool from_zero, uint64_t zero_mask);
 // op_buf: the device buffer the entries' op offsets point into
 // cut: some entry of the launch holds CUT_PHASE ops
 // zero: some entry starts from |0...0> or has a nonzero zero_mask

@@ -56,6 +56,7 @@ constexpr uint32_t kTileD1RX = 21;
 constexpr uint32_t kTileCutPhase = 22;
 constexpr uint32_t kTileData = 23;
 constexpr int kCutMaxEdges = 32;
+constexpr int kCutHeader = 192;  // bytes of CUT_PHASE before its table in a packed program
 
 // Register bits per thread (measured on MI355X): 3 (8 amplitudes) for FP64
 // and for exact FP32, 4 (16) for FP32 with FMA contraction; fewer for small
@@ -82,44 +83,168 @@ __device__ inline uint64_t thread_offset(const TileArgs &a, uint32_t t) {
 __device__ __forceinline__ double qfma(double a, double b, double c) { return __builtin_fma(a, b, c); }
 __device__ __forceinline__ float qfma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
-// Complex product.  FMA = false: four separately rounded products, as the
-// plain kernels; FMA = true: one product and one fused multiply-add per part.
-template <typename T, bool FMA = false>
-__device__ __forceinline__ void cmul(T ar, T ai, T br, T bi, T &r, T &i) {
-    if constexpr (FMA) {
-        r = qfma(ar, br, -(ai * bi));
-        i = qfma(ar, bi, ai * br);
-    } else {
-        r = ar * br - ai * bi;
-        i = ar * bi + ai * br;
-    }
-}
-
-// y = a*u + b*v (complex): the sum of two rounded products, or (FMA) one
-// product and three fused multiply-adds per part.
-template <typename T, bool FMA>
-__device__ __forceinline__ void cmac2(T ar, T ai, T ur, T ui, T br, T bi, T vr, T vi, T &yr, T &yi) {
-    if constexpr (FMA) {
-        yr = qfma(ar, ur, qfma(-ai, ui, qfma(br, vr, -(bi * vi))));
-        yi = qfma(ar, ui, qfma(ai, ur, qfma(br, vi, bi * vr)));
-    } else {
-        T p0r, p0i, p1r, p1i;
-        cmul(ar, ai, ur, ui, p0r, p0i);
-        cmul(br, bi, vr, vi, p1r, p1i);
-        yr = p0r + p1r;
-        yi = p0i + p1i;
-    }
-}
-
-// Operand i of a scheduled op: FP64 passes keep the doubles of the public op;
-// for FP32 passes the scheduler stores the values as floats in the same
-// bytes, so the kernel reads them without a conversion.
-template <typename T>
-__device__ __forceinline__ T mval(const qvmhip_tile_op &op, int i) {
-    if constexpr (sizeof(T) == 8)
-        return op.m[i];
+// a * b + c and a * b - c as instructions whose result the register allocator
+// may place freely.  For __builtin_fma the compiler picks the two-address
+// form, whose result takes the register of c: right for accumulating into c,
+// a copy of the block where the result replaces another component.  SC: b is
+// in scalar registers at FP64.  FP32 operands are always vector registers (see
+// operand()).
+template <bool SC = true>
+__device__ __forceinline__ double fma_to(double a, double b, double c) {
+    double r;
+    if constexpr (SC)
+        asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
     else
-        return ((const float *)op.m)[i];
+        asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+template <bool SC = true>
+__device__ __forceinline__ float fma_to(float a, float b, float c) {
+    float r;
+    asm("v_fma_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+template <bool SC = true>
+__device__ __forceinline__ double fms_to(double a, double b, double c) {
+    double r;
+    if constexpr (SC)
+        asm("v_fma_f64 %0, %1, %2, -%3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
+    else
+        asm("v_fma_f64 %0, %1, %2, -%3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+template <bool SC = true>
+__device__ __forceinline__ float fms_to(float a, float b, float c) {
+    float r;
+    asm("v_fma_f32 %0, %1, %2, -%3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// An op's coefficient as the arithmetic wants it: FP64 stays in scalar
+// registers, FP32 is moved to a vector register.  FP32 vector instructions
+// with a scalar operand issue at the FP64 rate, without one nearly twice as
+// fast (per op over 2^30 amplitudes: RX 113 -> 68 us, general 1q 224 -> 130).
+__device__ __forceinline__ double operand(double s) { return s; }
+__device__ __forceinline__ float operand(float s) {
+    float r;
+    asm("v_mov_b32 %0, %1" : "=v"(r) : "s"(s));
+    return r;
+}
+
+// A move the compiler cannot see through: keeps the block's components out of
+// the register tuples of the 16-byte loads and stores.
+__device__ __forceinline__ double vmov(double a) {
+    double r;
+    asm("v_mov_b64 %0, %1" : "=v"(r) : "v"(a));
+    return r;
+}
+
+// The arithmetic below is written as in-place updates in an order that needs
+// no copy of the block: a component is overwritten only by an instruction
+// after which its old value has no reader.  The compiler follows that order;
+// written as y = f(x) it kept old and new values side by side and moved one
+// of them back after every op.
+
+// x *= f (complex).  FMA = false: four separately rounded products, as the
+// plain kernels; FMA = true: one product and one fused multiply-add per part.
+// SC: f is in scalar registers.
+template <typename T, bool FMA, bool SC = false>
+__device__ __forceinline__ void cmul(vec2_t<T> &x, T fr, T fi) {
+    if constexpr (FMA) {
+        const T t = x.y * fi;
+        x.y = x.y * fr;
+        x.y = qfma(x.x, fi, x.y);
+        x.x = fms_to<SC>(x.x, fr, t);
+    } else {
+        const T t = x.y * fi, u = x.x * fi;
+        x.y = x.y * fr;
+        x.y = u + x.y;
+        x.x = x.x * fr;
+        x.x = x.x - t;
+    }
+}
+
+// (p, q) = (a p + s b q, c p + d q) for real a..d, s = +1 or -1 (NEG); each
+// output is its p term plus its q term, as the general complex form rounds it.
+template <typename T, bool FMA, bool NEG>
+__device__ __forceinline__ void rot2(T &p, T &q, T a, T b, T c, T d) {
+    if constexpr (FMA) {
+        const T t = q * b;
+        q = q * d;
+        q = qfma(p, c, q);
+        if constexpr (NEG)
+            p = fms_to(p, a, t);
+        else
+            p = fma_to(p, a, t);
+    } else {
+        const T t = q * b, u = p * c;
+        q = q * d;
+        q = u + q;
+        p = p * a;
+        p = NEG ? p - t : p + t;
+    }
+}
+
+// What the kernels run: the scheduled op list packed into 80-byte slots
+// (pack_tile_ops).  `f` says what to do with one bit per case, tested in turn
+// as nested one-armed ifs.  A switch over op kinds looks simpler and costs
+// far more: the block (32 VGPRs at FP64) is then a value merged from many
+// arms, of which the compiler keeps old and new copies -- it moved the whole
+// block twice per op and needed 95 VGPRs.  Operands are in the pass's type;
+// an op with more than 64 bytes of them runs on into the following slots
+// (`f` >> 28 of them).
+struct TileDevOp {
+    uint32_t f;
+    uint32_t a, b, c;  // lane mask, wanted lane bits, register mask (bit r: register r takes part)
+    double m[8];
+};
+static_assert(sizeof(TileDevOp) == 80, "slot size");
+
+enum : uint32_t {
+    kF_Bit0 = 1u << 0,   // the target is register bit 0 (.. 3)
+    kF_Gen = 1u << 4,    // 1q: general
+    kF_GenC = 1u << 5,   // 1q: general, where lane and register controls hold
+    kF_Real = 1u << 6,   // 1q: real entries
+    kF_RX = 1u << 7,     // 1q: real diagonal, imaginary off-diagonal
+    kF_1q = 0xF0u,
+    kF_X = 1u << 8,      // exchange register pairs where the lane condition holds
+    kF_DL = 1u << 9,     // diagonal: one of two entries per lane, on registers c
+    kF_DL4 = 1u << 10,   // diagonal: one of four entries per lane (bits a & 0xff, a >> 8)
+    kF_DR = 1u << 11,    // diagonal: entry by lane condition and target register bit
+    kF_RDiag = 1u << 12, // diagonal: entry r on register r
+    kF_Out = 1u << 13,   // with DL / DR: qubits outside the tile select the entry pair
+    kF_Diag = kF_DL | kF_DL4 | kF_DR | kF_RDiag,
+    kF_Remap = 1u << 14,
+    kF_Dense2 = 1u << 15,
+    kF_Dense2C = 1u << 16,
+    kF_SwapC = 1u << 17,
+    kF_RSwap = 1u << 18,
+    kF_Cut = 1u << 19,
+    kF_Rare = kF_Dense2 | kF_Dense2C | kF_SwapC | kF_RSwap | kF_Cut,
+    kF_End = 1u << 20,
+};
+
+// The 80 bytes of a slot, loaded as scalars one op ahead (as 64-bit words:
+// half the scalar moves when the next op becomes the current one).
+struct TileHead {
+    uint64_t w[10];
+    __device__ __forceinline__ uint32_t f() const { return (uint32_t)w[0]; }
+    __device__ __forceinline__ uint32_t a() const { return (uint32_t)(w[0] >> 32); }
+    __device__ __forceinline__ uint32_t b() const { return (uint32_t)w[1]; }
+    __device__ __forceinline__ uint32_t c() const { return (uint32_t)(w[1] >> 32); }
+    template <typename T>
+    __device__ __forceinline__ T m(int i) const {
+        if constexpr (sizeof(T) == 8)
+            return __longlong_as_double((long long)w[2 + i]);
+        else
+            return operand(__uint_as_float((uint32_t)(w[2 + i / 2] >> (32 * (i & 1)))));
+    }
+};
+
+// Operands of an op that is not only its own slot long.
+template <typename T>
+__device__ __forceinline__ const T *operands(const TileDevOp *op) {
+    return reinterpret_cast<const T *>(op->m);
 }
 
 // register index with a zero inserted at bit I
@@ -138,67 +263,81 @@ __device__ __forceinline__ vec2_t<T> vsel(bool c, vec2_t<T> a, vec2_t<T> b) {
 
 // The register ops compute every pair unconditionally and, for controlled
 // ops (CTRL), keep the old values by selection where the control bits are not
-// all 1 (lane part lane_ok, register part rcm): straight-line code, so the
-// pairs of all registers interleave.
+// all 1 (lane part lane_ok, register part in the op's register mask):
+// straight-line code, so the pairs of all registers interleave.
 
+// (xa, xb) = U (xa, xb), each output the sum of its rounded products in
+// column order or (FMA) one product and three fused multiply-adds.
 template <typename T, int R, int I, bool CTRL, bool FMA>
-__device__ __forceinline__ void reg_dense1(vec2_t<T> (&x)[R], const qvmhip_tile_op &op, bool lane_ok,
-                                           uint32_t rcm) {
+__device__ __forceinline__ void reg_dense1(vec2_t<T> (&x)[R], const TileHead &h, bool lane_ok) {
     using V = vec2_t<T>;
-    const T u00r = mval<T>(op, 0), u00i = mval<T>(op, 1), u01r = mval<T>(op, 2), u01i = mval<T>(op, 3);
-    const T u10r = mval<T>(op, 4), u10i = mval<T>(op, 5), u11r = mval<T>(op, 6), u11i = mval<T>(op, 7);
+    const T u00r = h.m<T>(0), u00i = h.m<T>(1), u01r = h.m<T>(2), u01i = h.m<T>(3);
+    const T u10r = h.m<T>(4), u10i = h.m<T>(5), u11r = h.m<T>(6), u11i = h.m<T>(7);
 #pragma unroll
     for (int p = 0; p < R / 2; ++p) {
-        const int ra = rins0<I>(p), rb = ra | (1 << I);
-        const V xa = x[ra], xb = x[rb];
-        V ya, yb;
-        cmac2<T, FMA>(xa.x, xa.y, u00r, u00i, xb.x, xb.y, u01r, u01i, ya.x, ya.y);
-        cmac2<T, FMA>(xa.x, xa.y, u10r, u10i, xb.x, xb.y, u11r, u11i, yb.x, yb.y);
-        if constexpr (CTRL) {
-            const bool ok = lane_ok && ((uint32_t)ra & rcm) == rcm;
-            x[ra] = vsel<T>(ok, ya, xa);
-            x[rb] = vsel<T>(ok, yb, xb);
+        V &a = x[rins0<I>(p)], &b = x[rins0<I>(p) | (1 << I)];
+        const V a0 = a, b0 = b;
+        if constexpr (FMA) {
+            T tr = qfma(b.x, u01r, -(b.y * u01i));
+            T ti = qfma(b.x, u01i, b.y * u01r);
+            cmul<T, true, true>(b, u11r, u11i);
+            b.x = qfma(-a.y, u10i, b.x);
+            b.y = qfma(a.y, u10r, b.y);
+            b.x = qfma(a.x, u10r, b.x);
+            b.y = qfma(a.x, u10i, b.y);
+            tr = qfma(-a.y, u00i, tr);
+            ti = qfma(a.y, u00r, ti);
+            a.y = fma_to(a.x, u00i, ti);
+            a.x = fma_to(a.x, u00r, tr);
         } else {
-            x[ra] = ya;
-            x[rb] = yb;
+            V s = b, t = a;
+            cmul<T, false>(s, u01r, u01i);
+            cmul<T, false>(b, u11r, u11i);
+            cmul<T, false>(t, u10r, u10i);
+            b.x = t.x + b.x;
+            b.y = t.y + b.y;
+            cmul<T, false>(a, u00r, u00i);
+            a.x = a.x + s.x;
+            a.y = a.y + s.y;
+        }
+        if constexpr (CTRL) {
+            const bool ok = lane_ok && ((h.c() >> rins0<I>(p)) & 1u);
+            a = vsel<T>(ok, a, a0);
+            b = vsel<T>(ok, b, b0);
         }
     }
 }
 
 // 4x4 on register bits 0 (matrix bit 0) and 1 (matrix bit 1)
 template <typename T, int R, bool CTRL, bool FMA>
-__device__ __forceinline__ void reg_dense2(vec2_t<T> (&x)[R], const qvmhip_tile_op &op, bool lane_ok,
-                                           uint32_t rcm) {
+__device__ __forceinline__ void reg_dense2(vec2_t<T> (&x)[R], const T *__restrict__ u, bool lane_ok, uint32_t regs) {
     using V = vec2_t<T>;
 #pragma unroll
     for (int p = 0; p < R / 4; ++p) {
         const int r0 = p << 2;
-        V in[4], out[4];
+        V in[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) in[j] = x[r0 | j];
+        const bool ok = !CTRL || (lane_ok && ((regs >> r0) & 1u));
 #pragma unroll
         for (int row = 0; row < 4; ++row) {
-            T yr, yi;
-            cmul<T, FMA>(in[0].x, in[0].y, mval<T>(op, 8 * row), mval<T>(op, 8 * row + 1), yr, yi);
+            V y = in[0];
+            cmul<T, FMA>(y, u[8 * row], u[8 * row + 1]);
 #pragma unroll
             for (int c = 1; c < 4; ++c) {
-                const T ur = mval<T>(op, 8 * row + 2 * c), ui = mval<T>(op, 8 * row + 2 * c + 1);
+                const T ur = u[8 * row + 2 * c], ui = u[8 * row + 2 * c + 1];
                 if constexpr (FMA) {
-                    yr = qfma(in[c].x, ur, qfma(-in[c].y, ui, yr));
-                    yi = qfma(in[c].x, ui, qfma(in[c].y, ur, yi));
+                    y.x = qfma(in[c].x, ur, qfma(-in[c].y, ui, y.x));
+                    y.y = qfma(in[c].x, ui, qfma(in[c].y, ur, y.y));
                 } else {
-                    T pr, pi;
-                    cmul(in[c].x, in[c].y, ur, ui, pr, pi);
-                    yr = yr + pr;
-                    yi = yi + pi;
+                    V p = in[c];
+                    cmul<T, false>(p, ur, ui);
+                    y.x = y.x + p.x;
+                    y.y = y.y + p.y;
                 }
             }
-            out[row].x = yr;
-            out[row].y = yi;
+            x[r0 | row] = CTRL ? vsel<T>(ok, y, in[row]) : y;
         }
-        const bool ok = !CTRL || (lane_ok && ((uint32_t)r0 & rcm) == rcm);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) x[r0 | j] = CTRL ? vsel<T>(ok, out[j], in[j]) : out[j];
     }
 }
 
@@ -209,25 +348,11 @@ __device__ __forceinline__ void reg_dense2(vec2_t<T> (&x)[R], const qvmhip_tile_
 // result may differ in its sign only).  Half the multiplies of reg_dense1.
 template <typename T, int R, int I, bool FMA>
 __device__ __forceinline__ void reg_dense1_real(vec2_t<T> (&x)[R], T u00, T u01, T u10, T u11) {
-    using V = vec2_t<T>;
 #pragma unroll
     for (int p = 0; p < R / 2; ++p) {
-        const int ra = rins0<I>(p), rb = ra | (1 << I);
-        const V xa = x[ra], xb = x[rb];
-        V ya, yb;
-        if constexpr (FMA) {
-            ya.x = qfma(xa.x, u00, xb.x * u01);
-            ya.y = qfma(xa.y, u00, xb.y * u01);
-            yb.x = qfma(xa.x, u10, xb.x * u11);
-            yb.y = qfma(xa.y, u10, xb.y * u11);
-        } else {
-            ya.x = xa.x * u00 + xb.x * u01;
-            ya.y = xa.y * u00 + xb.y * u01;
-            yb.x = xa.x * u10 + xb.x * u11;
-            yb.y = xa.y * u10 + xb.y * u11;
-        }
-        x[ra] = ya;
-        x[rb] = yb;
+        vec2_t<T> &a = x[rins0<I>(p)], &b = x[rins0<I>(p) | (1 << I)];
+        rot2<T, FMA, false>(a.x, b.x, u00, u01, u10, u11);
+        rot2<T, FMA, false>(a.y, b.y, u00, u01, u10, u11);
     }
 }
 
@@ -235,36 +360,33 @@ __device__ __forceinline__ void reg_dense1_real(vec2_t<T> (&x)[R], T u00, T u01,
 // ya = (a xa.re - b xb.im, a xa.im + b xb.re), yb = (d xb.re - c xa.im,
 // d xb.im + c xa.re), each sum in the general form's order.
 template <typename T, int R, int I, bool FMA>
-__device__ __forceinline__ void reg_dense1_rx(vec2_t<T> (&x)[R], T a, T b, T c, T d) {
-    using V = vec2_t<T>;
+__device__ __forceinline__ void reg_dense1_rx(vec2_t<T> (&x)[R], T u00, T u01, T u10, T u11) {
 #pragma unroll
     for (int p = 0; p < R / 2; ++p) {
-        const int ra = rins0<I>(p), rb = ra | (1 << I);
-        const V xa = x[ra], xb = x[rb];
-        V ya, yb;
+        vec2_t<T> &a = x[rins0<I>(p)], &b = x[rins0<I>(p) | (1 << I)];
+        rot2<T, FMA, true>(a.x, b.y, u00, u01, u10, u11);
         if constexpr (FMA) {
-            ya.x = qfma(xa.x, a, -(xb.y * b));
-            ya.y = qfma(xa.y, a, xb.x * b);
-            yb.x = qfma(-xa.y, c, xb.x * d);
-            yb.y = qfma(xa.x, c, xb.y * d);
+            const T t = b.x * u01;
+            b.x = b.x * u11;
+            b.x = qfma(-a.y, u10, b.x);
+            a.y = fma_to(a.y, u00, t);
         } else {
-            ya.x = xa.x * a - xb.y * b;
-            ya.y = xa.y * a + xb.x * b;
-            yb.x = xb.x * d - xa.y * c;
-            yb.y = xa.x * c + xb.y * d;
+            const T t = b.x * u01, s = a.y * u10;
+            b.x = b.x * u11;
+            b.x = b.x - s;
+            a.y = a.y * u00;
+            a.y = a.y + t;
         }
-        x[ra] = ya;
-        x[rb] = yb;
     }
 }
 
 template <typename T, int R, int I>
-__device__ __forceinline__ void reg_x(vec2_t<T> (&x)[R], bool lane_ok, uint32_t rcm) {
+__device__ __forceinline__ void reg_x(vec2_t<T> (&x)[R], bool lane_ok, uint32_t regs) {
     using V = vec2_t<T>;
 #pragma unroll
     for (int p = 0; p < R / 2; ++p) {
         const int ra = rins0<I>(p), rb = ra | (1 << I);
-        const bool ok = lane_ok && ((uint32_t)ra & rcm) == rcm;
+        const bool ok = lane_ok && ((regs >> ra) & 1u);
         const V xa = x[ra], xb = x[rb];
         x[ra] = vsel<T>(ok, xb, xa);
         x[rb] = vsel<T>(ok, xa, xb);
@@ -273,12 +395,12 @@ __device__ __forceinline__ void reg_x(vec2_t<T> (&x)[R], bool lane_ok, uint32_t 
 
 // controlled SWAP of register bits 0 and 1
 template <typename T, int R>
-__device__ __forceinline__ void reg_swap01(vec2_t<T> (&x)[R], bool lane_ok, uint32_t rcm) {
+__device__ __forceinline__ void reg_swap01(vec2_t<T> (&x)[R], bool lane_ok, uint32_t regs) {
     using V = vec2_t<T>;
 #pragma unroll
     for (int p = 0; p < R / 4; ++p) {
         const int r0 = p << 2;
-        const bool ok = lane_ok && ((uint32_t)r0 & rcm) == rcm;
+        const bool ok = lane_ok && ((regs >> r0) & 1u);
         const V a = x[r0 | 1], b = x[r0 | 2];
         x[r0 | 1] = vsel<T>(ok, b, a);
         x[r0 | 2] = vsel<T>(ok, a, b);
@@ -302,46 +424,41 @@ __device__ __forceinline__ void reg_rswap(vec2_t<T> (&x)[R]) {
 }
 
 template <typename T, int R>
-__device__ __forceinline__ void reg_rswap_any(vec2_t<T> (&x)[R], uint32_t a, uint32_t b) {
-    const uint32_t code = a * 8 + b;
-    switch (code) {
-#define QH_RS(A, B)                                                 \
-    case A * 8 + B:                                                 \
-        if constexpr ((1 << B) < R) reg_rswap<T, R, A, B>(x);       \
-        break;
-        QH_RS(0, 1) QH_RS(0, 2) QH_RS(0, 3) QH_RS(0, 4) QH_RS(1, 2) QH_RS(1, 3) QH_RS(1, 4)
-        QH_RS(2, 3) QH_RS(2, 4) QH_RS(3, 4)
+__device__ __forceinline__ void reg_rswap_any(vec2_t<T> (&x)[R], uint32_t pair) {
+#define QH_RS(BIT, A, B)                                        \
+    if constexpr ((1 << B) < R) {                               \
+        if ((pair >> BIT) & 1u) reg_rswap<T, R, A, B>(x);       \
+    }
+    QH_RS(0, 0, 1) QH_RS(1, 0, 2) QH_RS(2, 0, 3) QH_RS(3, 1, 2) QH_RS(4, 1, 3) QH_RS(5, 2, 3)
 #undef QH_RS
-        default: break;
+}
+
+// Diagonals.  A diagonal's index has a lane part (the same for all registers)
+// and a register part.  No case needs a per-register vector select: the lane
+// part picks one entry (or two) per lane once per op, and the register part
+// is a scalar choice or a compile-time one.  Registers outside `regs` are
+// skipped; a lane whose condition fails multiplies by exactly 1, which leaves
+// its amplitude's value unchanged.
+template <typename T, int R, bool FMA>
+__device__ __forceinline__ void diag_lane(vec2_t<T> (&x)[R], T dr, T di, uint32_t regs) {
+    if (regs == (1u << R) - 1u) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) cmul<T, FMA>(x[r], dr, di);
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if ((regs >> r) & 1u) cmul<T, FMA>(x[r], dr, di);
     }
 }
 
-// 4-way select of a complex entry of m by a (per-lane) index j
-template <typename T>
-__device__ __forceinline__ void pick4(const qvmhip_tile_op &op, uint32_t j, T &dr, T &di) {
-    const T r0 = mval<T>(op, 0), i0 = mval<T>(op, 1), r1 = mval<T>(op, 2), i1 = mval<T>(op, 3);
-    const T r2 = mval<T>(op, 4), i2 = mval<T>(op, 5), r3 = mval<T>(op, 6), i3 = mval<T>(op, 7);
-    const T ra = (j & 1u) ? r1 : r0, ia = (j & 1u) ? i1 : i0;
-    const T rb = (j & 1u) ? r3 : r2, ib = (j & 1u) ? i3 : i2;
-    dr = (j & 2u) ? rb : ra;
-    di = (j & 2u) ? ib : ia;
-}
-
-// Register r takes entry (c1) when its bit RS is set, (c0) otherwise;
-// registers whose register-control bits (rcm) are not all set are skipped (a
-// uniform test).  Lane controls are folded into the entries by the caller.
+// Register r takes entry c1 when its bit RS is set, c0 otherwise.
 template <typename T, int R, int RS, bool FMA>
-__device__ __forceinline__ void diag_rbit(vec2_t<T> (&x)[R], T c0r, T c0i, T c1r, T c1i, uint32_t rcm) {
-    if constexpr ((1 << RS) < R) {
+__device__ __forceinline__ void diag_rbit(vec2_t<T> (&x)[R], T c0r, T c0i, T c1r, T c1i) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (((uint32_t)r & rcm) == rcm) {
-                const bool one = ((r >> RS) & 1) != 0;
-                vec2_t<T> y;
-                cmul<T, FMA>(x[r].x, x[r].y, one ? c1r : c0r, one ? c1i : c0i, y.x, y.y);
-                x[r] = y;
-            }
-        }
+    for (int r = 0; r < R; ++r) {
+        const bool one = ((r >> RS) & 1) != 0;
+        cmul<T, FMA>(x[r], one ? c1r : c0r, one ? c1i : c0i);
     }
 }
 
@@ -349,156 +466,72 @@ __device__ __forceinline__ void diag_rbit(vec2_t<T> (&x)[R], T c0r, T c0i, T c1r
 // all register bits, with its per-register entries worked out by the
 // scheduler.
 template <typename T, int R, bool FMA>
-__device__ __forceinline__ void reg_rdiag(vec2_t<T> (&x)[R], const qvmhip_tile_op &op) {
+__device__ __forceinline__ void reg_rdiag(vec2_t<T> (&x)[R], const T *__restrict__ d) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-        vec2_t<T> y;
-        cmul<T, FMA>(x[r].x, x[r].y, mval<T>(op, 2 * r), mval<T>(op, 2 * r + 1), y.x, y.y);
-        x[r] = y;
-    }
+    for (int r = 0; r < R; ++r) cmul<T, FMA, true>(x[r], operand(d[2 * r]), operand(d[2 * r + 1]));
 }
 
-// diagonal 1q / 2q and CPHASE on any slot bits.  The diagonal index has a
-// lane part (target bits that are thread bits, the same for all registers)
-// and a register part (uniform per register).  No case needs a per-register
-// vector select: the lane part picks one entry (or two) per lane once per op,
-// a lane control (or CPHASE condition) turns a lane's entry into 1, register
-// controls skip whole registers, and the register part is a scalar choice or,
-// for one lane and one register bit, a compile-time one (switch on the
-// register bit).  A lane whose condition fails multiplies by exactly 1, which
-// leaves its amplitude's value unchanged.
-template <typename T, int R, int TB, bool CTRL, bool FMA>
-__device__ __forceinline__ void reg_diag(vec2_t<T> (&x)[R], const qvmhip_tile_op &op, uint32_t t, bool lane_ok,
-                                         uint32_t rcm_in) {
-    using V = vec2_t<T>;
-    const uint32_t kind = op.kind, q0 = op.q0, q1 = op.q1;
-    constexpr uint32_t lanes = (1u << TB) - 1u;
-    const uint32_t rcm = CTRL ? rcm_in : 0u;
-    if (kind == QVMHIP_TILE_CPHASE) {
-        const uint32_t need = op.ctrl_mask | (1u << q0) | (1u << q1);
-        const uint32_t rn = need >> TB, ln = need & lanes;
-        T fr = mval<T>(op, 0), fi = mval<T>(op, 1);
-        if (ln) {
-            const bool lok = (t & ln) == ln;
-            fr = lok ? fr : T(1);
-            fi = lok ? fi : T(0);
-        }
+// DL, DL4, DR and RDIAG (see the flags).  Out: the bits of the block's base
+// index named by b (g0 | g1 << 8 | count << 16) select one of the op's entry
+// pairs; c has bit `sel` set where that pair is (1, 1), which is skipped.
+template <typename T, int R, bool FMA>
+__device__ __forceinline__ void reg_diag(vec2_t<T> (&x)[R], const TileHead &h, const TileDevOp *__restrict__ op,
+                                         uint32_t t, uint64_t gb) {
+    const uint32_t f = h.f();
+    if (f & kF_RDiag) {
+        reg_rdiag<T, R, FMA>(x, operands<T>(op));
+    } else if (f & kF_DL4) {
+        const bool b0 = ((t >> (h.a() & 0xFFu)) & 1u) != 0, b1 = ((t >> (h.a() >> 8)) & 1u) != 0;
+        const T ra = b0 ? h.m<T>(2) : h.m<T>(0), ia = b0 ? h.m<T>(3) : h.m<T>(1);
+        const T rb = b0 ? h.m<T>(6) : h.m<T>(4), ib = b0 ? h.m<T>(7) : h.m<T>(5);
+        diag_lane<T, R, FMA>(x, b1 ? rb : ra, b1 ? ib : ia, (1u << R) - 1u);
+    } else {
+        T e[4] = {h.m<T>(0), h.m<T>(1), h.m<T>(2), h.m<T>(3)};
+        uint32_t want = h.b(), regs = h.c();
+        bool go = true;
+        if (f & kF_Out) {
+            const uint32_t d = h.b();
+            uint32_t sel = (uint32_t)(gb >> (d & 63u)) & 1u;
+            if ((d >> 16) == 2u) sel |= ((uint32_t)(gb >> ((d >> 8) & 63u)) & 1u) << 1;
+            const T *m = operands<T>(op) + 4 * sel;
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (((uint32_t)r & rn) == rn) {
-                V y;
-                cmul<T, FMA>(x[r].x, x[r].y, fr, fi, y.x, y.y);
-                x[r] = y;
-            }
+            for (int i = 0; i < 4; ++i) e[i] = operand(m[i]);
+            go = ((regs >> sel) & 1u) == 0;
+            want = h.a();
+            regs = (1u << R) - 1u;
         }
-        return;
-    }
-    const bool two = kind == QVMHIP_TILE_DIAG2;
-    const bool reg0 = q0 >= TB, reg1 = two && q1 >= TB;
-    if (reg0 && (!two || reg1)) {
-        // index bits all on registers (the scheduler turns such ops into
-        // register diagonals unless a control bit is a lane bit)
-        const uint32_t rs0 = q0 - TB, rs1 = two ? q1 - TB : 0u;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (((uint32_t)r & rcm) == rcm) {
-                const uint32_t jr = (((uint32_t)r >> rs0) & 1u) | (two ? ((((uint32_t)r >> rs1) & 1u) << 1) : 0u);
-                T dr, di;
-                pick4<T>(op, jr, dr, di);
-                if constexpr (CTRL) {
-                    dr = lane_ok ? dr : T(1);
-                    di = lane_ok ? di : T(0);
+        if (go) {
+            const bool hit = (t & h.a()) == want;
+            if (f & kF_DL) {
+                diag_lane<T, R, FMA>(x, hit ? e[2] : e[0], hit ? e[3] : e[1], regs);
+            } else {
+                // entries (lane, register): e[0..3] without the lane condition, m[4..7] with it
+                T c0r = e[0], c0i = e[1], c1r = e[2], c1i = e[3];
+                if (!(f & kF_Out)) {
+                    c0r = hit ? h.m<T>(4) : c0r;
+                    c0i = hit ? h.m<T>(5) : c0i;
+                    c1r = hit ? h.m<T>(6) : c1r;
+                    c1i = hit ? h.m<T>(7) : c1i;
                 }
-                V y;
-                cmul<T, FMA>(x[r].x, x[r].y, dr, di, y.x, y.y);
-                x[r] = y;
+                if (f & (kF_Bit0 << 0)) {
+                    diag_rbit<T, R, 0, FMA>(x, c0r, c0i, c1r, c1i);
+                } else if (f & (kF_Bit0 << 1)) {
+                    diag_rbit<T, R, 1, FMA>(x, c0r, c0i, c1r, c1i);
+                } else if (f & (kF_Bit0 << 2)) {
+                    if constexpr (R > 4) diag_rbit<T, R, 2, FMA>(x, c0r, c0i, c1r, c1i);
+                } else {
+                    if constexpr (R > 8) diag_rbit<T, R, 3, FMA>(x, c0r, c0i, c1r, c1i);
+                }
             }
         }
-        return;
-    }
-    // lane part of the index
-    const uint32_t jl = (reg0 ? 0u : ((t >> q0) & 1u)) | ((two && !reg1) ? (((t >> q1) & 1u) << 1) : 0u);
-    if (!reg0 && !reg1) {
-        // index bits all on lanes: one entry per lane for every register
-        T dr, di;
-        if (two) {
-            pick4<T>(op, jl, dr, di);
-        } else {
-            dr = jl ? mval<T>(op, 2) : mval<T>(op, 0);
-            di = jl ? mval<T>(op, 3) : mval<T>(op, 1);
-        }
-        if constexpr (CTRL) {
-            dr = lane_ok ? dr : T(1);
-            di = lane_ok ? di : T(0);
-        }
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (((uint32_t)r & rcm) == rcm) {
-                V y;
-                cmul<T, FMA>(x[r].x, x[r].y, dr, di, y.x, y.y);
-                x[r] = y;
-            }
-        }
-        return;
-    }
-    // one lane bit and one register bit: two entries per lane, and the
-    // register bit (a compile-time position below) chooses between them
-    const uint32_t rs = reg0 ? q0 - TB : q1 - TB;
-    const uint32_t w = reg0 ? 1u : 2u;
-    T c0r, c0i, c1r, c1i;
-    pick4<T>(op, jl, c0r, c0i);
-    pick4<T>(op, jl | w, c1r, c1i);
-    if constexpr (CTRL) {
-        c0r = lane_ok ? c0r : T(1);
-        c0i = lane_ok ? c0i : T(0);
-        c1r = lane_ok ? c1r : T(1);
-        c1i = lane_ok ? c1i : T(0);
-    }
-    switch (rs) {
-        case 0: diag_rbit<T, R, 0, FMA>(x, c0r, c0i, c1r, c1i, rcm); break;
-        case 1: diag_rbit<T, R, 1, FMA>(x, c0r, c0i, c1r, c1i, rcm); break;
-        case 2: diag_rbit<T, R, 2, FMA>(x, c0r, c0i, c1r, c1i, rcm); break;
-        case 3: diag_rbit<T, R, 3, FMA>(x, c0r, c0i, c1r, c1i, rcm); break;
-        case 4: diag_rbit<T, R, 4, FMA>(x, c0r, c0i, c1r, c1i, rcm); break;
-        default: break;
     }
 }
 
-// Diagonal on local slot bit q0 whose entries also depend on state qubits
-// outside the tile: `sel` (their bits in the block's base index, uniform)
-// picks the entry pair (2 sel, 2 sel + 1), and q0 picks within it.
-template <typename T, int R, int TB, bool FMA>
-__device__ __forceinline__ void reg_gdiag(vec2_t<T> (&x)[R], const qvmhip_tile_op &op, uint32_t sel, uint32_t t) {
-    using V = vec2_t<T>;
-    const T r0 = mval<T>(op, 4 * sel), i0 = mval<T>(op, 4 * sel + 1);
-    const T r1 = mval<T>(op, 4 * sel + 2), i1 = mval<T>(op, 4 * sel + 3);
-    const uint32_t q0 = op.q0;
-    if (q0 >= TB) {
-        const uint32_t rs = q0 - TB;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const bool one = (((uint32_t)r >> rs) & 1u) != 0;  // uniform per register
-            V y;
-            cmul<T, FMA>(x[r].x, x[r].y, one ? r1 : r0, one ? i1 : i0, y.x, y.y);
-            x[r] = y;
-        }
-        return;
-    }
-    const bool one = ((t >> q0) & 1u) != 0;
-    const T dr = one ? r1 : r0, di = one ? i1 : i0;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        V y;
-        cmul<T, FMA>(x[r].x, x[r].y, dr, di, y.x, y.y);
-        x[r] = y;
-    }
-}
-
-// CUT_PHASE (the layout of its bytes is described at cut_phase_op): the
-// phase table T of the DATA ops after it goes to LDS, each thread counts the
+// CUT_PHASE (the layout of its bytes is described at cut_phase_op; the phase
+// table T follows them): T goes to LDS, each thread counts the
 // cut pairs of its amplitudes and multiplies register r by T[cut].
 template <typename T, int R, int TB, bool FMA>
-__device__ __forceinline__ void reg_cut_phase(vec2_t<T> (&x)[R], const qvmhip_tile_op *__restrict__ op,
+__device__ __forceinline__ void reg_cut_phase(vec2_t<T> (&x)[R], const TileDevOp *__restrict__ op,
                                               vec2_t<T> *sa, uint32_t t, uint64_t gb) {
     const uint8_t *b = (const uint8_t *)op->m;
     const uint32_t E = b[0];
@@ -506,13 +539,7 @@ __device__ __forceinline__ void reg_cut_phase(vec2_t<T> (&x)[R], const qvmhip_ti
     // they would hold registers through every other op)
     asm volatile("" : "+v"(t));
     __syncthreads();  // earlier readers of sa are done
-    if (t <= E) {
-        const qvmhip_tile_op &d = op[1 + t / 16];
-        vec2_t<T> v;
-        v.x = mval<T>(d, 2 * (t & 15u));
-        v.y = mval<T>(d, 2 * (t & 15u) + 1);
-        sa[t] = v;
-    }
+    if (t <= E) sa[t] = reinterpret_cast<const vec2_t<T> *>(b + kCutHeader)[t];
     uint32_t c = 0, A = 0;
 #pragma unroll 4  // by four: one scalar load per four pairs (a full unroll computed the pair terms ahead and spilled)
     for (uint32_t i = 0; i < E; ++i) {
@@ -530,9 +557,7 @@ __device__ __forceinline__ void reg_cut_phase(vec2_t<T> (&x)[R], const qvmhip_ti
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const vec2_t<T> f = sa[c + (uint32_t)__popc(A ^ B[r])];
-        vec2_t<T> y;
-        cmul<T, FMA>(x[r].x, x[r].y, f.x, f.y, y.x, y.y);
-        x[r] = y;
+        cmul<T, FMA>(x[r], f.x, f.y);
         __builtin_amdgcn_sched_barrier(0);  // one table read at a time: R reads ahead hold 2R registers
     }
 }
@@ -572,16 +597,6 @@ __device__ __forceinline__ void reg_remap(vec2_t<T> (&x)[R], T *sa, const uint32
             if ((r >> b) & 1) off |= pw[b];
         return lds_addr<TB>(base | off);
     };
-    if constexpr (sizeof(T) != 8) {
-        vec2_t<T> *sv = reinterpret_cast<vec2_t<T> *>(sa);
-        __syncthreads();  // readers of the previous layout are done with sa
-#pragma unroll
-        for (int r = 0; r < R; ++r) sv[t + (uint32_t)r * (NT + 1)] = x[r];
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < R; ++r) x[r] = sv[addr(r)];
-        return;
-    }
     __syncthreads();  // readers of the previous layout are done with sa
 #pragma unroll
     for (int r = 0; r < R; ++r) sa[t + (uint32_t)r * (NT + 1)] = x[r].x;
@@ -608,6 +623,13 @@ __device__ __forceinline__ void tile_load(const vec2_t<T> *__restrict__ psi, con
     const vec2_t<T> *p = psi + gb + toff;
 #pragma unroll
     for (int r = 0; r < (1 << RB); ++r) x[r] = ldg<true>(&p[a.roff[r]]);
+    if constexpr (sizeof(T) == 8) {
+#pragma unroll
+        for (int r = 0; r < (1 << RB); ++r) {
+            x[r].x = vmov(x[r].x);
+            x[r].y = vmov(x[r].y);
+        }
+    }
 }
 
 template <typename T, int M, int RB>
@@ -621,142 +643,100 @@ __device__ __forceinline__ void tile_store(vec2_t<T> *__restrict__ psi, const Ti
     asm volatile("" : "+v"(o));
     vec2_t<T> *p = psi + o;
 #pragma unroll
-    for (int r = 0; r < (1 << RB); ++r) stg<true>(&p[a.roff[r]], x[r]);
+    for (int r = 0; r < (1 << RB); ++r) {
+        vec2_t<T> v = x[r];
+        if constexpr (sizeof(T) == 8) {
+            v.x = vmov(v.x);
+            v.y = vmov(v.y);
+        }
+        stg<true>(&p[a.roff[r]], v);
+    }
 }
 
-// Run a scheduled op list on the block held in x.
+// Run a packed op list (ended by kF_End) on the block held in x.  Each op's
+// slot is loaded as scalars while the op before it runs: read on demand, the
+// load was a wait of some 500 cycles in every op.
 // CUT: the op list holds CUT_PHASE ops (FMA passes only).  Kernels without
 // them are built without that code: its registers and code size slow every
 // other op down.
 template <typename T, int M, int RB, bool FMA, bool CUT>
-__device__ inline void tile_ops(vec2_t<T> (&x)[1 << RB], const qvmhip_tile_op *__restrict__ ops, uint32_t nops,
-                                T *sa, uint64_t gb) {
+__device__ inline void tile_ops(vec2_t<T> (&x)[1 << RB], const TileDevOp *__restrict__ op, T *sa, uint64_t gb) {
     constexpr int R = 1 << RB, TB = M - RB;
     const uint32_t t = threadIdx.x;
-    for (uint32_t oi = 0; oi < nops; ++oi) {
-        const qvmhip_tile_op &op = ops[oi];
-        // the header and the first 32 operand bytes in one scalar load: the
-        // reduced 1q ops (most ops of a pass) then start after a single wait
-        struct Head48 {
-            uint32_t w[12];
-        };
-        const Head48 h48 = *reinterpret_cast<const Head48 *>(&op);
-        asm volatile("" ::"s"(h48.w[1]), "s"(h48.w[2]), "s"(h48.w[4]), "s"(h48.w[5]), "s"(h48.w[6]),
-                     "s"(h48.w[7]), "s"(h48.w[8]), "s"(h48.w[9]), "s"(h48.w[10]), "s"(h48.w[11]));
-        const uint4 hdr = make_uint4(h48.w[0], h48.w[1], h48.w[2], h48.w[3]);
-        auto coef = [&](int k) -> T {  // operand k of a reduced 1q op
-            if constexpr (sizeof(T) == 8)
-                return __hiloint2double((int)h48.w[5 + 2 * k], (int)h48.w[4 + 2 * k]);
-            else
-                return __uint_as_float(h48.w[4 + k]);
-        };
-        const uint32_t kind = hdr.x, cm = hdr.w;
-        const bool lane_ok = (t & cm) == (cm & ((1u << TB) - 1u));
-        const uint32_t rcm = cm >> TB;
-        const bool ctrl = cm != 0;
-        switch (kind) {
-            case QVMHIP_TILE_DENSE1:
-#define QH_D1(I)                                                             \
-    case I:                                                                  \
-        if constexpr (I < RB) {                                              \
-            if (ctrl)                                                        \
-                reg_dense1<T, R, I, true, FMA>(x, op, lane_ok, rcm);            \
-            else                                                             \
-                reg_dense1<T, R, I, false, FMA>(x, op, lane_ok, rcm);            \
-        }                                                                    \
-        break;
-                switch (hdr.y - TB) {
-                    QH_D1(0) QH_D1(1) QH_D1(2) QH_D1(3) QH_D1(4)
-                    default: break;
-                }
-#undef QH_D1
-                break;
-            case kTileD1Real:
-#define QH_D1R(I)                                                        \
-    case I:                                                              \
-        if constexpr (I < RB) reg_dense1_real<T, R, I, FMA>(x, coef(0), coef(1), coef(2), coef(3)); \
-        break;
-                switch (hdr.y - TB) {
-                    QH_D1R(0) QH_D1R(1) QH_D1R(2) QH_D1R(3) QH_D1R(4)
-                    default: break;
-                }
-#undef QH_D1R
-                break;
-            case kTileD1RX:
-#define QH_D1X(I)                                                        \
-    case I:                                                              \
-        if constexpr (I < RB) reg_dense1_rx<T, R, I, FMA>(x, coef(0), coef(1), coef(2), coef(3)); \
-        break;
-                switch (hdr.y - TB) {
-                    QH_D1X(0) QH_D1X(1) QH_D1X(2) QH_D1X(3) QH_D1X(4)
-                    default: break;
-                }
-#undef QH_D1X
-                break;
-            case QVMHIP_TILE_DENSE2:
-                if (ctrl)
-                    reg_dense2<T, R, true, FMA>(x, op, lane_ok, rcm);
-                else
-                    reg_dense2<T, R, false, FMA>(x, op, lane_ok, rcm);
-                break;
-            case kTileXReg:
-                switch (hdr.y - TB) {
-                    case 0: reg_x<T, R, 0>(x, lane_ok, rcm); break;
-                    case 1: reg_x<T, R, 1>(x, lane_ok, rcm); break;
-                    case 2: if constexpr (RB > 2) reg_x<T, R, 2>(x, lane_ok, rcm); break;
-                    case 3: if constexpr (RB > 3) reg_x<T, R, 3>(x, lane_ok, rcm); break;
-                    case 4: if constexpr (RB > 4) reg_x<T, R, 4>(x, lane_ok, rcm); break;
-                    default: break;
-                }
-                break;
-            case QVMHIP_TILE_SWAP:
-                reg_swap01<T, R>(x, lane_ok, rcm);
-                break;
-            case kTileRSwap:
-                reg_rswap_any<T, R>(x, hdr.y, hdr.z);
-                break;
-            case kTileRemap:
-                {
-                    const uint32_t src4[4] = {h48.w[4], h48.w[5], h48.w[6], h48.w[7]};
-                    reg_remap<T, R, TB>(x, sa, src4, t);
-                }
-                break;
-            case kTileRDiag:
-                reg_rdiag<T, R, FMA>(x, op);
-                break;
-            case QVMHIP_TILE_GDIAG: {
-                const uint32_t d = hdr.z;
-                uint32_t sel = (uint32_t)(gb >> (d & 63u)) & 1u;
-                if ((d >> 16) == 2u) sel |= ((uint32_t)(gb >> ((d >> 8) & 63u)) & 1u) << 1;
-                reg_gdiag<T, R, TB, FMA>(x, op, sel, t);
-                break;
-            }
-            default:  // DIAG1, DIAG2, CPHASE; CUT_PHASE (no case label of its own: each label
-                      // deepens the dispatch of every op)
-                if constexpr (FMA && CUT) {
-                    if (kind == kTileCutPhase) {
-                        reg_cut_phase<T, R, TB, FMA>(x, ops + oi, reinterpret_cast<vec2_t<T> *>(sa), t, gb);
-                        oi += ((const uint8_t *)op.m)[1];  // its DATA ops
-                        break;
-                    }
-                }
-                if (ctrl)
-                    reg_diag<T, R, TB, true, FMA>(x, op, t, lane_ok, rcm);
-                else
-                    reg_diag<T, R, TB, false, FMA>(x, op, t, lane_ok, rcm);
-                break;
-        }
+    TileHead h = *reinterpret_cast<const TileHead *>(op);
+    while (!(h.f() & kF_End)) {
+        const TileDevOp *next = op + 1 + (h.f() >> 28);
+        const TileHead hn = *reinterpret_cast<const TileHead *>(next);
+        const uint32_t f = h.f();
+// CALL(I) for the op's target register bit I
+#define QH_BITS(CALL)                          \
+    if (f & (kF_Bit0 << 0)) {                  \
+        CALL(0);                               \
+    } else if (f & (kF_Bit0 << 1)) {           \
+        if constexpr (RB > 1) CALL(1);         \
+    } else if (f & (kF_Bit0 << 2)) {           \
+        if constexpr (RB > 2) CALL(2);         \
+    } else {                                   \
+        if constexpr (RB > 3) CALL(3);         \
     }
-
+        if (f & kF_1q) {
+            if (f & kF_RX) {
+#define QH_C(I) reg_dense1_rx<T, R, I, FMA>(x, h.m<T>(0), h.m<T>(1), h.m<T>(2), h.m<T>(3))
+                QH_BITS(QH_C)
+#undef QH_C
+            } else if (f & kF_Gen) {
+#define QH_C(I) reg_dense1<T, R, I, false, FMA>(x, h, true)
+                QH_BITS(QH_C)
+#undef QH_C
+            } else if (f & kF_Real) {
+#define QH_C(I) reg_dense1_real<T, R, I, FMA>(x, h.m<T>(0), h.m<T>(1), h.m<T>(2), h.m<T>(3))
+                QH_BITS(QH_C)
+#undef QH_C
+            } else {
+                const bool lane_ok = (t & h.a()) == h.b();
+#define QH_C(I) reg_dense1<T, R, I, true, FMA>(x, h, lane_ok)
+                QH_BITS(QH_C)
+#undef QH_C
+            }
+        } else if (f & kF_Diag) {
+            reg_diag<T, R, FMA>(x, h, op, t, gb);
+        } else if (f & kF_X) {
+            const bool lane_ok = (t & h.a()) == h.b();
+#define QH_C(I) reg_x<T, R, I>(x, lane_ok, h.c())
+            QH_BITS(QH_C)
+#undef QH_C
+        } else if (f & kF_Remap) {
+            const uint32_t src4[4] = {(uint32_t)h.w[2], (uint32_t)(h.w[2] >> 32), (uint32_t)h.w[3],
+                                      (uint32_t)(h.w[3] >> 32)};
+            reg_remap<T, R, TB>(x, sa, src4, t);
+        } else {
+            const bool lane_ok = (t & h.a()) == h.b();
+            if (f & kF_Dense2) {
+                reg_dense2<T, R, false, FMA>(x, operands<T>(op), true, 0u);
+            } else if (f & kF_Dense2C) {
+                reg_dense2<T, R, true, FMA>(x, operands<T>(op), lane_ok, h.c());
+            } else if (f & kF_SwapC) {
+                reg_swap01<T, R>(x, lane_ok, h.c());
+            } else if (f & kF_RSwap) {
+                reg_rswap_any<T, R>(x, h.c());
+            } else {
+                if constexpr (FMA && CUT)
+                    reg_cut_phase<T, R, TB, FMA>(x, op, reinterpret_cast<vec2_t<T> *>(sa), t, gb);
+            }
+        }
+#undef QH_BITS
+        h = hn;
+        op = next;
+    }
 }
 
 template <typename T, int M, int RB, bool FMA, bool CUT>
 __global__ __launch_bounds__(1 << (M - RB)) void k_tile(vec2_t<T> *__restrict__ psi, const TileArgs a,
-                                                       const qvmhip_tile_op *__restrict__ ops, uint32_t nops) {
+                                                       const TileDevOp *__restrict__ ops) {
     using V = vec2_t<T>;
     // the remap buffer: 2^M + 2^RB reals for FP64 (one component at a time),
     // as many amplitudes for FP32
-    __shared__ __align__(16) T sa[(sizeof(T) == 8 ? 1 : 2) * ((1 << M) + (1 << RB))];
+    __shared__ __align__(16) T sa[(1 << M) + (1 << RB)];
     const uint64_t toff = thread_offset<M - RB>(a, threadIdx.x);
     // One tile per workgroup (grid-striding only past the dispatch limit):
     // many resident workgroups overlap each other's loads, ops and stores.
@@ -764,7 +744,7 @@ __global__ __launch_bounds__(1 << (M - RB)) void k_tile(vec2_t<T> *__restrict__ 
         V x[1 << RB];
         const uint64_t gb = group_base(a.g, tile);
         tile_load<T, M, RB>(psi, a, gb, toff, x);
-        tile_ops<T, M, RB, FMA, CUT>(x, ops, nops, sa, gb);
+        tile_ops<T, M, RB, FMA, CUT>(x, ops, sa, gb);
         tile_store<T, M, RB>(psi, a, gb, toff, x);
     }
 }
@@ -787,7 +767,6 @@ struct TileEntry {
     // run starts from |0...0>, so a block whose base index has one of them set
     // is all zeros before this pass, and every tile op keeps it zero
     uint64_t zero_mask;
-    uint32_t nops;
     uint32_t from_zero;    // 1: the state is |0...0>, built in registers instead of loaded
 };
 
@@ -805,7 +784,7 @@ __attribute__((amdgpu_waves_per_eu(FMA && sizeof(T) == 8 ? 5 : 1))) void k_tile_
     using V = vec2_t<T>;
     // the remap buffer: 2^M + 2^RB reals for FP64 (one component at a time),
     // as many amplitudes for FP32
-    __shared__ __align__(16) T sa[(sizeof(T) == 8 ? 1 : 2) * ((1 << M) + (1 << RB))];
+    __shared__ __align__(16) T sa[(1 << M) + (1 << RB)];
     // round robin over the XCDs (no xcd_block): work blocks of different
     // entries differ in cost, and contiguous shares per XCD measured 5-6 %
     // slower on the 512-instance QAOA batch
@@ -820,7 +799,7 @@ __attribute__((amdgpu_waves_per_eu(FMA && sizeof(T) == 8 ? 5 : 1))) void k_tile_
             const uint64_t gb = group_base(e.args.g, tile);
             if (!ZERO) {
                 tile_load<T, M, RB>(psi, e.args, gb, toff, x);
-                tile_ops<T, M, RB, FMA, CUT>(x, (const qvmhip_tile_op *)(op_buf + e.op_off), e.nops, sa, gb);
+                tile_ops<T, M, RB, FMA, CUT>(x, (const TileDevOp *)(op_buf + e.op_off), sa, gb);
                 tile_store<T, M, RB>(psi, e.args, gb, toff, x);
                 continue;
             }
@@ -845,7 +824,7 @@ __attribute__((amdgpu_waves_per_eu(FMA && sizeof(T) == 8 ? 5 : 1))) void k_tile_
             } else {
                 tile_load<T, M, RB>(psi, e.args, gb, toff, x);
             }
-            tile_ops<T, M, RB, FMA, CUT>(x, (const qvmhip_tile_op *)(op_buf + e.op_off), e.nops, sa, gb);
+            tile_ops<T, M, RB, FMA, CUT>(x, (const TileDevOp *)(op_buf + e.op_off), sa, gb);
             tile_store<T, M, RB>(psi, e.args, gb, toff, x);
         }
     }
@@ -1364,6 +1343,141 @@ void schedule_tile_ops(int dtype, bool fma, uint32_t m, const qvmhip_tile_op *in
     }
 }
 
+// Packs a scheduled program into the slots the kernels run.
+static void pack_tile_ops(int dtype, bool fma, uint32_t m, const std::vector<qvmhip_tile_op> &sched,
+                          std::vector<TileDevOp> &out) {
+    const bool f64 = dtype == QVMHIP_F64;
+    const size_t ts = f64 ? 8 : 4;
+    const uint32_t rb = (uint32_t)tile_reg_bits((int)m, f64, fma), tb = m - rb, R = 1u << rb;
+    const uint32_t lanes = (1u << tb) - 1u, all = (1u << R) - 1u;
+    // registers whose bits under rmask equal rwant
+    auto regs_with = [&](uint32_t rmask, uint32_t rwant) {
+        uint32_t o = 0;
+        for (uint32_t r = 0; r < R; ++r)
+            if ((r & rmask) == rwant) o |= 1u << r;
+        return o;
+    };
+    // operand i of a scheduled op (already floats for FP32 passes)
+    auto val = [&](const qvmhip_tile_op &o, int i) -> double {
+        return f64 ? o.m[i] : (double)reinterpret_cast<const float *>(o.m)[i];
+    };
+    auto emit = [&](uint32_t f, uint32_t a, uint32_t b, uint32_t c, const void *data, size_t bytes) {
+        const size_t slots = bytes <= 64 ? 1 : 1 + (bytes - 64 + sizeof(TileDevOp) - 1) / sizeof(TileDevOp);
+        const size_t at = out.size();
+        out.resize(at + slots);
+        std::memset(&out[at], 0, slots * sizeof(TileDevOp));
+        out[at].f = f | (uint32_t)((slots - 1) << 28);
+        out[at].a = a;
+        out[at].b = b;
+        out[at].c = c;
+        if (bytes) std::memcpy(out[at].m, data, bytes);
+    };
+    auto emit_vals = [&](uint32_t f, uint32_t a, uint32_t b, uint32_t c, const double *v, size_t count) {
+        if (f64) return emit(f, a, b, c, v, count * 8);
+        std::vector<float> w(v, v + count);
+        emit(f, a, b, c, w.data(), count * 4);
+    };
+    out.clear();
+    for (size_t i = 0; i < sched.size(); ++i) {
+        const qvmhip_tile_op &o = sched[i];
+        const uint32_t ln = o.ctrl_mask & lanes, rn = o.ctrl_mask >> tb;
+        const uint32_t bit = o.q0 >= tb && o.q0 < m ? kF_Bit0 << (o.q0 - tb) : 0u;
+        switch (o.kind) {
+            case QVMHIP_TILE_DENSE1:
+                emit((o.ctrl_mask ? kF_GenC : kF_Gen) | bit, ln, ln, regs_with(rn, rn), o.m, 8 * ts);
+                break;
+            case kTileD1Real: emit(kF_Real | bit, 0, 0, 0, o.m, 4 * ts); break;
+            case kTileD1RX: emit(kF_RX | bit, 0, 0, 0, o.m, 4 * ts); break;
+            case kTileXReg: emit(kF_X | bit, ln, ln, regs_with(rn, rn), nullptr, 0); break;
+            case kTileRDiag: emit(kF_RDiag, 0, 0, 0, o.m, 2 * R * ts); break;
+            case kTileRemap: emit(kF_Remap, 0, 0, 0, o.m, 16); break;
+            case QVMHIP_TILE_DENSE2:
+                emit(o.ctrl_mask ? kF_Dense2C : kF_Dense2, ln, ln, regs_with(rn, rn), o.m, 32 * ts);
+                break;
+            case QVMHIP_TILE_SWAP: emit(kF_SwapC, ln, ln, regs_with(rn, rn), nullptr, 0); break;
+            case kTileRSwap: {
+                static const uint32_t pairs[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
+                uint32_t c = 0;
+                for (uint32_t k = 0; k < 6; ++k)
+                    if (pairs[k][0] == o.q0 && pairs[k][1] == o.q1) c = 1u << k;
+                emit(kF_RSwap, 0, 0, c, nullptr, 0);
+                break;
+            }
+            case QVMHIP_TILE_GDIAG: {
+                const uint32_t ng = o.q1 >> 16, sels = 1u << ng;
+                uint32_t ident = 0;
+                for (uint32_t k = 0; k < sels; ++k)
+                    if (val(o, 4 * k) == 1.0 && val(o, 4 * k + 1) == 0.0 && val(o, 4 * k + 2) == 1.0 &&
+                        val(o, 4 * k + 3) == 0.0)
+                        ident |= 1u << k;
+                emit(kF_Out | (bit ? kF_DR | bit : kF_DL), bit ? 0u : 1u << o.q0, o.q1, ident, o.m, 4 * sels * ts);
+                break;
+            }
+            case kTileCutPhase: {
+                const uint8_t *b = (const uint8_t *)o.m;
+                const size_t E = b[0], ndata = b[1];
+                std::vector<char> d(kCutHeader + (E + 1) * 2 * ts);
+                std::memcpy(d.data(), o.m, kCutHeader);
+                for (size_t c = 0; c <= E; ++c)
+                    std::memcpy(d.data() + kCutHeader + c * 2 * ts,
+                                (const char *)sched[i + 1 + c / 16].m + (c % 16) * 2 * ts, 2 * ts);
+                emit(kF_Cut, 0, 0, 0, d.data(), d.size());
+                i += ndata;
+                break;
+            }
+            default: {  // DIAG1, DIAG2, CPHASE with at least one lane bit among targets and controls
+                const bool two = o.kind != QVMHIP_TILE_DIAG1;
+                const bool r0 = o.q0 >= tb, r1 = two && o.q1 >= tb;
+                if (o.kind != QVMHIP_TILE_CPHASE && o.ctrl_mask == 0) {
+                    if (!two) {
+                        emit(kF_DL, 1u << o.q0, 1u << o.q0, all, o.m, 4 * ts);
+                        break;
+                    }
+                    if (!r0 && !r1) {
+                        emit(kF_DL4, o.q0 | (o.q1 << 8), 0, 0, o.m, 8 * ts);
+                        break;
+                    }
+                    // one lane bit, one register bit: entries ordered (lane, register)
+                    double v[8];
+                    for (int l = 0; l < 2; ++l)
+                        for (int r = 0; r < 2; ++r) {
+                            const int j = r0 ? (r | (l << 1)) : (l | (r << 1));
+                            v[4 * l + 2 * r] = val(o, 2 * j);
+                            v[4 * l + 2 * r + 1] = val(o, 2 * j + 1);
+                        }
+                    const uint32_t lp = r0 ? o.q1 : o.q0, rp = (r0 ? o.q0 : o.q1) - tb;
+                    emit_vals(kF_DR | (kF_Bit0 << rp), 1u << lp, 1u << lp, 0, v, 8);
+                    break;
+                }
+                // every entry other than 1 multiplies where the target bits
+                // spell it and the controls hold
+                const uint32_t tmask = (1u << o.q0) | (two ? 1u << o.q1 : 0u);
+                const uint32_t entries = o.kind == QVMHIP_TILE_CPHASE ? 1u : two ? 4u : 2u;
+                for (uint32_t j = 0; j < entries; ++j) {
+                    const uint32_t jj = o.kind == QVMHIP_TILE_CPHASE ? 3u : j;
+                    const double v[4] = {1.0, 0.0, val(o, 2 * (int)j), val(o, 2 * (int)j + 1)};
+                    if (v[2] == 1.0 && v[3] == 0.0) continue;
+                    const uint32_t mask = o.ctrl_mask | tmask;
+                    const uint32_t want = o.ctrl_mask | ((jj & 1u) << o.q0) | (two ? ((jj >> 1) & 1u) << o.q1 : 0u);
+                    emit_vals(kF_DL, mask & lanes, want & lanes, regs_with(mask >> tb, want >> tb), v, 4);
+                }
+            }
+        }
+    }
+    emit(kF_End, 0, 0, 0, nullptr, 0);
+}
+
+TileCode compile_tile_ops(int dtype, bool fma, uint32_t m, const qvmhip_tile_op *ops, uint32_t nops) {
+    std::vector<qvmhip_tile_op> sched;
+    schedule_tile_ops(dtype, fma, m, ops, nops, sched);
+    std::vector<TileDevOp> packed;
+    pack_tile_ops(dtype, fma, m, sched, packed);
+    TileCode c;
+    c.bytes.assign((const char *)packed.data(), (const char *)(packed.data() + packed.size()));
+    for (const qvmhip_tile_op &o : sched) c.cut = c.cut || o.kind == kTileCutPhase;
+    return c;
+}
+
 namespace {
 
 // Host-side tile arguments of an n-qubit state and tile qubits tq[0..m).
@@ -1387,8 +1501,7 @@ void make_tile_args(uint32_t n, uint32_t m, const uint32_t *tq, int tb, TileArgs
 }
 
 template <typename T, int M, bool FMA, bool CUT>
-int run_tile(qvmhip_state *s, const uint32_t *tq, uint32_t m, const qvmhip_tile_op *ops_dev,
-             uint32_t nops) {
+int run_tile(qvmhip_state *s, const uint32_t *tq, uint32_t m, const TileDevOp *ops_dev) {
     constexpr int RB = tile_reg_bits(M, sizeof(T) == 8, FMA);
     constexpr int NT = 1 << (M - RB);
     TileArgs a;
@@ -1396,31 +1509,28 @@ int run_tile(qvmhip_state *s, const uint32_t *tq, uint32_t m, const qvmhip_tile_
     prof_begin(s, QVMHIP_K_TILE);
     const uint32_t grid = (uint32_t)std::min<uint64_t>(a.g.ngroups, kMaxGrid);
     hipLaunchKernelGGL((k_tile<T, M, RB, FMA, CUT>), dim3(grid), dim3(NT), 0, s->stream, (vec2_t<T> *)s->amps, a,
-                       ops_dev, nops);
+                       ops_dev);
     prof_end(s);
     QH_LAUNCH_CHECK();
     return QVMHIP_OK;
 }
 
 template <typename T, int M>
-int run_tile_f(qvmhip_state *s, const uint32_t *tq, uint32_t m, const qvmhip_tile_op *ops_dev, uint32_t nops,
-               bool cut) {
-    if (!(s->flags & QVMHIP_FLAG_FMA_TILES)) return run_tile<T, M, false, false>(s, tq, m, ops_dev, nops);
-    return cut ? run_tile<T, M, true, true>(s, tq, m, ops_dev, nops)
-               : run_tile<T, M, true, false>(s, tq, m, ops_dev, nops);
+int run_tile_f(qvmhip_state *s, const uint32_t *tq, uint32_t m, const TileDevOp *ops_dev, bool cut) {
+    if (!(s->flags & QVMHIP_FLAG_FMA_TILES)) return run_tile<T, M, false, false>(s, tq, m, ops_dev);
+    return cut ? run_tile<T, M, true, true>(s, tq, m, ops_dev) : run_tile<T, M, true, false>(s, tq, m, ops_dev);
 }
 
 template <typename T>
-int run_tile_m(qvmhip_state *s, uint32_t m, const uint32_t *tq, const qvmhip_tile_op *ops_dev,
-               uint32_t nops, bool cut) {
+int run_tile_m(qvmhip_state *s, uint32_t m, const uint32_t *tq, const TileDevOp *ops_dev, bool cut) {
     switch (m) {
-        case 8: return run_tile_f<T, 8>(s, tq, m, ops_dev, nops, cut);
-        case 9: return run_tile_f<T, 9>(s, tq, m, ops_dev, nops, cut);
-        case 10: return run_tile_f<T, 10>(s, tq, m, ops_dev, nops, cut);
-        case 11: return run_tile_f<T, 11>(s, tq, m, ops_dev, nops, cut);
-        case 12: return run_tile_f<T, 12>(s, tq, m, ops_dev, nops, cut);
+        case 8: return run_tile_f<T, 8>(s, tq, m, ops_dev, cut);
+        case 9: return run_tile_f<T, 9>(s, tq, m, ops_dev, cut);
+        case 10: return run_tile_f<T, 10>(s, tq, m, ops_dev, cut);
+        case 11: return run_tile_f<T, 11>(s, tq, m, ops_dev, cut);
+        case 12: return run_tile_f<T, 12>(s, tq, m, ops_dev, cut);
         case 13:
-            if constexpr (sizeof(T) == 4) return run_tile_f<T, 13>(s, tq, m, ops_dev, nops, cut);
+            if constexpr (sizeof(T) == 4) return run_tile_f<T, 13>(s, tq, m, ops_dev, cut);
             break;
     }
     return fail(QVMHIP_EINVAL, "tile size m must be 8..12 (F64) or 8..13 (F32)");
@@ -1428,38 +1538,27 @@ int run_tile_m(qvmhip_state *s, uint32_t m, const uint32_t *tq, const qvmhip_til
 
 }  // namespace
 
-bool tile_ops_have_cut(const qvmhip_tile_op *ops, size_t n) {
-    for (size_t i = 0; i < n; ++i)
-        if (ops[i].kind == kTileCutPhase) return true;
-    return false;
+int launch_tile_code(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, const void *code_dev, bool cut) {
+    const TileDevOp *dev = (const TileDevOp *)code_dev;
+    return s->dtype == QVMHIP_F64 ? run_tile_m<double>(s, m, tile_qubits, dev, cut)
+                                  : run_tile_m<float>(s, m, tile_qubits, dev, cut);
 }
 
 int launch_tile_pass(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, uint32_t nops,
-                     const qvmhip_tile_op *ops, int ops_on_device, bool cut) {
-    const qvmhip_tile_op *dev = ops;
-    qvmhip_tile_op *tmp = nullptr;
-    if (!ops_on_device) {
-        std::vector<qvmhip_tile_op> sched;
-        schedule_tile_ops(s->dtype, (s->flags & QVMHIP_FLAG_FMA_TILES) != 0, m, ops, nops, sched);
-        nops = (uint32_t)sched.size();
-        cut = tile_ops_have_cut(sched.data(), sched.size());
-        // Operands go through the matrix slot (64 KiB = 240 ops); longer lists
-        // get a temporary buffer released after the stream drains.  The slot
-        // is reused by the next call, so wait for any earlier reader first.
-        const size_t bytes = sizeof(qvmhip_tile_op) * (size_t)nops;
-        if (bytes <= 64 * 1024) {
-            QH_CHECK(hipMemcpyAsync(s->mat, sched.data(), bytes, hipMemcpyHostToDevice, s->stream));
-            QH_CHECK(hipStreamSynchronize(s->stream));  // sched is a host temporary
-            dev = (const qvmhip_tile_op *)s->mat;
-        } else {
-            QH_CHECK(hipMalloc((void **)&tmp, bytes));
-            QH_CHECK(hipMemcpyAsync(tmp, sched.data(), bytes, hipMemcpyHostToDevice, s->stream));
-            QH_CHECK(hipStreamSynchronize(s->stream));
-            dev = tmp;
-        }
+                     const qvmhip_tile_op *ops) {
+    const TileCode code = compile_tile_ops(s->dtype, (s->flags & QVMHIP_FLAG_FMA_TILES) != 0, m, ops, nops);
+    // Operands go through the matrix slot's first half (64 KiB, some 800
+    // ops); longer lists get a temporary buffer released after the stream
+    // drains.  The copy is ordered on the stream after every earlier reader.
+    void *dev = s->mat, *tmp = nullptr;
+    if (code.bytes.size() > kFusedMatOffset) {
+        QH_CHECK(hipMalloc(&tmp, code.bytes.size()));
+        dev = tmp;
     }
-    int rc = s->dtype == QVMHIP_F64 ? run_tile_m<double>(s, m, tile_qubits, dev, nops, cut)
-                                    : run_tile_m<float>(s, m, tile_qubits, dev, nops, cut);
+    hipError_t e = hipMemcpyAsync(dev, code.bytes.data(), code.bytes.size(), hipMemcpyHostToDevice, s->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);  // code is a host temporary
+    const int rc = e == hipSuccess ? launch_tile_code(s, m, tile_qubits, dev, code.cut)
+                                   : fail(QVMHIP_EDEVICE, std::string("tile ops upload: ") + hipGetErrorString(e));
     if (tmp) {
         (void)hipStreamSynchronize(s->stream);
         (void)hipFree(tmp);
@@ -1470,15 +1569,14 @@ int launch_tile_pass(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, u
 size_t tile_entry_bytes() { return sizeof(TileEntry); }
 
 uint64_t build_tile_entry(void *entry, int dtype, bool fma, uint32_t n, uint32_t m, const uint32_t *tq,
-                          uint64_t amp_offset, uint64_t block_start, uint64_t op_off, uint32_t nops,
-                          uint32_t tiles_per_block, bool from_zero, uint64_t zero_mask) {
+                          uint64_t amp_offset, uint64_t block_start, uint64_t op_off, uint32_t tiles_per_block,
+                          bool from_zero, uint64_t zero_mask) {
     TileEntry e;
     std::memset(&e, 0, sizeof(e));
     make_tile_args(n, m, tq, (int)m - tile_reg_bits((int)m, dtype == QVMHIP_F64, fma), e.args);
     e.amp_offset = amp_offset;
     e.block_start = block_start;
     e.op_off = op_off;
-    e.nops = nops;
     e.from_zero = from_zero ? 1u : 0u;
     e.zero_mask = zero_mask;
     std::memcpy(entry, &e, sizeof(e));
