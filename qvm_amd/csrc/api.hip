@@ -57,13 +57,6 @@ bool finite_matrix(const double *U, uint32_t k) {
     return true;
 }
 
-int scalar_to_host(qvmhip_state *s, double *dev, double *out) {
-    QH_CHECK(hipMemcpyAsync(s->host, dev, sizeof(double), hipMemcpyDeviceToHost, s->stream));
-    QH_CHECK(hipStreamSynchronize(s->stream));
-    *out = s->host[0];
-    return QVMHIP_OK;
-}
-
 void free_state(qvmhip_state *s) {
     if (!s) return;
     for (auto &r : s->prof) {
@@ -158,7 +151,7 @@ int qvmhip_create(uint32_t n, int dtype, const qvmhip_config *cfg, qvmhip_state 
         return bail(e, "hipMalloc(prefix)");
     if ((e = hipMalloc((void **)&s->scan_tmp, sizeof(double) * nseg)) != hipSuccess)
         return bail(e, "hipMalloc(scan)");
-    if ((e = hipHostMalloc((void **)&s->host, sizeof(double) * 64, hipHostMallocDefault)) != hipSuccess)
+    if ((e = hipHostMalloc((void **)&s->host, sizeof(double) * kHostSums, hipHostMallocDefault)) != hipSuccess)
         return bail(e, "hipHostMalloc");
     s->stage_bytes = kStageBytes;
     if ((e = hipHostMalloc(&s->stage, s->stage_bytes, hipHostMallocDefault)) != hipSuccess)
@@ -316,27 +309,21 @@ int qvmhip_prob_excited(qvmhip_state *s, uint32_t q, double *p1) {
     if (!s || !p1) return fail(QVMHIP_EINVAL, "null argument");
     DeviceScope ds(s->device);
     if (q >= s->n) return fail(QVMHIP_EINVAL, "qubit out of range");
-    int rc = reduce_probability(s, 1, q, s->red + kRedBlocks * 2);
-    if (rc) return rc;
-    return scalar_to_host(s, s->red + kRedBlocks * 2, p1);
+    return reduce_probability(s, 1, q, p1);
 }
 
 int qvmhip_prob_ground(qvmhip_state *s, uint32_t q, double *p0) {
     if (!s || !p0) return fail(QVMHIP_EINVAL, "null argument");
     DeviceScope ds(s->device);
     if (q >= s->n) return fail(QVMHIP_EINVAL, "qubit out of range");
-    int rc = reduce_probability(s, 2, q, s->red + kRedBlocks * 2);
-    if (rc) return rc;
-    return scalar_to_host(s, s->red + kRedBlocks * 2, p0);
+    return reduce_probability(s, 2, q, p0);
 }
 
 int qvmhip_norm(qvmhip_state *s, double *out) {
     if (!s || !out) return fail(QVMHIP_EINVAL, "null argument");
     DeviceScope ds(s->device);
     double n2 = 0;
-    int rc = reduce_norm2(s, s->red + kRedBlocks * 2);
-    if (rc) return rc;
-    rc = scalar_to_host(s, s->red + kRedBlocks * 2, &n2);
+    int rc = reduce_norm2(s, &n2);
     if (rc) return rc;
     *out = std::sqrt(n2);
     return QVMHIP_OK;
@@ -345,9 +332,7 @@ int qvmhip_norm(qvmhip_state *s, double *out) {
 int qvmhip_total_probability(qvmhip_state *s, double *out) {
     if (!s || !out) return fail(QVMHIP_EINVAL, "null argument");
     DeviceScope ds(s->device);
-    int rc = reduce_norm2(s, s->red + kRedBlocks * 2);
-    if (rc) return rc;
-    return scalar_to_host(s, s->red + kRedBlocks * 2, out);
+    return reduce_norm2(s, out);
 }
 
 int qvmhip_normalize(qvmhip_state *s, double length) {

@@ -168,7 +168,7 @@ static int kraus_norms(qvmhip_state *s, const cd *ops, uint32_t count, const uin
     }
     const uint32_t grid = (uint32_t)std::min<uint64_t>((a.g.ngroups + kBlock - 1) / kBlock, kNormBlocks);
     hipLaunchKernelGGL((k_kraus_norms<T, K>), dim3(grid), dim3(kBlock), 0, s->stream, (const vec2_t<T> *)s->amps, a,
-                       s->red);
+                       partials_of(s, (int)grid, C));
     QH_LAUNCH_CHECK();
     return sums_to_host(s, (int)grid, C, out, (int)count);
 }

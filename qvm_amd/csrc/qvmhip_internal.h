@@ -20,6 +20,7 @@ constexpr int kBlock = 256;         // threads per workgroup for streaming kerne
 constexpr int kMaxK = 6;            // widest dense block (64 x 64)
 constexpr int kMaxSorted = 16;      // targets + controls of one gate
 constexpr int kRedBlocks = 2048;    // partial sums of one reduction launch
+constexpr int kHostSums = 64;       // doubles of a state's pinned host page
 constexpr int kChunkLog2 = 8;       // sampling chunk: 256 amplitudes
 // A dispatch holds at most 2^32 work-items; sweep kernels cap their grid at
 // 2^22 workgroups and grid-stride over the rest (34-qubit states).
@@ -249,16 +250,18 @@ int launch_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, 
 // reaches r (the last one when none does); 1 <= k <= 2
 int launch_kraus_choice(qvmhip_state *s, const double *K, uint32_t count, uint32_t k, const uint32_t *qubits, double r,
                         uint32_t *index);
-// adds the `n` partials in s->red (`width` interleaved sums) and waits: the
-// first `count` sums go to out
+// a reduction's partials (`n`, `width` interleaved sums) go to partials_of;
+// sums_to_host adds them up and waits: the first `count` sums go to out
+double *partials_of(qvmhip_state *s, int n, int width);
 int sums_to_host(qvmhip_state *s, int n, int width, double *out, int count);
 int launch_diagonal(qvmhip_state *s, const double *d, uint32_t k, const uint32_t *qubits);
 int launch_permutation(qvmhip_state *s, const uint32_t *perm, uint32_t k, const uint32_t *qubits);
 int launch_fill_zero_state(qvmhip_state *s);
 void program_detach(qvmhip_program *p);  // the state is being destroyed
 int launch_scale(qvmhip_state *s, double factor);
-int reduce_probability(qvmhip_state *s, int mode, uint32_t q, double *out_dev);
-int reduce_norm2(qvmhip_state *s, double *out_dev);
+// mode 0: all amplitudes, 1 / 2: the bit q = 1 / 0 half; *out on the host
+int reduce_probability(qvmhip_state *s, int mode, uint32_t q, double *out);
+int reduce_norm2(qvmhip_state *s, double *out);
 int launch_force_measure(qvmhip_state *s, uint32_t q, int bit, double inv_norm, int compiled_form);
 int sample_shots(qvmhip_state *s, const double *u, uint64_t nshots, uint64_t *out, int rule_ge, double eps = 0.0,
                  uint8_t *near_flags = nullptr, uint64_t *n_near = nullptr);
@@ -294,8 +297,6 @@ enum { kExportAmps = 0, kExportAmpsBE = 1, kExportProbs = 2, kExportProbsBE = 3 
 int export_range(qvmhip_state *s, uint64_t start, uint64_t count, int mode, void *host_out);
 int convert_f32_to_f64(qvmhip_state *s, uint64_t start, uint64_t count, double *dev_out);
 int convert_f64_to_f32(qvmhip_state *s, uint64_t start, uint64_t count, const double *dev_in);
-// Capturable (kernel launches only) forms used by batches and programs.
-int expectation_zz_to_device(qvmhip_state *s, const uint32_t *edges_dev, uint32_t nedges, double *out_dev);
 // Device tables of a batch's finishing pass (all instances in one set of
 // launches): per instance its amplitude offset and length, the prefix over
 // instances of sampling chunks (count + 1 entries) and of work blocks

@@ -66,53 +66,154 @@ __global__ void k_fill_u64(uint64_t *__restrict__ out, uint64_t count, uint64_t 
         out[i] = v;
 }
 
-// mode 0: all amplitudes; 1: bit q = 1 half; 2: bit q = 0 half.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_prob_partial(const vec2_t<T> *__restrict__ psi,
-                                                         uint64_t count, int mode, uint32_t q,
-                                                         double *__restrict__ partial) {
+// 16 bytes of the state: one FP64 amplitude or two FP32 ones.
+template <typename T> struct Elem;
+template <> struct Elem<double> {
+    typedef double type __attribute__((ext_vector_type(2)));
+    static __device__ inline double p(const type &v, int) { return v.x * v.x + v.y * v.y; }
+};
+template <> struct Elem<float> {
+    typedef float type __attribute__((ext_vector_type(4)));
+    // probability of amplitude h of the pair
+    static __device__ inline double p(const type &v, int h) {
+        const double re = h ? v.z : v.x, im = h ? v.w : v.y;
+        return re * re + im * im;
+    }
+};
+
+template <typename T, bool NTM>
+__device__ inline typename Elem<T>::type load_elem(const vec2_t<T> *psi, uint64_t e) {
+    const typename Elem<T>::type *p = reinterpret_cast<const typename Elem<T>::type *>(psi) + e;
+    if constexpr (NTM)
+        return __builtin_nontemporal_load(p);
+    else
+        return *p;
+}
+
+// Read-only sweeps.  A workgroup takes one contiguous segment of the elements
+// (its XCD's share is contiguous too) and keeps kReadAhead 16-byte loads per
+// thread in flight, non-temporal when the state is larger than the Infinity
+// Cache.  16 GiB reads (probe): 7.05 TB/s, against 5.87 for a grid-stride
+// loop over 2048 workgroups with four loads in flight, 6.2 without the hint.
+constexpr int kReadAhead = 8;
+constexpr uint64_t kReadStep = uint64_t(kBlock) * kReadAhead;  // elements per workgroup and step
+
+// Sum of probabilities.  mode 0: all elements; 1: the bit q = 1 half; 2: the
+// bit q = 0 half.  q is a bit of the element index; `part` (FP32, qubit 0)
+// takes only the first (0) or second (1) amplitude of every element, -1 both.
+template <typename T, bool NTM>
+__global__ __launch_bounds__(kBlock) void k_prob_partial(const vec2_t<T> *__restrict__ psi, uint64_t elems, int mode,
+                                                         uint32_t q, int part, double *__restrict__ partial) {
     __shared__ double sm[kBlock / kWave];
-    const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-    const uint64_t qbit = uint64_t(1) << q;
+    using E = typename Elem<T>::type;
+    const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
+    const uint64_t seg = elems / gridDim.x, first = seg * b + threadIdx.x;
+    const uint64_t set = mode == 1 ? uint64_t(1) << q : 0;
     double acc = 0.0;
-    uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-    for (; i + 3 * stride < count; i += 4 * stride) {
-        vec2_t<T> v[4];
+    for (uint64_t i = 0; i < seg; i += kReadStep) {
+        E v[kReadAhead];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            uint64_t a = i + u * stride;
-            if (mode == 1) a = insert_zero(a, q) | qbit;
-            if (mode == 2) a = insert_zero(a, q);
-            v[u] = psi[a];
+        for (int u = 0; u < kReadAhead; ++u) {
+            uint64_t e = first + i + (uint64_t)u * kBlock;
+            if (e >= elems) e = 0;  // fewer than kReadStep elements in all
+            if (mode) e = insert_zero(e, q) | set;
+            v[u] = load_elem<T, NTM>(psi, e);
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) acc += prob<T>(v[u]);
-    }
-    for (; i < count; i += stride) {
-        uint64_t a = i;
-        if (mode == 1) a = insert_zero(a, q) | qbit;
-        if (mode == 2) a = insert_zero(a, q);
-        acc += prob<T>(psi[a]);
+        for (int u = 0; u < kReadAhead; ++u) {
+            double p = 0.0;
+            if (part != 1) p += Elem<T>::p(v[u], 0);
+            if (sizeof(T) == 4 && part != 0) p += Elem<T>::p(v[u], 1);
+            if (first + i + (uint64_t)u * kBlock < elems) acc += p;
+        }
     }
     const double t = block_sum(acc, sm);
     if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
-// sum over edges of <Z_a Z_b>: weight(i) = nedges - 2 * #cut edges.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_zz_partial(const vec2_t<T> *__restrict__ psi,
-                                                       uint64_t count, const uint32_t *edges,
-                                                       uint32_t nedges, double *__restrict__ partial) {
+// sum over edges of <Z_a Z_b>: weight(i) = nedges - 2 * #cut edges.  The
+// amplitudes are taken 2^11 at a time; the edges come ordered by where their
+// ends lie: both below bit 11 (ll; a constant of the thread's amplitude), one
+// below (cr), both above (hh; a constant of the chunk).  The cross edges of
+// an amplitude are popcount(A(low bits) ^ B(chunk)), one bit per edge, so an
+// amplitude costs a handful of instructions instead of five per edge (30
+// qubits, ring of 30 edges, FP32: 4.4 ms of instruction issue for a 1.2 ms read).
+constexpr int kZZBits = 11;
+struct ZZArgs {
+    uint32_t nll, ncr, nhh, fast;  // fast: at most 32 cross edges
+    uint8_t lo[256], hi[256];      // ends of edge e, lo[e] <= hi[e]
+};
+
+template <typename T, bool NTM>
+__global__ __launch_bounds__(kBlock) void k_zz_partial(const vec2_t<T> *__restrict__ psi, uint64_t len,
+                                                       const ZZArgs a, double *__restrict__ partial) {
     __shared__ double sm[kBlock / kWave];
-    __shared__ uint32_t se[2 * 256];
-    for (uint32_t e = threadIdx.x; e < 2 * nedges && e < 512; e += kBlock) se[e] = edges[e];
-    __syncthreads();
-    const uint64_t stride = (uint64_t)gridDim.x * kBlock;
+    using E = typename Elem<T>::type;
+    constexpr int H = sizeof(T) == 8 ? 1 : 2;             // amplitudes per element
+    constexpr int U = (1 << kZZBits) / kBlock / H;        // elements per thread and chunk
+    const uint64_t nchunk = (len + (1u << kZZBits) - 1) >> kZZBits;
+    const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
+    const uint64_t per = nchunk / gridDim.x;
+    const uint32_t ne = a.nll + a.ncr + a.nhh;
+    // low bits of the thread's amplitude k (bit 0 is the place in an FP32 pair)
+    auto low = [&](int k) { return (uint32_t)H * (threadIdx.x + (uint32_t)(k / H) * kBlock) + (uint32_t)(k % H); };
+    int win[U * H];
+    uint32_t A[U * H];
+#pragma unroll
+    for (int k = 0; k < U * H; ++k) {
+        win[k] = 0;
+        A[k] = 0;
+    }
+    // lane l looks after edge l of the upper classes (and l + 64, ...): their
+    // bits of a chunk are one ballot
+    const uint32_t lane = threadIdx.x % kWave;
+    uint32_t cr_hi = 63, hh_lo[4], hh_hi[4];
+    if (a.fast) {
+        for (uint32_t e = 0; e < a.nll; ++e) {
+            const uint32_t x = a.lo[e], y = a.hi[e];
+#pragma unroll
+            for (int k = 0; k < U * H; ++k) win[k] += (int)(((low(k) >> x) ^ (low(k) >> y)) & 1u);
+        }
+        for (uint32_t e = 0; e < a.ncr; ++e) {
+            const uint32_t x = a.lo[a.nll + e];
+#pragma unroll
+            for (int k = 0; k < U * H; ++k) A[k] |= ((low(k) >> x) & 1u) << e;
+        }
+        if (lane < a.ncr) cr_hi = a.hi[a.nll + lane] - kZZBits;
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+            const uint32_t e = lane + r * kWave;
+            const bool on = e < a.nhh;
+            hh_lo[r] = on ? a.lo[a.nll + a.ncr + e] - kZZBits : 63u;
+            hh_hi[r] = on ? a.hi[a.nll + a.ncr + e] - kZZBits : 63u;
+        }
+    }
     double acc = 0.0;
-    for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < count; i += stride) {
-        int cut = 0;
-        for (uint32_t e = 0; e < nedges; ++e) cut += (int)(((i >> se[2 * e]) ^ (i >> se[2 * e + 1])) & 1u);
-        acc += prob<T>(psi[i]) * (double)((int)nedges - 2 * cut);
+    for (uint64_t c = per * b; c < per * (b + 1); ++c) {
+        E v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint64_t e = ((c << kZZBits) / H) + threadIdx.x + (uint64_t)u * kBlock;
+            v[u] = load_elem<T, NTM>(psi, e < len / H ? e : 0);
+        }
+        uint32_t B = 0;
+        int hh = 0;
+        if (a.fast) {
+            B = (uint32_t)__ballot((c >> cr_hi) & 1u);
+#pragma unroll
+            for (uint32_t r = 0; r < 4; ++r)
+                if (r * kWave < a.nhh) hh += __popcll(__ballot(((c >> hh_lo[r]) ^ (c >> hh_hi[r])) & 1u));
+        }
+#pragma unroll
+        for (int k = 0; k < U * H; ++k) {
+            const uint64_t x = (c << kZZBits) + (uint64_t)H * (threadIdx.x + (uint64_t)(k / H) * kBlock) + (k % H);
+            int cut = win[k] + hh + __popc(A[k] ^ B);
+            if (!a.fast) {
+                cut = 0;
+                for (uint32_t e = 0; e < ne; ++e) cut += (int)(((x >> a.lo[e]) ^ (x >> a.hi[e])) & 1u);
+            }
+            if (x < len) acc += Elem<T>::p(v[k / H], k % H) * (double)((int)ne - 2 * cut);
+        }
     }
     const double t = block_sum(acc, sm);
     if (threadIdx.x == 0) partial[blockIdx.x] = t;
@@ -203,29 +304,40 @@ __global__ __launch_bounds__(kBlock) void k_final_sum(const double *__restrict__
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_force_measure(vec2_t<T> *__restrict__ psi, uint64_t len,
-                                                          uint32_t q, int bit, double inv_norm,
-                                                          int compiled_form) {
-    const uint64_t stride = (uint64_t)gridDim.x * kBlock;
+// Collapse on qubit q.  Each thread takes one 16-byte element (an XCD's
+// share contiguous, non-temporal when the state is larger than the Infinity
+// Cache); the annihilated half of the interpreted form is written without
+// being read.
+template <typename T, bool NTM>
+__global__ __launch_bounds__(kBlock) void k_force_measure(vec2_t<T> *__restrict__ psi, uint64_t elems, uint32_t q,
+                                                          int bit, double inv_norm, int compiled_form) {
+    using E = typename Elem<T>::type;
+    constexpr int H = sizeof(T) == 8 ? 1 : 2, W = sizeof(T) == 8 ? 2 : 4;  // amplitudes, reals per element
+    E *p = reinterpret_cast<E *>(psi);
+    const uint64_t step = (uint64_t)gridDim.x * kBlock;
     const T f = (T)inv_norm;
-    for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < len; i += stride) {
-        vec2_t<T> v = psi[i];
-        const int ab = (int)((i >> q) & 1u);
-        if (compiled_form) {
-            // src/compile-gate.lisp:248-254: amp *= inv_norm * [bit matches]
-            const T g = f * (T)(ab == bit ? 1 : 0);
-            v.x = g * v.x;
-            v.y = g * v.y;
-        } else if (ab != bit) {
-            // src/measurement.lisp:29-39: annihilated half -> 0, kept half *= inv_norm
-            v.x = T(0);
-            v.y = T(0);
+    for (uint64_t i = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x; i < elems; i += step) {
+        bool keep[H];
+#pragma unroll
+        for (int h = 0; h < H; ++h) keep[h] = (int)(((i * H + h) >> q) & 1u) == bit;
+        E v;
+        if (compiled_form || keep[0] || keep[H - 1]) {
+            v = load_elem<T, NTM>(psi, i);
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+                if (compiled_form)  // src/compile-gate.lisp:248-254: amp *= inv_norm * [bit matches]
+                    v[k] = (f * (T)(keep[k / 2] ? 1 : 0)) * v[k];
+                else  // src/measurement.lisp:29-39: annihilated half -> 0, kept half *= inv_norm
+                    v[k] = keep[k / 2] ? f * v[k] : T(0);
+            }
         } else {
-            v.x = f * v.x;
-            v.y = f * v.y;
+#pragma unroll
+            for (int k = 0; k < W; ++k) v[k] = T(0);
         }
-        psi[i] = v;
+        if constexpr (NTM)
+            __builtin_nontemporal_store(v, p + i);
+        else
+            p[i] = v;
     }
 }
 
@@ -255,19 +367,44 @@ __device__ inline void chunk_lane_load(const vec2_t<T> *__restrict__ psi, uint64
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_chunk_sums(const vec2_t<T> *__restrict__ psi,
-                                                       uint64_t len, uint64_t nchunks,
-                                                       double *__restrict__ sums) {
-    const int lane = threadIdx.x % kWave;
-    const uint64_t step = (uint64_t)gridDim.x * (kBlock / kWave);
-    for (uint64_t chunk = (uint64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave; chunk < nchunks;
-         chunk += step) {
-        double p[4];
-        chunk_lane_probs<T>(psi, len, chunk, lane, p);
-        const double local = ((p[0] + p[1]) + p[2]) + p[3];
-        const double incl = wave_inclusive_scan(local, lane);
-        if (lane == kWave - 1) sums[chunk] = incl;
+// The sums of k_chunk_sums as chunk_lane_probs forms them, from loads that
+// cover a contiguous KB each: the probabilities change lanes through LDS.
+// Loaded where they are used, the four amplitudes of a lane make every load
+// touch every other line of a 4 KB chunk (16 GiB: 3.50 ms, 4.9 TB/s).  A wave
+// takes `per` consecutive chunks and loads the next one before it scans this.
+template <typename T, bool NTM>
+__global__ __launch_bounds__(kBlock) void k_chunk_sums(const vec2_t<T> *__restrict__ psi, uint64_t len,
+                                                       uint64_t nchunks, uint64_t per, double *__restrict__ sums) {
+    constexpr int kChunk = 1 << kChunkLog2;
+    __shared__ __align__(16) double sm[kBlock / kWave][kChunk];
+    const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
+    const uint64_t wave = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * (kBlock / kWave) + wid;
+    const uint64_t c0 = wave * per, c1 = c0 + per < nchunks ? c0 + per : nchunks;
+    if (c0 >= nchunks) return;  // no workgroup barrier follows
+    auto load = [&](uint64_t c, vec2_t<T> (&v)[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint64_t i = (c << kChunkLog2) + (uint64_t)(u * kWave + lane);
+            v[u] = ldg<NTM>(&psi[i < len ? i : 0]);
+            if (i >= len) v[u].x = v[u].y = T(0);
+        }
+    };
+    vec2_t<T> cur[4], nxt[4];
+    load(c0, cur);
+    for (uint64_t c = c0; c < c1; ++c) {
+        if (c + 1 < c1) load(c + 1, nxt);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) sm[wid][u * kWave + lane] = prob<T>(cur[u]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wave's own LDS row
+        __builtin_amdgcn_wave_barrier();
+        const double2 a = *reinterpret_cast<const double2 *>(&sm[wid][4 * lane]);
+        const double2 b = *reinterpret_cast<const double2 *>(&sm[wid][4 * lane + 2]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const double incl = wave_inclusive_scan(((a.x + a.y) + b.x) + b.y, lane);
+        if (lane == kWave - 1) sums[c] = incl;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) cur[u] = nxt[u];
     }
 }
 
@@ -600,8 +737,8 @@ template <typename T>
 __global__ __launch_bounds__(kBlock) void k_collapse_basis(vec2_t<T> *__restrict__ psi, uint64_t len,
                                                            const uint64_t *__restrict__ index) {
     const uint64_t b = *index;
-    const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-    for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < len; i += stride) {
+    const uint64_t step = (uint64_t)gridDim.x * kBlock;
+    for (uint64_t i = (uint64_t)xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x; i < len; i += step) {
         vec2_t<T> z;
         z.x = (i == b) ? T(1) : T(0);
         z.y = T(0);
@@ -691,41 +828,77 @@ uint32_t sweep_grid(uint64_t count) {
 }
 }  // namespace
 
-int reduce_probability(qvmhip_state *s, int mode, uint32_t q, double *out_dev) {
-    const uint64_t count = mode == 0 ? s->len : s->len / 2;
-    const uint32_t grid = red_grid(count);
-    if (s->dtype == QVMHIP_F64)
-        hipLaunchKernelGGL(k_prob_partial<double>, dim3(grid), dim3(kBlock), 0, s->stream,
-                           (const double2 *)s->amps, count, mode, q, s->red);
-    else
-        hipLaunchKernelGGL(k_prob_partial<float>, dim3(grid), dim3(kBlock), 0, s->stream,
-                           (const float2 *)s->amps, count, mode, q, s->red);
-    QH_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(kBlock), 0, s->stream, s->red, (int)grid, 1, out_dev);
-    QH_LAUNCH_CHECK();
-    return QVMHIP_OK;
+// Where the partials of a reduction go: few of them straight to the pinned
+// host page, which sums_to_host then adds up itself.
+double *partials_of(qvmhip_state *s, int n, int width) {
+    return n * width <= kHostSums ? s->host : s->red;
 }
 
+// Adds the partials of a reduction launched on s (`n` of them, `width`
+// interleaved sums) in a fixed order and waits.  More than a page of them are
+// added by one block that writes the pinned host page: no device-to-host copy.
 int sums_to_host(qvmhip_state *s, int n, int width, double *out, int count) {
-    double *dev = s->red + kRedBlocks * 2;
-    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(kBlock), 0, s->stream, s->red, n, width, dev);
+    if (n * width <= kHostSums) {
+        QH_CHECK(hipStreamSynchronize(s->stream));
+        for (int w = 0; w < count; ++w) {
+            double acc = 0.0;
+            for (int i = 0; i < n; ++i) acc += s->host[(size_t)i * width + w];
+            out[w] = acc;
+        }
+        return QVMHIP_OK;
+    }
+    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(kBlock), 0, s->stream, s->red, n, width, s->host);
     QH_LAUNCH_CHECK();
-    QH_CHECK(hipMemcpyAsync(s->host, dev, sizeof(double) * width, hipMemcpyDeviceToHost, s->stream));
     QH_CHECK(hipStreamSynchronize(s->stream));
     std::copy(s->host, s->host + count, out);
     return QVMHIP_OK;
 }
 
-int reduce_norm2(qvmhip_state *s, double *out_dev) { return reduce_probability(s, 0, 0, out_dev); }
+int reduce_probability(qvmhip_state *s, int mode, uint32_t q, double *out) {
+    const bool f64 = s->dtype == QVMHIP_F64;
+    uint64_t elems = f64 ? s->len : s->len / 2;
+    int part = -1;
+    if (!f64 && mode) {  // an FP32 element holds both values of qubit 0
+        if (q == 0) {
+            part = mode == 1 ? 1 : 0;
+            mode = 0;
+        } else {
+            q -= 1;
+        }
+    }
+    if (mode) elems /= 2;
+    // powers of two: equal segments of at least kReadStep elements
+    const uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(elems / kReadStep, kRedBlocks));
+    double *partial = partials_of(s, (int)grid, 1);
+    const bool nt = stream_accesses(s);
+    auto go = [&](auto kernel, auto *psi) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), 0, s->stream, psi, elems, mode, q, part, partial);
+    };
+    if (f64)
+        nt ? go(k_prob_partial<double, true>, (const double2 *)s->amps)
+           : go(k_prob_partial<double, false>, (const double2 *)s->amps);
+    else
+        nt ? go(k_prob_partial<float, true>, (const float2 *)s->amps)
+           : go(k_prob_partial<float, false>, (const float2 *)s->amps);
+    QH_LAUNCH_CHECK();
+    return sums_to_host(s, (int)grid, 1, out, 1);
+}
+
+int reduce_norm2(qvmhip_state *s, double *out) { return reduce_probability(s, 0, 0, out); }
 
 int launch_force_measure(qvmhip_state *s, uint32_t q, int bit, double inv_norm, int compiled_form) {
-    const uint32_t grid = sweep_grid(s->len);
-    if (s->dtype == QVMHIP_F64)
-        hipLaunchKernelGGL(k_force_measure<double>, dim3(grid), dim3(kBlock), 0, s->stream,
-                           (double2 *)s->amps, s->len, q, bit, inv_norm, compiled_form);
+    const bool f64 = s->dtype == QVMHIP_F64;
+    const uint64_t elems = f64 ? s->len : s->len / 2;
+    const uint32_t grid = (uint32_t)std::min<uint64_t>((elems + kBlock - 1) / kBlock, kMaxGrid);
+    const bool nt = stream_accesses(s);
+    auto go = [&](auto kernel, auto *psi) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), 0, s->stream, psi, elems, q, bit, inv_norm,
+                           compiled_form);
+    };
+    if (f64)
+        nt ? go(k_force_measure<double, true>, (double2 *)s->amps) : go(k_force_measure<double, false>, (double2 *)s->amps);
     else
-        hipLaunchKernelGGL(k_force_measure<float>, dim3(grid), dim3(kBlock), 0, s->stream,
-                           (float2 *)s->amps, s->len, q, bit, inv_norm, compiled_form);
+        nt ? go(k_force_measure<float, true>, (float2 *)s->amps) : go(k_force_measure<float, false>, (float2 *)s->amps);
     QH_LAUNCH_CHECK();
     return QVMHIP_OK;
 }
@@ -736,13 +909,26 @@ int launch_force_measure(qvmhip_state *s, uint32_t q, int bit, double inv_norm, 
 int launch_chunk_prefix(hipStream_t st, int dtype, const void *amps, uint64_t len, double *chunk_sum,
                         double *scan_tmp, double *chunk_pre) {
     const uint64_t nch = (len + (uint64_t(1) << kChunkLog2) - 1) >> kChunkLog2;
-    const uint32_t g1 = (uint32_t)std::min<uint64_t>((nch + (kBlock / kWave) - 1) / (kBlock / kWave), kMaxGrid);
-    if (dtype == QVMHIP_F64)
-        hipLaunchKernelGGL(k_chunk_sums<double>, dim3(g1), dim3(kBlock), 0, st, (const double2 *)amps, len, nch,
-                           chunk_sum);
-    else
-        hipLaunchKernelGGL(k_chunk_sums<float>, dim3(g1), dim3(kBlock), 0, st, (const float2 *)amps, len, nch,
-                           chunk_sum);
+    // up to 8192 workgroups of four waves, each wave with an equal run of chunks
+    const uint64_t per = std::max<uint64_t>(1, nch / (8192 * (kBlock / kWave)));
+    const uint64_t waves = (nch + per - 1) / per;
+    const dim3 g1((uint32_t)((waves + kBlock / kWave - 1) / (kBlock / kWave)));
+    const bool nt = len * (dtype == QVMHIP_F64 ? 16 : 8) > kStreamBytes;
+    if (dtype == QVMHIP_F64) {
+        if (nt)
+            hipLaunchKernelGGL((k_chunk_sums<double, true>), g1, dim3(kBlock), 0, st, (const double2 *)amps, len, nch,
+                               per, chunk_sum);
+        else
+            hipLaunchKernelGGL((k_chunk_sums<double, false>), g1, dim3(kBlock), 0, st, (const double2 *)amps, len,
+                               nch, per, chunk_sum);
+    } else {
+        if (nt)
+            hipLaunchKernelGGL((k_chunk_sums<float, true>), g1, dim3(kBlock), 0, st, (const float2 *)amps, len, nch,
+                               per, chunk_sum);
+        else
+            hipLaunchKernelGGL((k_chunk_sums<float, false>), g1, dim3(kBlock), 0, st, (const float2 *)amps, len, nch,
+                               per, chunk_sum);
+    }
     QH_LAUNCH_CHECK();
     const uint64_t nseg = (nch + kScanSeg - 1) / kScanSeg;
     hipLaunchKernelGGL(k_scan_seg_totals, dim3((uint32_t)nseg), dim3(kBlock), 0, st, chunk_sum, nch, scan_tmp);
@@ -855,23 +1041,9 @@ int sample_to_device(qvmhip_state *s, const double *u_dev, uint64_t nshots, uint
                                 0.0, nullptr, nullptr);
 }
 
-int expectation_zz_to_device(qvmhip_state *s, const uint32_t *edges_dev, uint32_t nedges, double *out_dev) {
-    if (nedges > 256) return fail(QVMHIP_EINVAL, "at most 256 edges");
-    const uint32_t grid = red_grid(s->len);
-    if (s->dtype == QVMHIP_F64)
-        hipLaunchKernelGGL(k_zz_partial<double>, dim3(grid), dim3(kBlock), 0, s->stream, (const double2 *)s->amps,
-                           s->len, edges_dev, nedges, s->red);
-    else
-        hipLaunchKernelGGL(k_zz_partial<float>, dim3(grid), dim3(kBlock), 0, s->stream, (const float2 *)s->amps,
-                           s->len, edges_dev, nedges, s->red);
-    QH_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(kBlock), 0, s->stream, s->red, (int)grid, 1, out_dev);
-    QH_LAUNCH_CHECK();
-    return QVMHIP_OK;
-}
-
 int collapse_to_basis(qvmhip_state *s, const uint64_t *index_dev) {
-    const uint32_t grid = sweep_grid(s->len);
+    // one amplitude per thread, as k_fill_zero_state
+    const uint32_t grid = (uint32_t)std::min<uint64_t>((s->len + kBlock - 1) / kBlock, kMaxGrid);
     if (s->dtype == QVMHIP_F64)
         hipLaunchKernelGGL(k_collapse_basis<double>, dim3(grid), dim3(kBlock), 0, s->stream,
                            (double2 *)s->amps, s->len, index_dev);
@@ -884,18 +1056,36 @@ int collapse_to_basis(qvmhip_state *s, const uint64_t *index_dev) {
 
 int expectation_zz(qvmhip_state *s, const uint32_t *edges, uint32_t nedges, double *out) {
     if (nedges > 256) return fail(QVMHIP_EINVAL, "at most 256 edges");
-    // the edges go to the state's matrix slot (2 KiB of its 128 KiB), in
-    // stream order after every earlier use of the slot: no allocation
-    uint32_t *dedges = (uint32_t *)s->mat;
-    if (nedges)
-        QH_CHECK(hipMemcpyAsync(dedges, edges, sizeof(uint32_t) * 2 * nedges, hipMemcpyHostToDevice, s->stream));
-    int rc = expectation_zz_to_device(s, dedges, nedges, s->red + kRedBlocks * 2);
-    if (rc) return rc;
-    QH_CHECK(hipMemcpyAsync(s->host, s->red + kRedBlocks * 2, sizeof(double), hipMemcpyDeviceToHost,
-                            s->stream));
-    QH_CHECK(hipStreamSynchronize(s->stream));
-    *out = s->host[0];
-    return QVMHIP_OK;
+    // the edges travel with the launch, ordered ll, cr, hh (see k_zz_partial)
+    ZZArgs a;
+    std::memset(&a, 0, sizeof(a));
+    uint32_t at = 0;
+    for (int cls = 0; cls < 3; ++cls) {
+        const uint32_t from = at;
+        for (uint32_t e = 0; e < nedges; ++e) {
+            const uint32_t lo = std::min(edges[2 * e], edges[2 * e + 1]), hi = std::max(edges[2 * e], edges[2 * e + 1]);
+            if ((hi < (uint32_t)kZZBits ? 0 : lo < (uint32_t)kZZBits ? 1 : 2) != cls) continue;
+            a.lo[at] = (uint8_t)lo;
+            a.hi[at++] = (uint8_t)hi;
+        }
+        (cls == 0 ? a.nll : cls == 1 ? a.ncr : a.nhh) = at - from;
+    }
+    a.fast = a.ncr <= 32 ? 1u : 0u;
+    const uint64_t nchunk = (s->len + (1u << kZZBits) - 1) >> kZZBits;
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(nchunk, kRedBlocks);  // powers of two
+    double *partial = partials_of(s, (int)grid, 1);
+    const bool nt = stream_accesses(s);
+    auto go = [&](auto kernel, auto *psi) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), 0, s->stream, psi, s->len, a, partial);
+    };
+    if (s->dtype == QVMHIP_F64)
+        nt ? go(k_zz_partial<double, true>, (const double2 *)s->amps)
+           : go(k_zz_partial<double, false>, (const double2 *)s->amps);
+    else
+        nt ? go(k_zz_partial<float, true>, (const float2 *)s->amps)
+           : go(k_zz_partial<float, false>, (const float2 *)s->amps);
+    QH_LAUNCH_CHECK();
+    return sums_to_host(s, (int)grid, 1, out, 1);
 }
 
 template <template <typename, typename> class Launch>
@@ -931,10 +1121,8 @@ int tv_distance(qvmhip_state *a, qvmhip_state *b, double *out) {
     const uint32_t grid = red_grid(a->len);
     dispatch2<TvLaunch>(a, b, grid);
     QH_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(kBlock), 0, a->stream, a->red, (int)grid, 1,
-                       a->red + kRedBlocks * 2);
+    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(kBlock), 0, a->stream, a->red, (int)grid, 1, a->host);
     QH_LAUNCH_CHECK();
-    QH_CHECK(hipMemcpyAsync(a->host, a->red + kRedBlocks * 2, sizeof(double), hipMemcpyDeviceToHost, a->stream));
     QH_CHECK(hipStreamSynchronize(a->stream));
     *out = 0.5 * a->host[0];
     return QVMHIP_OK;
@@ -944,9 +1132,8 @@ int max_abs_diff(qvmhip_state *a, qvmhip_state *b, double *out) {
     const uint32_t grid = red_grid(a->len);
     dispatch2<DiffLaunch>(a, b, grid);
     QH_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_final_max, dim3(1), dim3(64), 0, a->stream, a->red, (int)grid, a->red + kRedBlocks * 2);
+    hipLaunchKernelGGL(k_final_max, dim3(1), dim3(64), 0, a->stream, a->red, (int)grid, a->host);
     QH_LAUNCH_CHECK();
-    QH_CHECK(hipMemcpyAsync(a->host, a->red + kRedBlocks * 2, sizeof(double), hipMemcpyDeviceToHost, a->stream));
     QH_CHECK(hipStreamSynchronize(a->stream));
     *out = a->host[0];
     return QVMHIP_OK;
@@ -956,11 +1143,8 @@ int inner_product(qvmhip_state *a, qvmhip_state *b, double *re, double *im) {
     const uint32_t grid = red_grid(a->len);
     dispatch2<DotLaunch>(a, b, grid);
     QH_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(kBlock), 0, a->stream, a->red, (int)grid, 2,
-                       a->red + kRedBlocks * 2);
+    hipLaunchKernelGGL(k_final_sum, dim3(1), dim3(kBlock), 0, a->stream, a->red, (int)grid, 2, a->host);
     QH_LAUNCH_CHECK();
-    QH_CHECK(hipMemcpyAsync(a->host, a->red + kRedBlocks * 2, 2 * sizeof(double), hipMemcpyDeviceToHost,
-                            a->stream));
     QH_CHECK(hipStreamSynchronize(a->stream));
     *re = a->host[0];
     *im = a->host[1];
