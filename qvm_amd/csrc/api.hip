@@ -241,9 +241,9 @@ int qvmhip_apply_fused(qvmhip_state *s, const double *U, uint32_t k, const uint3
     if (k < 3) return fail(QVMHIP_EINVAL, "fused blocks are 3..6 qubits");
     if (!U || !finite_matrix(U, k)) return fail(QVMHIP_EINVAL, "matrix is null or not finite");
     // upload to the matrix slot's second half (first half: ops / dense)
-    const size_t bytes = sizeof(double) * 2 * (size_t(1) << (2 * k));
+    const std::vector<char> A = fused_operand(s->dtype, U, k, qubits);
     void *dst = (char *)s->mat + kFusedMatOffset;
-    QH_CHECK(hipMemcpyAsync(dst, U, bytes, hipMemcpyHostToDevice, s->stream));
+    QH_CHECK(hipMemcpyAsync(dst, A.data(), A.size(), hipMemcpyHostToDevice, s->stream));
     return launch_fused_dense(s, dst, k, qubits);
 }
 

@@ -69,8 +69,9 @@ int launch_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, 
     // (CZ, CNOT, SWAP) keep the structured kernels; dense ones (16x16, 64x64)
     // go to the matrix cores.
     if (k == 1 || !gate_is_dense(m, 2 * k, q)) return launch_gate(s, m, 2 * k, q, 0);
+    const std::vector<char> A = fused_operand(s->dtype, m, 2 * k, q);
     void *dst = (char *)s->mat + kFusedMatOffset;
-    QH_CHECK(hipMemcpyAsync(dst, m, S.size() * sizeof(cd), hipMemcpyHostToDevice, s->stream));
+    QH_CHECK(hipMemcpyAsync(dst, A.data(), A.size(), hipMemcpyHostToDevice, s->stream));
     return launch_fused_dense(s, dst, 2 * k, q);
 }
 

@@ -15,8 +15,8 @@
 // Rows of U are renumbered so that bit b of a row index is the b-th lowest
 // target qubit; a k-step's four rows then differ in the two lowest targets,
 // and 16 consecutive complement groups x those rows are contiguous runs.  The
-// A fragments (U_re, U_im per 16x4 block and lane) are built once per
-// workgroup in LDS from U in nat-tuple order.  Each wave takes 16 complement
+// A fragments (U_re, U_im per 16x4 block and lane) are copied to LDS once per
+// workgroup.  Each wave takes 16 complement
 // groups at a time, striding through the contiguous share of column groups
 // that its XCD owns, with the next group's loads issued before the current
 // group's MFMAs.  The four real products per complex product are
@@ -52,49 +52,45 @@ template <> struct Mfma<float> {
 
 struct FusedOff {
     uint64_t o[64];  // offset of sorted-order row a: sum of 2^sorted[b] over the bits of a
-    uint32_t nat[6]; // position in the nat-tuple of the b-th lowest target
 };
 
-// A fragments in LDS: fr[(mt*KS + ks)*64 + lane] = U_s[mt*16 + i][ks*4 + k],
-// lane = i + 16k, U_s = U with rows and columns in sorted-target order
-// (rows past 2^K, for K = 3, are zero).  Ends with a barrier.
+// A fragments: fr[(mt*KS + ks)*64 + lane] = U_s[mt*16 + i][ks*4 + k], lane =
+// i + 16k, U_s = U with rows and columns in sorted-target order (rows past
+// 2^K, for K = 3, are zero).  The host lays them out (fused_operand), so a
+// workgroup copies them to LDS in order with independent 16-byte loads
+// (against a gather from U in nat-tuple order by every workgroup: K = 6 FP64
+// at 2^24 amplitudes 141.8 -> 134.6 us, 2^16 13.6 -> 11.6).  Ends with a
+// barrier.
 template <typename T, int K>
-__device__ __forceinline__ void build_fragments(vec2_t<T> *fr, const double *__restrict__ U, const FusedOff &off) {
+__device__ __forceinline__ void copy_fragments(vec2_t<T> *fr, const void *__restrict__ src) {
     constexpr int D = 1 << K;
     constexpr int MT = D < 16 ? 1 : D / 16;
     constexpr int KS = D / 4;
-    for (int e = threadIdx.x; e < MT * KS * 64; e += 256) {
-        const int ln = e & 63, blk = e >> 6;
-        const int mt = blk / KS, ks = blk % KS;
-        const int rs = mt * 16 + (ln & 15), cs = ks * 4 + (ln >> 4);
-        vec2_t<T> v;
-        v.x = T(0);
-        v.y = T(0);
-        if (rs < D) {
-            int rn = 0, cn = 0;
+    constexpr int N = MT * KS * 64 * (int)sizeof(vec2_t<T>) / 16;  // 16-byte pieces
+    const uint4 *in = reinterpret_cast<const uint4 *>(src);
+    uint4 *out = reinterpret_cast<uint4 *>(fr);
+    if constexpr (N >= 256) {
+        uint4 v[N / 256];
 #pragma unroll
-            for (int b = 0; b < K; ++b) {
-                rn |= ((rs >> b) & 1) << off.nat[b];
-                cn |= ((cs >> b) & 1) << off.nat[b];
-            }
-            v.x = (T)U[2 * (rn * D + cn)];
-            v.y = (T)U[2 * (rn * D + cn) + 1];
-        }
-        fr[e] = v;
+        for (int i = 0; i < N / 256; ++i) v[i] = in[i * 256 + threadIdx.x];
+#pragma unroll
+        for (int i = 0; i < N / 256; ++i) out[i * 256 + threadIdx.x] = v[i];
+    } else {
+        if ((int)threadIdx.x < N) out[threadIdx.x] = in[threadIdx.x];
     }
     __syncthreads();
 }
 
 template <typename T, int K, bool NTM>
-__global__ __launch_bounds__(256) void k_fused(vec2_t<T> *__restrict__ psi, const double *__restrict__ U,
+__global__ __launch_bounds__(256) void k_fused(vec2_t<T> *__restrict__ psi, const void *__restrict__ A,
                                                GroupSpec g, FusedOff off) {
     using V = vec2_t<T>;
     using v4 = typename Mfma<T>::v4;
     constexpr int D = 1 << K;
     constexpr int MT = D < 16 ? 1 : D / 16;  // 16-row output blocks
     constexpr int KS = D / 4;                // 4-row k-steps
-    __shared__ V fr[MT * KS * 64];
-    build_fragments<T, K>(fr, U, off);
+    __shared__ __align__(16) V fr[MT * KS * 64];
+    copy_fragments<T, K>(fr, A);
 
     const int lane = threadIdx.x & 63;
     const int j = lane & 15, kk = lane >> 4;
@@ -245,15 +241,15 @@ __device__ __forceinline__ void xpose4(X &a0, X &a1, X &a2, X &a3) {
 // for K = 4, and K = 5 in FP32 (the four column groups' accumulators of FP64
 // K = 5 and of K = 6 leave room for one wave per SIMD).
 template <typename T, int K, bool NTM>
-__global__ __launch_bounds__(256) void k_fused_rows(vec2_t<T> *__restrict__ psi, const double *__restrict__ U,
+__global__ __launch_bounds__(256) void k_fused_rows(vec2_t<T> *__restrict__ psi, const void *__restrict__ A,
                                                     GroupSpec g, FusedOff off) {
     using V = vec2_t<T>;
     using v4 = typename Mfma<T>::v4;
     constexpr int D = 1 << K;
     constexpr int MT = D < 16 ? 1 : D / 16;
     constexpr int KS = D / 4;
-    __shared__ V fr[MT * KS * 64];
-    build_fragments<T, K>(fr, U, off);
+    __shared__ __align__(16) V fr[MT * KS * 64];
+    copy_fragments<T, K>(fr, A);
 
     const int lane = threadIdx.x & 63;
     const uint64_t ncb = g.ngroups / 64;
@@ -370,15 +366,15 @@ __device__ __forceinline__ void xpose2(X &a0, X &a1) {
 // target sets above the line: 5.85-6.74 ms against 6.81-7.01 for k_fused,
 // 5.5 % less in total (+20 % on 5,11,17,23,27).
 template <typename T, int K, bool NTM>
-__global__ __launch_bounds__(256) void k_fused_rows2(vec2_t<T> *__restrict__ psi, const double *__restrict__ U,
+__global__ __launch_bounds__(256) void k_fused_rows2(vec2_t<T> *__restrict__ psi, const void *__restrict__ A,
                                                      GroupSpec g, FusedOff off) {
     using V = vec2_t<T>;
     using v4 = typename Mfma<T>::v4;
     constexpr int D = 1 << K;
     constexpr int MT = D < 16 ? 1 : D / 16;
     constexpr int KS = D / 4;
-    __shared__ V fr[MT * KS * 64];
-    build_fragments<T, K>(fr, U, off);
+    __shared__ __align__(16) V fr[MT * KS * 64];
+    copy_fragments<T, K>(fr, A);
 
     const int lane = threadIdx.x & 63;
     const int half = lane >> 5;
@@ -490,9 +486,6 @@ int run_fused(qvmhip_state *s, const void *mat_dev, const uint32_t *qubits) {
     g.ngroups = uint64_t(1) << (s->n - K);
     FusedOff off;
     std::memset(&off, 0, sizeof(off));
-    for (int b = 0; b < K; ++b)
-        for (int c = 0; c < K; ++c)
-            if (qubits[c] == pos[b]) off.nat[b] = (uint32_t)c;
     for (int a = 0; a < 64; ++a) {
         uint64_t o = 0;
         for (int b = 0; b < K; ++b)
@@ -529,10 +522,10 @@ int run_fused(qvmhip_state *s, const void *mat_dev, const uint32_t *qubits) {
             prof_begin(s, QVMHIP_K_FUSED);
             if (stream)
                 hipLaunchKernelGGL((k_fused_rows2<T, K, true>), dim3(grid2), dim3(256), 0, s->stream,
-                                   (vec2_t<T> *)s->amps, (const double *)mat_dev, g, off);
+                                   (vec2_t<T> *)s->amps, mat_dev, g, off);
             else
                 hipLaunchKernelGGL((k_fused_rows2<T, K, false>), dim3(grid2), dim3(256), 0, s->stream,
-                                   (vec2_t<T> *)s->amps, (const double *)mat_dev, g, off);
+                                   (vec2_t<T> *)s->amps, mat_dev, g, off);
             prof_end(s);
             QH_LAUNCH_CHECK();
             return QVMHIP_OK;
@@ -557,10 +550,10 @@ int run_fused(qvmhip_state *s, const void *mat_dev, const uint32_t *qubits) {
             prof_begin(s, QVMHIP_K_FUSED);
             if (nt_rows)
                 hipLaunchKernelGGL((k_fused_rows<T, K, true>), dim3(grid_rows), dim3(256), 0, s->stream,
-                                   (vec2_t<T> *)s->amps, (const double *)mat_dev, g, off);
+                                   (vec2_t<T> *)s->amps, mat_dev, g, off);
             else
                 hipLaunchKernelGGL((k_fused_rows<T, K, false>), dim3(grid_rows), dim3(256), 0, s->stream,
-                                   (vec2_t<T> *)s->amps, (const double *)mat_dev, g, off);
+                                   (vec2_t<T> *)s->amps, mat_dev, g, off);
             prof_end(s);
             QH_LAUNCH_CHECK();
             return QVMHIP_OK;
@@ -571,10 +564,10 @@ int run_fused(qvmhip_state *s, const void *mat_dev, const uint32_t *qubits) {
     prof_begin(s, QVMHIP_K_FUSED);
     if (ntm)
         hipLaunchKernelGGL((k_fused<T, K, true>), dim3(grid), dim3(256), 0, s->stream, (vec2_t<T> *)s->amps,
-                           (const double *)mat_dev, g, off);
+                           mat_dev, g, off);
     else
         hipLaunchKernelGGL((k_fused<T, K, false>), dim3(grid), dim3(256), 0, s->stream, (vec2_t<T> *)s->amps,
-                           (const double *)mat_dev, g, off);
+                           mat_dev, g, off);
     prof_end(s);
     QH_LAUNCH_CHECK();
     return QVMHIP_OK;
@@ -591,6 +584,43 @@ int run_fused_k(qvmhip_state *s, const void *mat_dev, uint32_t k, const uint32_t
     return fail(QVMHIP_EINVAL, "fused blocks are 3..6 qubits");
 }
 }  // namespace
+
+// U (row-major, index bit j <-> qubits[j]) as the kernels' A fragments.
+template <typename T>
+static void fragments(const double *U, uint32_t k, const uint32_t *qubits, vec2_t<T> *out) {
+    const int D = 1 << k, MT = D < 16 ? 1 : D / 16, KS = D / 4;
+    int nat[6] = {0};  // position in the nat-tuple of the b-th lowest target
+    for (uint32_t c = 0; c < k; ++c) {
+        int rank = 0;
+        for (uint32_t o = 0; o < k; ++o) rank += qubits[o] < qubits[c];
+        nat[rank] = (int)c;
+    }
+    int to_nat[64];
+    for (int a = 0; a < D; ++a) {
+        to_nat[a] = 0;
+        for (uint32_t b = 0; b < k; ++b) to_nat[a] |= ((a >> b) & 1) << nat[b];
+    }
+    for (int e = 0; e < MT * KS * 64; ++e) {
+        const int ln = e & 63, mt = (e >> 6) / KS, ks = (e >> 6) % KS;
+        const int row = mt * 16 + (ln & 15), col = ks * 4 + (ln >> 4);
+        out[e].x = out[e].y = T(0);
+        if (row < D) {
+            const double *u = U + 2 * ((size_t)to_nat[row] * D + to_nat[col]);
+            out[e].x = (T)u[0];
+            out[e].y = (T)u[1];
+        }
+    }
+}
+
+std::vector<char> fused_operand(int dtype, const double *U, uint32_t k, const uint32_t *qubits) {
+    const size_t D = size_t(1) << k, count = (D < 16 ? 16 : D) * D;
+    std::vector<char> out(count * (dtype == QVMHIP_F64 ? sizeof(double2) : sizeof(float2)));
+    if (dtype == QVMHIP_F64)
+        fragments<double>(U, k, qubits, (double2 *)out.data());
+    else
+        fragments<float>(U, k, qubits, (float2 *)out.data());
+    return out;
+}
 
 int launch_fused_dense(qvmhip_state *s, const void *mat_dev, uint32_t k, const uint32_t *qubits) {
     if (s->dtype == QVMHIP_F64) return run_fused_k<double>(s, mat_dev, k, qubits);

@@ -126,8 +126,9 @@ int qvmhip_program_add_fused(qvmhip_program *p, const double *U, uint32_t k, con
     it.kind = kFused;
     it.k = k;
     std::copy(qubits, qubits + k, it.qubits);
-    it.bytes = sizeof(double) * (size_t(2) << (2 * k));
-    it.host_off = push_blob(p, U, it.bytes);
+    const std::vector<char> A = fused_operand(p->s->dtype, U, k, qubits);
+    it.bytes = A.size();
+    it.host_off = push_blob(p, A.data(), it.bytes);
     p->items.push_back(std::move(it));
     return QVMHIP_OK;
 }

@@ -284,6 +284,9 @@ TileCode compile_tile_ops(int dtype, bool fma, uint32_t m, const qvmhip_tile_op 
 int launch_tile_pass(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, uint32_t nops,
                      const qvmhip_tile_op *ops);
 int launch_tile_code(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, const void *code_dev, bool cut);
+// A fused block's matrix in the layout its kernels read, and the launch with
+// that operand on the device.
+std::vector<char> fused_operand(int dtype, const double *U, uint32_t k, const uint32_t *qubits);
 int launch_fused_dense(qvmhip_state *s, const void *mat_dev, uint32_t k, const uint32_t *qubits);
 int expectation_zz(qvmhip_state *s, const uint32_t *edges, uint32_t nedges, double *out);
 int inner_product(qvmhip_state *a, qvmhip_state *b, double *re, double *im);
