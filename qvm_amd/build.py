@@ -26,8 +26,11 @@ SOURCES = {
     "api.hip": [],
     "gates.hip": ["-ffp-contract=off"],
     # every branch of the tile kernels' op loop is uniform: left unstructured,
-    # an op's arm goes straight back to the loop and the block stays in place
-    "tile.hip": ["-ffp-contract=off", "-mllvm", "-structurizecfg-skip-uniform-regions=true"],
+    # an op's arm goes straight back to the loop and the block stays in place.
+    # Common tails of two arms stay apart: merged, they would address the
+    # block by a run-time index, which puts it into scratch memory
+    "tile.hip": ["-ffp-contract=off", "-mllvm", "-structurizecfg-skip-uniform-regions=true",
+                 "-mllvm", "-sink-common-insts=false"],
     "reduce.hip": ["-ffp-contract=off"],
     "fused.hip": [],
     "channel.hip": ["-ffp-contract=off"],

@@ -208,7 +208,8 @@ enum : uint32_t {
     kF_RX = 1u << 7,     // 1q: real diagonal, imaginary off-diagonal
     kF_1q = 0xF0u,
     kF_X = 1u << 8,      // exchange register pairs where the lane condition holds
-    kF_DL = 1u << 9,     // diagonal: one of two entries per lane, on registers c
+    kF_DL = 1u << 9,     // diagonal: one of two entries per lane, on all registers, those with the
+                         // target bit set, or (Mask) those of c
     kF_DL4 = 1u << 10,   // diagonal: one of four entries per lane (bits a & 0xff, a >> 8)
     kF_DR = 1u << 11,    // diagonal: entry by lane condition and target register bit
     kF_RDiag = 1u << 12, // diagonal: entry r on register r
@@ -222,6 +223,9 @@ enum : uint32_t {
     kF_Cut = 1u << 19,
     kF_Rare = kF_Dense2 | kF_Dense2C | kF_SwapC | kF_RSwap | kF_Cut,
     kF_End = 1u << 20,
+    kF_Mask = 1u << 21,  // DL on the registers of c
+    kF_Id0 = 1u << 22,   // DL: lanes outside the condition keep their amplitudes (entry 0 is 1)
+    kF_Neg = 1u << 23,   // DL with Id0: entry 1 is -1
 };
 
 // The 80 bytes of a slot, loaded as scalars one op ahead (as 64-bit words:
@@ -436,21 +440,44 @@ __device__ __forceinline__ void reg_rswap_any(vec2_t<T> (&x)[R], uint32_t pair) 
 // Diagonals.  A diagonal's index has a lane part (the same for all registers)
 // and a register part.  No case needs a per-register vector select: the lane
 // part picks one entry (or two) per lane once per op, and the register part
-// is a scalar choice or a compile-time one.  Registers outside `regs` are
-// skipped; a lane whose condition fails multiplies by exactly 1, which leaves
-// its amplitude's value unchanged.
-template <typename T, int R, bool FMA>
-__device__ __forceinline__ void diag_lane(vec2_t<T> (&x)[R], T dr, T di, uint32_t regs) {
-    if (regs == (1u << R) - 1u) {
+// is a scalar choice or a compile-time one.  A lane whose condition fails
+// multiplies by exactly 1, which leaves its amplitude's value unchanged; a
+// wave without a lane that meets it skips the op.
+
+// apply(x[r]) on the registers an op names: all, those with target bit I set,
+// or those of its mask.  The first two are compile-time sets: tested one by
+// one, eight registers cost sixteen scalar instructions and branches.
+template <typename T, int R, int I, typename F>
+__device__ __forceinline__ void on_bit(vec2_t<T> (&x)[R], const F &apply) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) cmul<T, FMA>(x[r], dr, di);
-        return;
-    }
+    for (int u = 0; u < R / 2; ++u) apply(x[((u >> I) << (I + 1)) | (1 << I) | (u & ((1 << I) - 1))]);
+}
+
+template <typename T, int R, typename F>
+__device__ __forceinline__ void on_registers(vec2_t<T> (&x)[R], uint32_t f, uint32_t mask, const F &apply) {
+    if (f & kF_Mask) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-        if ((regs >> r) & 1u) cmul<T, FMA>(x[r], dr, di);
+        for (int r = 0; r < R; ++r)
+            if ((mask >> r) & 1u) apply(x[r]);
+    } else if (f & (kF_Bit0 << 0)) {
+        on_bit<T, R, 0>(x, apply);
+    } else if (f & (kF_Bit0 << 1)) {
+        on_bit<T, R, 1>(x, apply);
+    } else if (R > 4 && (f & (kF_Bit0 << 2))) {
+        if constexpr (R > 4) on_bit<T, R, 2>(x, apply);
+    } else if (R > 8 && (f & (kF_Bit0 << 3))) {
+        if constexpr (R > 8) on_bit<T, R, 3>(x, apply);
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r) apply(x[r]);
     }
 }
+
+// Flips the sign of v where `bit` is 0x80000000 (0 elsewhere).
+__device__ __forceinline__ double flip_sign(double v, uint32_t bit) {
+    return __hiloint2double((int)((uint32_t)__double2hiint(v) ^ bit), __double2loint(v));
+}
+__device__ __forceinline__ float flip_sign(float v, uint32_t bit) { return __uint_as_float(__float_as_uint(v) ^ bit); }
 
 // Register r takes entry c1 when its bit RS is set, c0 otherwise.
 template <typename T, int R, int RS, bool FMA>
@@ -473,7 +500,7 @@ __device__ __forceinline__ void reg_rdiag(vec2_t<T> (&x)[R], const T *__restrict
 
 // DL, DL4, DR and RDIAG (see the flags).  Out: the bits of the block's base
 // index named by b (g0 | g1 << 8 | count << 16) select one of the op's entry
-// pairs; c has bit `sel` set where that pair is (1, 1), which is skipped.
+// pairs; bit 20 + sel of b is set where that pair is (1, 1), which is skipped.
 template <typename T, int R, bool FMA>
 __device__ __forceinline__ void reg_diag(vec2_t<T> (&x)[R], const TileHead &h, const TileDevOp *__restrict__ op,
                                          uint32_t t, uint64_t gb) {
@@ -484,29 +511,36 @@ __device__ __forceinline__ void reg_diag(vec2_t<T> (&x)[R], const TileHead &h, c
         const bool b0 = ((t >> (h.a() & 0xFFu)) & 1u) != 0, b1 = ((t >> (h.a() >> 8)) & 1u) != 0;
         const T ra = b0 ? h.m<T>(2) : h.m<T>(0), ia = b0 ? h.m<T>(3) : h.m<T>(1);
         const T rb = b0 ? h.m<T>(6) : h.m<T>(4), ib = b0 ? h.m<T>(7) : h.m<T>(5);
-        diag_lane<T, R, FMA>(x, b1 ? rb : ra, b1 ? ib : ia, (1u << R) - 1u);
+        const T dr = b1 ? rb : ra, di = b1 ? ib : ia;
+#pragma unroll
+        for (int r = 0; r < R; ++r) cmul<T, FMA>(x[r], dr, di);
     } else {
-        T e[4] = {h.m<T>(0), h.m<T>(1), h.m<T>(2), h.m<T>(3)};
-        uint32_t want = h.b(), regs = h.c();
+        // the pair of entries: by default the first, with qubits outside the
+        // tile the one they select (two pairs fit the slot)
+        T e0r = h.m<T>(0), e0i = h.m<T>(1), e1r = h.m<T>(2), e1i = h.m<T>(3);
+        uint32_t want = h.b();
         bool go = true;
         if (f & kF_Out) {
             const uint32_t d = h.b();
             uint32_t sel = (uint32_t)(gb >> (d & 63u)) & 1u;
-            if ((d >> 16) == 2u) sel |= ((uint32_t)(gb >> ((d >> 8) & 63u)) & 1u) << 1;
-            const T *m = operands<T>(op) + 4 * sel;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) e[i] = operand(m[i]);
-            go = ((regs >> sel) & 1u) == 0;
             want = h.a();
-            regs = (1u << R) - 1u;
+            if (((d >> 16) & 3u) == 2u) {
+                sel |= ((uint32_t)(gb >> ((d >> 8) & 63u)) & 1u) << 1;
+                const T *m = operands<T>(op) + 4 * sel;
+                e0r = operand(m[0]), e0i = operand(m[1]), e1r = operand(m[2]), e1i = operand(m[3]);
+            } else {
+                e0r = sel ? h.m<T>(4) : e0r;
+                e0i = sel ? h.m<T>(5) : e0i;
+                e1r = sel ? h.m<T>(6) : e1r;
+                e1i = sel ? h.m<T>(7) : e1i;
+            }
+            go = ((d >> (20 + sel)) & 1u) == 0;
         }
         if (go) {
             const bool hit = (t & h.a()) == want;
-            if (f & kF_DL) {
-                diag_lane<T, R, FMA>(x, hit ? e[2] : e[0], hit ? e[3] : e[1], regs);
-            } else {
-                // entries (lane, register): e[0..3] without the lane condition, m[4..7] with it
-                T c0r = e[0], c0i = e[1], c1r = e[2], c1i = e[3];
+            if (f & kF_DR) {
+                // entries (lane, register): the pair without the lane condition, m[4..7] with it
+                T c0r = e0r, c0i = e0i, c1r = e1r, c1i = e1i;
                 if (!(f & kF_Out)) {
                     c0r = hit ? h.m<T>(4) : c0r;
                     c0i = hit ? h.m<T>(5) : c0i;
@@ -521,6 +555,19 @@ __device__ __forceinline__ void reg_diag(vec2_t<T> (&x)[R], const TileHead &h, c
                     if constexpr (R > 4) diag_rbit<T, R, 2, FMA>(x, c0r, c0i, c1r, c1i);
                 } else {
                     if constexpr (R > 8) diag_rbit<T, R, 3, FMA>(x, c0r, c0i, c1r, c1i);
+                }
+            } else if (!(f & kF_Id0) || __ballot(hit) != 0) {
+                if (f & kF_Neg) {
+                    const uint32_t bit = hit ? 0x80000000u : 0u;
+                    on_registers<T, R>(x, f, h.c(), [&](vec2_t<T> &v) {
+                        v.x = flip_sign(v.x, bit);
+                        v.y = flip_sign(v.y, bit);
+                    });
+                } else if (h.a() == 0) {  // the same entry on every lane
+                    on_registers<T, R>(x, f, h.c(), [&](vec2_t<T> &v) { cmul<T, FMA, true>(v, e1r, e1i); });
+                } else {
+                    const T dr = hit ? e1r : e0r, di = hit ? e1i : e0i;
+                    on_registers<T, R>(x, f, h.c(), [&](vec2_t<T> &v) { cmul<T, FMA>(v, dr, di); });
                 }
             }
         }
@@ -660,7 +707,7 @@ __device__ __forceinline__ void tile_store(vec2_t<T> *__restrict__ psi, const Ti
 // them are built without that code: its registers and code size slow every
 // other op down.
 template <typename T, int M, int RB, bool FMA, bool CUT>
-__device__ inline void tile_ops(vec2_t<T> (&x)[1 << RB], const TileDevOp *__restrict__ op, T *sa, uint64_t gb) {
+__device__ __forceinline__ void tile_ops(vec2_t<T> (&x)[1 << RB], const TileDevOp *__restrict__ op, T *sa, uint64_t gb) {
     constexpr int R = 1 << RB, TB = M - RB;
     const uint32_t t = threadIdx.x;
     TileHead h = *reinterpret_cast<const TileHead *>(op);
@@ -730,8 +777,12 @@ __device__ inline void tile_ops(vec2_t<T> (&x)[1 << RB], const TileDevOp *__rest
     }
 }
 
+// FP32 FMA forms are held to eight waves per SIMD, which limits their scalar
+// registers to 96 (layered circuit, 28 qubits: 1791 -> 1742 us per pass); the
+// FP64 forms lose by it (exact 3502 -> 4366 us, FMA unchanged).
 template <typename T, int M, int RB, bool FMA, bool CUT>
-__global__ __launch_bounds__(1 << (M - RB)) void k_tile(vec2_t<T> *__restrict__ psi, const TileArgs a,
+__global__ __launch_bounds__(1 << (M - RB))
+__attribute__((amdgpu_waves_per_eu(FMA && sizeof(T) == 4 ? 8 : 1))) void k_tile(vec2_t<T> *__restrict__ psi, const TileArgs a,
                                                        const TileDevOp *__restrict__ ops) {
     using V = vec2_t<T>;
     // the remap buffer: 2^M + 2^RB reals for FP64 (one component at a time),
@@ -772,13 +823,10 @@ struct TileEntry {
 
 // ZERO: some entry of the launch starts from |0...0> or has all-zero
 // blocks; launches without (every level after the first few) are built
-// without that code, which costs the exact FP64 forms 60 VGPRs.
-// FP64 FMA forms held to five waves per SIMD (96 VGPRs, 11 spilled; left
-// alone they take 108 and four waves, 5 % slower on the 512-instance QAOA
-// batch); the exact forms would spill ~100 values at five.
+// without that code.
 template <typename T, int M, int RB, bool FMA, bool CUT, bool ZERO>
 __global__ __launch_bounds__(1 << (M - RB))
-__attribute__((amdgpu_waves_per_eu(FMA && sizeof(T) == 8 ? 5 : 1))) void k_tile_batch(
+__attribute__((amdgpu_waves_per_eu(FMA && sizeof(T) == 4 ? 8 : 1))) void k_tile_batch(
     vec2_t<T> *__restrict__ base, const TileEntry *__restrict__ ent, const uint32_t *__restrict__ blk_ent,
     uint64_t total_blocks, uint32_t tiles_per_block, const char *__restrict__ op_buf) {
     using V = vec2_t<T>;
@@ -1405,12 +1453,24 @@ static void pack_tile_ops(int dtype, bool fma, uint32_t m, const std::vector<qvm
             }
             case QVMHIP_TILE_GDIAG: {
                 const uint32_t ng = o.q1 >> 16, sels = 1u << ng;
+                auto one = [&](uint32_t k) { return val(o, 2 * k) == 1.0 && val(o, 2 * k + 1) == 0.0; };
                 uint32_t ident = 0;
-                for (uint32_t k = 0; k < sels; ++k)
-                    if (val(o, 4 * k) == 1.0 && val(o, 4 * k + 1) == 0.0 && val(o, 4 * k + 2) == 1.0 &&
-                        val(o, 4 * k + 3) == 0.0)
-                        ident |= 1u << k;
-                emit(kF_Out | (bit ? kF_DR | bit : kF_DL), bit ? 0u : 1u << o.q0, o.q1, ident, o.m, 4 * sels * ts);
+                bool id0 = true, neg = true, same = true;  // entry 0 is 1, entry 1 is 1 or -1, no use of the local bit
+                for (uint32_t k = 0; k < sels; ++k) {
+                    if (one(2 * k) && one(2 * k + 1)) ident |= 1u << k;
+                    id0 = id0 && one(2 * k);
+                    neg = neg && (one(2 * k + 1) || (val(o, 4 * k + 2) == -1.0 && val(o, 4 * k + 3) == 0.0));
+                    same = same && val(o, 4 * k) == val(o, 4 * k + 2) && val(o, 4 * k + 1) == val(o, 4 * k + 3);
+                }
+                const uint32_t where = o.q1 | (ident << 20);
+                if (same) {  // no local qubit: one entry for the whole block
+                    emit(kF_DL | kF_Out | (neg ? kF_Neg : 0u), 0, where, 0, o.m, 4 * sels * ts);
+                } else if (id0) {  // entry 1 where the local bit is set
+                    emit(kF_DL | kF_Out | kF_Id0 | (neg ? kF_Neg : 0u) | bit, bit ? 0u : 1u << o.q0, where, 0, o.m,
+                         4 * sels * ts);
+                } else {
+                    emit(kF_Out | (bit ? kF_DR | bit : kF_DL), bit ? 0u : 1u << o.q0, where, 0, o.m, 4 * sels * ts);
+                }
                 break;
             }
             case kTileCutPhase: {
@@ -1430,7 +1490,7 @@ static void pack_tile_ops(int dtype, bool fma, uint32_t m, const std::vector<qvm
                 const bool r0 = o.q0 >= tb, r1 = two && o.q1 >= tb;
                 if (o.kind != QVMHIP_TILE_CPHASE && o.ctrl_mask == 0) {
                     if (!two) {
-                        emit(kF_DL, 1u << o.q0, 1u << o.q0, all, o.m, 4 * ts);
+                        emit(kF_DL, 1u << o.q0, 1u << o.q0, 0, o.m, 4 * ts);
                         break;
                     }
                     if (!r0 && !r1) {
@@ -1459,7 +1519,14 @@ static void pack_tile_ops(int dtype, bool fma, uint32_t m, const std::vector<qvm
                     if (v[2] == 1.0 && v[3] == 0.0) continue;
                     const uint32_t mask = o.ctrl_mask | tmask;
                     const uint32_t want = o.ctrl_mask | ((jj & 1u) << o.q0) | (two ? ((jj >> 1) & 1u) << o.q1 : 0u);
-                    emit_vals(kF_DL, mask & lanes, want & lanes, regs_with(mask >> tb, want >> tb), v, 4);
+                    const uint32_t regs = regs_with(mask >> tb, want >> tb);
+                    uint32_t f = kF_DL | kF_Id0 | (v[2] == -1.0 && v[3] == 0.0 ? kF_Neg : 0u);
+                    if (regs != all) {
+                        f |= kF_Mask;
+                        for (uint32_t r = 0; r < rb; ++r)
+                            if (regs == regs_with(1u << r, 1u << r)) f = (f & ~kF_Mask) | (kF_Bit0 << r);
+                    }
+                    emit_vals(f, mask & lanes, want & lanes, regs, v, 4);
                 }
             }
         }
