@@ -192,20 +192,23 @@ def _gdiag_op(U: np.ndarray, nat: Sequence[int], local) -> N.TileOp:
     return op
 
 
-def tile_op(U: np.ndarray, quil_qubits: Sequence[int], local) -> N.TileOp:
+def tile_op(U: np.ndarray, quil_qubits: Sequence[int], local, diag: Optional[bool] = None) -> N.TileOp:
     """Translate one 1- or 2-qubit gate into a tile op on local positions
-    (a diagonal gate may also name qubits outside the tile: GDIAG)."""
+    (a diagonal gate may also name qubits outside the tile: GDIAG).  diag:
+    whether U is diagonal, where the caller knows."""
     op = N.TileOp()
+    if diag is None:
+        diag = _is_diag(U)
     m = np.zeros(32)
     nat = G.nat_tuple(*quil_qubits)
     k = len(nat)
     if any(q not in local for q in nat):
-        if not _is_diag(U):
+        if not diag:
             raise ValueError("only diagonal gates may name qubits outside the tile")
         return _gdiag_op(U, nat, local)
     if k == 1:
         op.q0 = local[nat[0]]
-        if _is_diag(U):
+        if diag:
             op.kind = N.TILE_DIAG1
             d = np.diag(U)
             m[0:4] = [d[0].real, d[0].imag, d[1].real, d[1].imag]
@@ -216,10 +219,10 @@ def tile_op(U: np.ndarray, quil_qubits: Sequence[int], local) -> N.TileOp:
         op.q0, op.q1 = local[nat[0]], local[nat[1]]
         I4 = np.eye(4)
         d = np.diag(U)
-        if _is_diag(U) and d[0] == 1 and d[1] == 1 and d[2] == 1:
+        if diag and d[0] == 1 and d[1] == 1 and d[2] == 1:
             op.kind = N.TILE_CPHASE
             m[0:2] = [d[3].real, d[3].imag]
-        elif _is_diag(U):
+        elif diag:
             op.kind = N.TILE_DIAG2
             m[0:8] = np.ascontiguousarray(d).view(np.float64)
         elif np.array_equal(U, G.gate_matrix("CNOT")):
@@ -238,8 +241,7 @@ def tile_op(U: np.ndarray, quil_qubits: Sequence[int], local) -> N.TileOp:
             m[0:32] = np.ascontiguousarray(U).reshape(-1).view(np.float64)
     else:
         raise ValueError("tile ops are 1- or 2-qubit gates")
-    for i in range(32):
-        op.m[i] = m[i]
+    op.m[:] = m.tolist()
     return op
 
 
@@ -402,7 +404,7 @@ def plan_tiled(gates: List[Gate], nq: int, m: int, low: int = 4, merge_1q: bool 
             q += 1
         tq = sorted(T)
         local = {x: j for j, x in enumerate(tq)}
-        ops = [tile_op(gates[i][0], gates[i][1], local) for i in members]
+        ops = [tile_op(gates[i][0], gates[i][1], local, diag[i]) for i in members]
         plan.append(PlanItem("tile", tq, ops=ops, gates=members))
     return plan
 
@@ -443,7 +445,28 @@ def build_program(state, plan: List[PlanItem], use_graph: bool = True):
     return p
 
 
-def default_tile_m(dtype: str) -> int:
+def default_tile_m(dtype: str, nq: Optional[int] = None) -> int:
+    """Tile width of a program on nq qubits (without nq: of a large state).
+
+    A state of up to 18 qubits leaves most of the chip idle whatever the width,
+    and a pass costs what its ops take one after another on one block: a
+    narrower tile gives blocks of one or two waves with four or eight
+    amplitudes a thread, whose ops and relayouts are shorter, and that
+    outweighs the additional launches.  Measured in graph replays (us; layered
+    depth 8 / mix depth 8 / QFT):
+      FP64 exact, 12 qubits: m = 8 69 / 43 / 42, m = 11 89 / 54 / 47;
+        14: 8 81 / 50 / 51, 11 103 / 61 / 60; 17: 8 112 / 68 / 76, 11 127 / 80 / 85;
+        18: 8 133 / 82 / 89, 9 135 / 89 / 86, 11 142 / 90 / 96;
+        19: 9 162 / 117 / 113, 11 162 / 107 / 112
+      FP64 FMA, 18: 8 116 / 70 / 85, 9 112 / 73 / 79, 11 120 / 72 / 88
+      FP32 FMA, 14: 9 78 / 45 / 52, 12 104 / 54 / 59; 18: 9 113 / 66 / 86,
+        12 135 / 76 / 97; 19: 9 133 / 90 / 103, 12 144 / 89 / 107
+      FP32 exact, 18: 9 139 / 82 / 91, 12 145 / 86 / 99; 19: 9 159 / 105 / 109,
+        12 156 / 100 / 111
+    Up to 11 qubits the whole state is one block and any gate list one pass
+    (FP64, 10 qubits, QFT: one pass 30.0, m = 8 31.6; FMA 26.6 against 30.6)."""
+    if nq is not None and 12 <= nq <= 18:
+        return 8 if dtype == "f64" and nq <= 17 else 9
     return 11 if dtype == "f64" else 12
 
 
@@ -470,7 +493,7 @@ def compile_gates(state, gates: List[Gate], mode: str = "tiled", use_graph: bool
     if mode == "plain":
         plan = plan_plain(gates, nq)
     elif mode == "tiled":
-        plan = plan_tiled(gates, nq, m or default_tile_m(state.dtype), default_low(state.dtype), merge_1q,
+        plan = plan_tiled(gates, nq, m or default_tile_m(state.dtype, nq), default_low(state.dtype), merge_1q,
                           reorder)
     elif mode == "fused":
         plan = plan_fused(gates, nq, kmax)
