@@ -207,6 +207,33 @@ def dptr(a: np.ndarray):
     return a.ctypes.data_as(_dp)
 
 
+def cbuf(a: np.ndarray):
+    """A double * argument on the data of a C-contiguous array: what
+    dptr(a.view(np.float64)) gives, at a fifth of its cost for a writable one
+    (1.9 us, of some 7 per gate call)."""
+    if a.flags.writeable and a.flags.c_contiguous and a.nbytes >= 8:
+        return C.byref(C.c_double.from_buffer(a))
+    return dptr(a.view(np.float64))
+
+
+_U32X = [C.c_uint32 * k for k in range(7)]
+
+
+def u32args(xs):
+    """(argument, count) of a qubit list: a uint32 array.  Python integers
+    in range go straight into a C array; everything else goes through numpy, which
+    refuses or converts it."""
+    k = len(xs) if type(xs) in (tuple, list) else 0
+    if 1 <= k <= 6:
+        for x in xs:
+            if type(x) is not int or not 0 <= x < 64:
+                break
+        else:
+            return _U32X[k](*xs), k
+    q = u32arr(xs)
+    return u32ptr(q), len(q)
+
+
 def u32arr(xs) -> np.ndarray:
     return np.ascontiguousarray(np.asarray(xs, dtype=np.uint32))
 

@@ -80,11 +80,10 @@ class HipPureState:
     # -- gate application -------------------------------------------------
     def _mat_call(self, fn, U, qubits):
         U = N.cmat(U)
-        q = N.u32arr(qubits)
-        k = len(q)
+        q, k = N.u32args(qubits)
         if U.shape != (1 << k, 1 << k):
             raise ValueError(f"matrix shape {U.shape} does not match {k} qubits")
-        N.check(fn(self._h, N.dptr(U.view(np.float64)), k, N.u32ptr(q)))
+        N.check(fn(self._h, N.cbuf(U), k, q))
 
     def apply_matrix(self, U, qubits) -> None:
         """apply-matrix-operator (src/wavefunction.lisp:308-330)."""
