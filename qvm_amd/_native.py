@@ -115,6 +115,7 @@ SIGNATURES = {
     "qvmhip_read_amplitudes": [_vp, _u64, _u64, _dp],
     "qvmhip_accumulate": [_vp, _vp],
     "qvmhip_density_apply_kraus": [_vp, _u32, _dp, _u32, _u32, _u32p],
+    "qvmhip_density_apply_kraus_run": [_vp, _u32, _u32, _u32p, _u32p, _dp],
     "qvmhip_density_diagonal": [_vp, _u32, _dp],
     "qvmhip_read_wavefunction_be": [_vp, _u64, _u64, C.c_void_p],
     "qvmhip_read_probabilities_be": [_vp, _u64, _u64, C.c_void_p],

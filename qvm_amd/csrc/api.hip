@@ -263,6 +263,29 @@ int qvmhip_density_apply_kraus(qvmhip_state *s, uint32_t nq, const double *K, ui
     return launch_kraus(s, nq, K, count, k, qubits);
 }
 
+int qvmhip_density_apply_kraus_run(qvmhip_state *s, uint32_t nq, uint32_t nmaps, const uint32_t *qubits,
+                                   const uint32_t *counts, const double *K) {
+    if (!s) return fail(QVMHIP_EINVAL, "null state");
+    if (2 * nq != s->n) return fail(QVMHIP_EINVAL, "a density state of nq qubits has 2*nq qubits");
+    if (!qubits || !counts || !K) return fail(QVMHIP_EINVAL, "null argument");
+    const double *k = K;
+    const char *bad = nullptr;
+    uint32_t good = 0;
+    for (; good < nmaps && !bad; ++good) {
+        if (qubits[good] >= nq) bad = "qubit out of range for the density state";
+        if (counts[good] < 1) bad = "no Kraus operators";
+        for (uint32_t j = 0; j < counts[good] && !bad; ++j, k += 8)
+            if (!finite_matrix(k, 1)) bad = "matrix is not finite";
+    }
+    if (bad) --good;  // the map that is refused
+    DeviceScope ds(s->device);
+    if (good) {
+        const int rc = launch_kraus_run(s, nq, good, qubits, counts, K);
+        if (rc) return rc;
+    }
+    return bad ? fail(QVMHIP_EINVAL, bad) : QVMHIP_OK;
+}
+
 int qvmhip_apply_kraus_choice(qvmhip_state *s, const double *K, uint32_t count, uint32_t k, const uint32_t *qubits,
                               double r, uint32_t *index) {
     int rc = check_qubits(s, k, qubits);

@@ -246,6 +246,8 @@ int launch_gate(qvmhip_state *s, const double *U, uint32_t k, const uint32_t *qu
 bool gate_is_dense(const double *U, uint32_t k, const uint32_t *qubits);  // neither diagonal nor a permutation
 // sum_j K_j rho K_j^H on the density matrix of nq qubits held in s, 1 <= k <= 3
 int launch_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, uint32_t k, const uint32_t *qubits);
+int launch_kraus_run(qvmhip_state *s, uint32_t nq, uint32_t nmaps, const uint32_t *qubits, const uint32_t *counts,
+                     const double *K);
 // psi -> K_j psi / |K_j psi| for the first j whose running sum of |K_j psi|^2
 // reaches r (the last one when none does); 1 <= k <= 2
 int launch_kraus_choice(qvmhip_state *s, const double *K, uint32_t count, uint32_t k, const uint32_t *qubits, double r,
@@ -283,6 +285,9 @@ TileCode compile_tile_ops(int dtype, bool fma, uint32_t m, const qvmhip_tile_op 
 // public ops on the host / a compiled list on the device
 int launch_tile_pass(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, uint32_t nops,
                      const qvmhip_tile_op *ops);
+// the same without waiting for the stream
+int launch_tile_pass_async(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, uint32_t nops,
+                           const qvmhip_tile_op *ops);
 int launch_tile_code(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, const void *code_dev, bool cut);
 // A fused block's matrix in the layout its kernels read, and the launch with
 // that operand on the device.

@@ -1633,6 +1633,31 @@ int launch_tile_pass(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, u
     return rc;
 }
 
+// An op list travels to the state's operand slot in the arguments of small
+// launches, which are copied when they are enqueued: no host buffer has to
+// outlive the call, and the host does not wait.
+struct OpChunk {
+    uint4 w[192];
+};
+__global__ __launch_bounds__(192) void k_put_ops(uint4 *__restrict__ dst, const OpChunk c, uint32_t n) {
+    if (threadIdx.x < n) dst[threadIdx.x] = c.w[threadIdx.x];
+}
+
+int launch_tile_pass_async(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, uint32_t nops,
+                           const qvmhip_tile_op *ops) {
+    const TileCode code = compile_tile_ops(s->dtype, (s->flags & QVMHIP_FLAG_FMA_TILES) != 0, m, ops, nops);
+    if (code.bytes.size() > kFusedMatOffset) return launch_tile_pass(s, m, tile_qubits, nops, ops);
+    for (size_t off = 0; off < code.bytes.size(); off += sizeof(OpChunk)) {
+        const size_t n = std::min(sizeof(OpChunk), code.bytes.size() - off);  // slots: a multiple of 16 bytes
+        OpChunk c;
+        std::memcpy(&c, code.bytes.data() + off, n);
+        hipLaunchKernelGGL(k_put_ops, dim3(1), dim3(192), 0, s->stream, (uint4 *)((char *)s->mat + off), c,
+                           (uint32_t)(n / 16));
+        QH_LAUNCH_CHECK();
+    }
+    return launch_tile_code(s, m, tile_qubits, s->mat, code.cut);
+}
+
 size_t tile_entry_bytes() { return sizeof(TileEntry); }
 
 uint64_t build_tile_entry(void *entry, int dtype, bool fma, uint32_t n, uint32_t m, const uint32_t *tq,

@@ -94,26 +94,60 @@ class DensityQVM:
             raise QVMError("no program loaded")
         code = self.program.executable_code
         self.pc = 0
+        # a subclass that handles instructions or maps itself sees each of them
+        fuse = (type(self).transition is DensityQVM.transition and type(self)._kraus_ops is DensityQVM._kraus_ops
+                and type(self).apply_superoperator is DensityQVM.apply_superoperator)
         while self.pc is not None and self.pc < len(code):
+            if fuse and self._run_maps(code):
+                continue
             self.pc = self.transition(code[self.pc])
         return self
+
+    def _run_maps(self, code) -> bool:
+        """Apply the 1-qubit gates from pc up to the next other instruction
+        in shared sweeps (12 qubits: 73 us a gate on its own) and advance pc.
+        False, with nothing done, when fewer than two follow each other.  A gate
+        that cannot be resolved ends the run: its own transition reports it."""
+        maps = []
+        for i in range(self.pc, len(code)):
+            ins = code[i]
+            if not isinstance(ins, Q.GateApplication) or len(ins.qubits) != 1:
+                break
+            q = ins.qubits[0]
+            try:
+                ops = self._kraus_ops(ins)
+            except Exception:
+                break
+            if not ops or not 0 <= q < self.number_of_qubits or any(K.shape != (2, 2) for K in ops):
+                break
+            maps.append((ops, q))
+        if len(maps) < 2:
+            return False
+        self.state.density_apply_kraus_run(self.number_of_qubits, maps)
+        self.pc += len(maps)
+        return True
 
     def _draw(self) -> float:
         self.draws_used += 1
         return float(self.rng())
 
+    def _kraus_ops(self, ins) -> List[np.ndarray]:
+        """The Kraus operators of a gate application: its noisy definition,
+        or its matrix."""
+        if ins.modifiers:
+            raise QVMError("The density QVM doesn't support gate modifiers.")
+        ops = self.noisy_gate_definitions.get((ins.name.upper(), tuple(ins.qubits)))
+        if ops is None:
+            U = Q.resolve_gate_matrix(ins, self.program.gate_definitions if self.program else {}, self.memory)
+            if G.num_qubits_of(U) != len(ins.qubits):
+                raise QVMError(f"Gate {ins.name} takes {G.num_qubits_of(U)} qubit(s), "
+                               f"applied to {len(ins.qubits)}")
+            ops = [U]
+        return ops
+
     def transition(self, ins):
         if isinstance(ins, Q.GateApplication):
-            if ins.modifiers:
-                raise QVMError("The density QVM doesn't support gate modifiers.")
-            ops = self.noisy_gate_definitions.get((ins.name.upper(), tuple(ins.qubits)))
-            if ops is None:
-                U = Q.resolve_gate_matrix(ins, self.program.gate_definitions if self.program else {}, self.memory)
-                if G.num_qubits_of(U) != len(ins.qubits):
-                    raise QVMError(f"Gate {ins.name} takes {G.num_qubits_of(U)} qubit(s), "
-                                   f"applied to {len(ins.qubits)}")
-                ops = [U]
-            self.apply_superoperator(ops, ins.qubits)
+            self.apply_superoperator(self._kraus_ops(ins), ins.qubits)
             return self.pc + 1
         if isinstance(ins, Q.Measure):
             if ins.target is None:

@@ -297,6 +297,16 @@ class HipPureState:
         N.check(N.lib().qvmhip_density_apply_kraus(self._h, int(nq), N.dptr(K.view(np.float64)), len(K), k,
                                                    N.u32ptr(q)))
 
+    def density_apply_kraus_run(self, nq: int, maps) -> None:
+        """The 1-qubit maps [(Kraus operators, qubit), ...] in order, as
+        density_apply_kraus one after another up to rounding, in shared sweeps."""
+        K = N.cmat([k for ops, _ in maps for k in ops])
+        if K.shape[1:] != (2, 2):
+            raise ValueError(f"matrix shape {K.shape[1:]} does not match 1 qubit")
+        q, counts = N.u32arr([q for _, q in maps]), N.u32arr([len(ops) for ops, _ in maps])
+        N.check(N.lib().qvmhip_density_apply_kraus_run(self._h, int(nq), len(maps), N.u32ptr(q), N.u32ptr(counts),
+                                                       N.cbuf(K)))
+
     def density_diagonal(self, nq: int) -> np.ndarray:
         """Re rho[i][i] of the density matrix this 2*nq-qubit state holds
         as vec(rho), row-major."""

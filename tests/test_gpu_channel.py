@@ -123,3 +123,74 @@ def test_kraus_choice_refuses_an_annihilated_state():
             st.apply_kraus_choice(np.full((1, 2, 2), np.inf), [0], 0.5)
         # an operator past the chosen one is never looked at
         assert st.apply_kraus_choice(np.stack([np.eye(2), np.eye(2) * np.nan]), [0], 0.5) == 0
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 6, 7])
+def test_density_run_of_maps_matches_kraus_sums(dtype, n):
+    """A run of 1-qubit maps (dense, diagonal, several on one qubit; below the
+    smallest tile, one pass, several passes) against numpy, entry by entry.
+    Bound: (4 + 2 count + 4) roundings per map as for a single one, of entries of
+    order 2^-n, the maps contracting."""
+    from qvm_amd.state import HipPureState
+    rng = np.random.default_rng(40 + n)
+    d = 1 << n
+    u = 2.0 ** (-53 if dtype == "f64" else -24)
+    maps = []
+    for i in range(2 * n + 3):
+        q = int(rng.integers(n)) if i < n + 3 else i - n - 3
+        if i % 3 == 2:
+            p = rng.uniform(0.1, 0.4)
+            maps.append(([np.sqrt(1 - p) * np.eye(2), np.sqrt(p) * G.gate_matrix("Z") @ G.gate_matrix("S")], q))
+        else:
+            maps.append((list(kraus_list(1 + i % 4, 1, rng)), q))
+    tol = sum(8 + 2 * len(ops) for ops, _ in maps) * u
+    A = rng.normal(size=(d, d)) + 1j * rng.normal(size=(d, d))
+    rho = A @ A.conj().T
+    rho /= np.trace(rho)
+    with HipPureState(2 * n, dtype) as st:
+        st.write_amplitudes(rho.reshape(-1))
+        st.density_apply_kraus_run(n, maps)
+        got = st.amplitudes().reshape(d, d)
+    for ops, q in maps:
+        rho = sum(embed(K, [q], n) @ rho @ embed(K, [q], n).conj().T for K in ops)
+    assert np.max(np.abs(got - rho)) <= tol
+
+
+def test_density_run_refuses_and_keeps_the_maps_before():
+    from qvm_amd._native import QVMHipError
+    from qvm_amd.state import HipPureState
+    X, bad = G.gate_matrix("X"), np.full((2, 2), np.nan)
+    for maps in ([([X], 1), ([bad], 0)], [([X], 1), ([X], 4)]):
+        with HipPureState(8) as st:
+            with pytest.raises(QVMHipError):
+                st.density_apply_kraus_run(4, maps)
+            assert st.density_diagonal(4)[2] == 1.0
+    with HipPureState(8) as st, pytest.raises(QVMHipError):
+        st.density_apply_kraus_run(3, [([X], 1), ([X], 2)])
+
+
+def test_density_program_fuses_runs_only_between_other_instructions():
+    """The interpreter's shared sweeps against one instruction at a time:
+    runs broken by 2-qubit gates, a label and a measurement, a noisy definition,
+    an unresolvable gate after a run."""
+    from qvm_amd.density import DensityQVM
+    from qvm_amd.qvm import QVMError
+    g = 0.3
+    noise = {("I", (1,)): [np.diag([1, np.sqrt(1 - g)]), np.array([[0, np.sqrt(g)], [0, 0]])]}
+    text = ("DECLARE ro BIT[5]\n" + "".join(f"RX(0.{q + 1}) {q}\nH {q}\n" for q in range(5))
+            + "I 1\nCNOT 0 1\nRZ(0.4) 2\nLABEL @a\nRY(1.0) 2\nI 1\nX 3\nMEASURE 3 ro[3]\nH 3\nT 3\n")
+    got = []
+    for cls in (DensityQVM, type("OneByOne", (DensityQVM,), {"transition": lambda s, i: DensityQVM.transition(s, i)})):
+        qvm = cls(5, noisy_gate_definitions=noise, rng=lambda: 0.25)
+        qvm.load_program(text)
+        qvm.run()
+        got.append((qvm.amplitudes(), list(qvm.memory["ro"]), qvm.pc))
+        qvm.reset_quantum_state()
+        qvm.load_program("X 0\nX 1\nDAGGER S 2\n")
+        with pytest.raises(QVMError):
+            qvm.run()
+        assert qvm.pc == 2 and qvm.measurement_probabilities()[3] == 1.0
+        qvm.close()
+    assert got[0][1:] == got[1][1:]
+    assert np.max(np.abs(got[0][0] - got[1][0])) <= 25 * 12 * 2.0 ** -53
