@@ -99,6 +99,7 @@ SIGNATURES = {
     "qvmhip_prob_ground": [_vp, _u32, _dp],
     "qvmhip_norm": [_vp, _dp],
     "qvmhip_total_probability": [_vp, _dp],
+    "qvmhip_apply_1q_run": [_vp, _u32, _u32p, _dp, C.c_int],
     "qvmhip_apply_kraus_choice": [_vp, _dp, _u32, _u32, _u32p, C.c_double, _u32p],
     "qvmhip_normalize": [_vp, C.c_double],
     "qvmhip_probabilities": [_vp, _u64, _u64, _dp],

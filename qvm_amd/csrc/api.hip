@@ -286,6 +286,17 @@ int qvmhip_density_apply_kraus_run(qvmhip_state *s, uint32_t nq, uint32_t nmaps,
     return bad ? fail(QVMHIP_EINVAL, bad) : QVMHIP_OK;
 }
 
+int qvmhip_apply_1q_run(qvmhip_state *s, uint32_t count, const uint32_t *qubits, const double *U, int normalize) {
+    if (!s) return fail(QVMHIP_EINVAL, "null state");
+    if (!qubits || !U || count < 1) return fail(QVMHIP_EINVAL, "null argument or no gates");
+    for (uint32_t i = 0; i < count; ++i) {
+        if (qubits[i] >= s->n) return fail(QVMHIP_EINVAL, "qubit out of range");
+        if (!finite_matrix(U + 8 * (size_t)i, 1)) return fail(QVMHIP_EINVAL, "matrix is not finite");
+    }
+    DeviceScope ds(s->device);
+    return launch_1q_run(s, count, qubits, U, normalize != 0);
+}
+
 int qvmhip_apply_kraus_choice(qvmhip_state *s, const double *K, uint32_t count, uint32_t k, const uint32_t *qubits,
                               double r, uint32_t *index) {
     int rc = check_qubits(s, k, qubits);

@@ -76,12 +76,40 @@ int launch_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, 
     return launch_fused_dense(s, dst, 2 * k, q);
 }
 
+// The tile of the next pass over the qubits on[i], on[i + 1], ...: as many as
+// fit 11 (FP64) or 12 (FP32) index bits beside the low bits that keep accesses
+// whole lines; a qubit brings bit q and, on a density state, bit q + nq.  i
+// moves past them.
+namespace {
+struct TileGroup {
+    uint32_t m, tq[16], local[64];
+    std::vector<uint32_t> members;
+    TileGroup(const qvmhip_state *s, const std::vector<uint32_t> &on, size_t &i, uint32_t nq) {
+        const bool f64 = s->dtype == QVMHIP_F64;
+        const uint32_t low = f64 ? 3 : 4;
+        m = std::min<uint32_t>(s->n, f64 ? 11 : 12);
+        uint64_t tile = (uint64_t(1) << low) - 1;
+        for (; i < on.size(); ++i) {
+            const uint64_t with = tile | uint64_t(1) << on[i] | uint64_t(1) << (on[i] + nq);
+            if ((uint32_t)__builtin_popcountll(with) > m) break;  // never at the first: low + 2 <= 8 <= m
+            tile = with;
+            members.push_back(on[i]);
+        }
+        for (uint32_t q = 0; (uint32_t)__builtin_popcountll(tile) < m; ++q) tile |= uint64_t(1) << q;
+        uint32_t nb = 0;
+        for (uint32_t q = 0; q < s->n; ++q)
+            if ((tile >> q) & 1u) {
+                local[q] = nb;
+                tq[nb++] = q;
+            }
+    }
+};
+}  // namespace
+
 // A run of 1-qubit maps.  Each would be a sweep of its own (73 us at 2^24 FP64
 // amplitudes, bound by memory), but maps on one qubit multiply to one 4x4 and
 // maps on different qubits commute, so the run is at most one 4x4 per qubit,
-// and these share tile passes: qubit q brings the index bits q and q + nq,
-// five or four qubits fit the 11 bits of a pass (FP64; 12 bits FP32) beside the
-// low bits that keep its accesses whole lines.  24 gates on 12 qubits: three
+// and these share tile passes, five or four qubits each.  24 gates on 12 qubits: three
 // passes of 124 us instead of 24 sweeps, and the noisy circuit above 6.3 ->
 // 2.1 ms (its 11 two-qubit maps are 0.9 of that).  Less than two qubits, or a
 // state below the smallest tile (2^8), stay sweeps.
@@ -124,40 +152,86 @@ int launch_kraus_run(qvmhip_state *s, uint32_t nq, uint32_t nmaps, const uint32_
         }
         return QVMHIP_OK;
     }
-    const bool f64 = s->dtype == QVMHIP_F64;
-    const uint32_t m = std::min<uint32_t>(s->n, f64 ? 11 : 12), low = f64 ? 3 : 4;
     for (size_t i = 0; i < on.size();) {
-        uint64_t tile = (uint64_t(1) << low) - 1;
-        std::vector<uint32_t> members;
-        for (; i < on.size(); ++i) {
-            const uint64_t with = tile | uint64_t(1) << on[i] | uint64_t(1) << (on[i] + nq);
-            if ((uint32_t)__builtin_popcountll(with) > m) break;  // never at the first: low + 2 <= m
-            tile = with;
-            members.push_back(on[i]);
-        }
-        for (uint32_t q = 0; (uint32_t)__builtin_popcountll(tile) < m; ++q) tile |= uint64_t(1) << q;
-        uint32_t tq[16], local[64], nb = 0;
-        for (uint32_t q = 0; q < s->n; ++q)
-            if ((tile >> q) & 1u) {
-                local[q] = nb;
-                tq[nb++] = q;
-            }
+        TileGroup g(s, on, i, nq);
         std::vector<qvmhip_tile_op> ops;
-        for (uint32_t q : members) {
+        for (uint32_t q : g.members) {
             qvmhip_tile_op op;
             std::memset(&op, 0, sizeof(op));
             op.kind = QVMHIP_TILE_DIAG2;
             for (int r = 0; r < 16; ++r)
                 if (r % 5 && S[q][r] != cd(0, 0)) op.kind = QVMHIP_TILE_DENSE2;
-            op.q0 = local[q];
-            op.q1 = local[q + nq];
+            op.q0 = g.local[q];
+            op.q1 = g.local[q + nq];
             for (int r = 0, j = 0; r < 16; r += op.kind == QVMHIP_TILE_DIAG2 ? 5 : 1, ++j) {
                 op.m[2 * j] = S[q][r].real();
                 op.m[2 * j + 1] = S[q][r].imag();
             }
             ops.push_back(op);
         }
-        if (const int rc = launch_tile_pass_async(s, m, tq, (uint32_t)ops.size(), ops.data())) return rc;
+        if (const int rc = launch_tile_pass_async(s, g.m, g.tq, (uint32_t)ops.size(), ops.data())) return rc;
+    }
+    return QVMHIP_OK;
+}
+
+// A run of 1-qubit gates on a pure state (a sweep of 73 us each at 2^24 FP64
+// amplitudes), multiplied together per qubit and applied up to eleven qubits a
+// pass.  normalize, for unitary gates: the state ends with norm 1; its norm is
+// read before the last pass, whose first matrix takes the factor.
+int launch_1q_run(qvmhip_state *s, uint32_t count, const uint32_t *qubits, const double *U, bool normalize) {
+    std::vector<std::vector<cd>> S(s->n);
+    const cd *u = reinterpret_cast<const cd *>(U);
+    bool finite = true;
+    for (uint32_t i = 0; i < count; ++i, u += 4) {
+        std::vector<cd> &B = S[qubits[i]];
+        if (B.empty()) {
+            B.assign(u, u + 4);
+            continue;
+        }
+        const cd P[4] = {u[0] * B[0] + u[1] * B[2], u[0] * B[1] + u[1] * B[3], u[2] * B[0] + u[3] * B[2],
+                         u[2] * B[1] + u[3] * B[3]};
+        for (const cd &x : P) finite = finite && std::isfinite(x.real()) && std::isfinite(x.imag());
+        B.assign(P, P + 4);
+    }
+    if (!finite) return fail(QVMHIP_ERANGE, "the product of the run's gates is not finite");
+    std::vector<uint32_t> on;
+    for (uint32_t q = 0; q < s->n; ++q)
+        if (!S[q].empty()) on.push_back(q);
+    auto scale = [&](std::vector<cd> &A) -> int {
+        double n2 = 0;
+        if (const int rc = reduce_norm2(s, &n2)) return rc;
+        const double len = std::sqrt(n2);
+        if (!(len > 0) || !std::isfinite(len)) return fail(QVMHIP_ERANGE, "cannot normalize a zero/non-finite state");
+        for (cd &x : A) x *= 1.0 / len;
+        return QVMHIP_OK;
+    };
+    if (on.size() < 2 || s->n < 8) {
+        for (uint32_t q : on) {
+            if (normalize && q == on.back())
+                if (const int rc = scale(S[q])) return rc;
+            if (const int rc = launch_gate(s, reinterpret_cast<const double *>(S[q].data()), 1, &q, 0)) return rc;
+        }
+        return QVMHIP_OK;
+    }
+    for (size_t i = 0; i < on.size();) {
+        TileGroup g(s, on, i, 0);
+        if (normalize && i == on.size())
+            if (const int rc = scale(S[g.members[0]])) return rc;
+        std::vector<qvmhip_tile_op> ops;
+        for (uint32_t q : g.members) {
+            const std::vector<cd> &A = S[q];
+            qvmhip_tile_op op;
+            std::memset(&op, 0, sizeof(op));
+            const bool diag = A[1] == cd(0, 0) && A[2] == cd(0, 0);
+            op.kind = diag ? QVMHIP_TILE_DIAG1 : QVMHIP_TILE_DENSE1;
+            op.q0 = g.local[q];
+            for (int r = 0, j = 0; r < 4; r += diag ? 3 : 1, ++j) {
+                op.m[2 * j] = A[r].real();
+                op.m[2 * j + 1] = A[r].imag();
+            }
+            ops.push_back(op);
+        }
+        if (const int rc = launch_tile_pass_async(s, g.m, g.tq, (uint32_t)ops.size(), ops.data())) return rc;
     }
     return QVMHIP_OK;
 }

@@ -246,6 +246,7 @@ int launch_gate(qvmhip_state *s, const double *U, uint32_t k, const uint32_t *qu
 bool gate_is_dense(const double *U, uint32_t k, const uint32_t *qubits);  // neither diagonal nor a permutation
 // sum_j K_j rho K_j^H on the density matrix of nq qubits held in s, 1 <= k <= 3
 int launch_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, uint32_t k, const uint32_t *qubits);
+int launch_1q_run(qvmhip_state *s, uint32_t count, const uint32_t *qubits, const double *U, bool normalize);
 int launch_kraus_run(qvmhip_state *s, uint32_t nq, uint32_t nmaps, const uint32_t *qubits, const uint32_t *counts,
                      const double *K);
 // psi -> K_j psi / |K_j psi| for the first j whose running sum of |K_j psi|^2

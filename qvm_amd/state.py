@@ -134,6 +134,15 @@ class HipPureState:
         N.check(N.lib().qvmhip_total_probability(self._h, C.byref(out)))
         return out.value
 
+    def apply_1q_run(self, mats, qubits, normalize: bool = False) -> None:
+        """The 1-qubit gates mats[i] on qubits[i], in order, as apply_matrix one
+        after another up to rounding, in shared sweeps; ``normalize`` (for
+        unitary gates) also divides the state by its norm."""
+        U, q = N.cmat(mats), N.u32arr(qubits)
+        if U.shape != (len(q), 2, 2):
+            raise ValueError(f"matrices of shape {U.shape} for {len(q)} 1-qubit gates")
+        N.check(N.lib().qvmhip_apply_1q_run(self._h, len(q), N.u32ptr(q), N.cbuf(U), 1 if normalize else 0))
+
     def apply_kraus_choice(self, kraus_ops, qubits, r: float) -> int:
         """The state becomes K_j psi / |K_j psi|, j the first operator whose
         running sum of |K_j psi|^2 reaches r (``qubits`` in nat-tuple order, 1

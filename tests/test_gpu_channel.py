@@ -194,3 +194,67 @@ def test_density_program_fuses_runs_only_between_other_instructions():
         qvm.close()
     assert got[0][1:] == got[1][1:]
     assert np.max(np.abs(got[0][0] - got[1][0])) <= 25 * 12 * 2.0 ** -53
+
+
+def _noisy_pair(n, dtype, defs, text, draws, amps=None):
+    """(amplitudes, memory, draws used) of a program run with shared sweeps
+    and one instruction at a time."""
+    from qvm_amd.noise import NoisyQVM
+    out = []
+    for cls in (NoisyQVM, type("OneByOne", (NoisyQVM,), {"transition": lambda s, i: NoisyQVM.transition(s, i)})):
+        qvm = cls(n, noisy_gate_definitions=defs, dtype=dtype, rng=iter(draws).__next__)
+        if amps is not None:
+            qvm.set_amplitudes(amps)
+        qvm.load_program(text)
+        qvm.run()
+        out.append((qvm.amplitudes(), list(qvm.memory.get("ro", [])), qvm.draws_used))
+        qvm.close()
+    return out
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("n", [2, 7, 8, 12, 13])
+def test_noisy_runs_match_one_by_one(dtype, n):
+    """Runs of unitary and unitary-mixture gates (below the smallest tile, one
+    pass, several) around gates that end a run: amplitude damping, a noisy CNOT, a
+    measurement.  The state starts with norm 1.5.  Bound: eight roundings of values
+    up to 1.5 per gate on either side."""
+    rng = np.random.default_rng(n)
+    m = G.gate_matrix
+    defs = {}
+    for q in range(n):
+        p = rng.uniform(0.1, 0.3, 3)
+        defs["H", (q,)] = [np.sqrt(1 - p.sum()) * m("H")] + [np.sqrt(x) * m(P) @ m("H") for x, P in zip(p, "XYZ")]
+    g = 0.4
+    defs["I", (0,)] = [np.diag([1, np.sqrt(1 - g)]), np.array([[0, np.sqrt(g)], [0, 0]])]
+    defs["CNOT", (0, 1)] = [np.sqrt(0.7) * m("CNOT"), np.sqrt(0.3) * np.kron(m("Z"), m("Z")) @ m("CNOT")]
+    layer = "".join(f"RX({rng.uniform(0, 6):.6f}) {q}\n" for q in range(n)) + "".join(f"H {q}\n" for q in range(n))
+    text = ("DECLARE ro BIT[2]\n" + layer + "I 0\nCNOT 0 1\n" + layer + "T 1\nMEASURE 0 ro[0]\nH 1\nS 0\nH 0\n"
+            + "I 0\nX 1\n")
+    amps = rng.normal(size=1 << n) + 1j * rng.normal(size=1 << n)
+    amps *= 1.5 / np.linalg.norm(amps)
+    for trial in range(4):
+        draws = rng.random(6 * n + 20)
+        (a, ra, da), (b, rb, db) = _noisy_pair(n, dtype, defs, text, draws, amps)
+        assert ra == rb and da == db
+        u = 2.0 ** (-53 if dtype == "f64" else -24)
+        assert np.max(np.abs(a - b)) <= 2 * 8 * 1.5 * (4 * n + 10) * u
+        assert abs(np.linalg.norm(a) - 1) <= (4 * n + 10) * 8 * u
+
+
+def test_noisy_run_takes_no_draw_for_a_gate_it_does_not_cover():
+    """Damping only, a plain matrix that is not unitary, a modifier on a noisy gate."""
+    from qvm_amd.noise import NoisyQVM
+    from qvm_amd.qvm import QVMError
+    g = 0.5
+    damp = [np.diag([1, np.sqrt(1 - g)]), np.array([[0, np.sqrt(g)], [0, 0]])]
+    mix = [np.sqrt(0.5) * G.gate_matrix("X"), np.sqrt(0.5) * G.gate_matrix("Z") @ G.gate_matrix("X")]
+    text = "DEFGATE A:\n    1.0, 0\n    0, 0.5\n\nX 0\nX 0\nA 0\nH 0\nI 0\nI 0\n"
+    (a, _, da), (b, _, db) = _noisy_pair(2, "f64", {("I", (0,)): damp, ("X", (0,)): mix}, text, [0.3, 0.9, 0.2, 0.6])
+    assert da == db == 4 and np.max(np.abs(a - b)) <= 1e-15 * 8
+    qvm = NoisyQVM(2, noisy_gate_definitions={("X", (0,)): mix}, rng=lambda: 0.1)
+    qvm.load_program("X 0\nX 0\nDAGGER X 0\n")
+    with pytest.raises(QVMError):
+        qvm.run()
+    assert qvm.draws_used == 2 and qvm.pc == 2
+    qvm.close()
