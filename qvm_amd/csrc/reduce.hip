@@ -1,9 +1,9 @@
 // reduce.hip -- probability reductions, measurement collapse and sampling.
 //
-// Reductions accumulate |psi_i|^2 in FP64 for both state dtypes: each thread
-// sums a grid-strided slice, a wavefront reduces with cross-lane shuffles, the
-// waves of a block combine in LDS, and one block adds the block partials in a
-// fixed order (deterministic: same input -> same bits).
+// Reductions accumulate |psi_i|^2 in FP64 for both state dtypes: each workgroup
+// sums a contiguous segment, a wavefront reduces with cross-lane shuffles, the
+// waves of a block combine in LDS, and the host (few partials) or one block adds
+// the block partials in a fixed order (deterministic: same input -> same bits).
 //
 // Sampling (measure-all and multi-shot) is a two-level search over the
 // cumulative distribution C(b) = sum_{i<=b} |psi_i|^2:

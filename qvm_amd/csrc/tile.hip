@@ -621,11 +621,9 @@ __device__ __forceinline__ uint32_t lds_addr(uint32_t s) {
 }
 
 // src4: the op's first 16 operand bytes as four words; byte j is the old
-// slot bit of new slot bit j.  FP64 blocks go through LDS one component at a
-// time (real parts, then imaginary parts): the exchange buffer is then 2^M
-// doubles, half a block, and five workgroups fit on a CU instead of four
-// (measured at n = 30: 8.23 -> 7.84 ms per exact pass, 7.50 -> 7.13 FMA).
-// FP32 blocks move whole amplitudes (split, they lost 2.5-6 %).
+// slot bit of new slot bit j.  Blocks go through LDS one component at a time
+// (real parts, then imaginary parts): the exchange buffer is half a block, and
+// more workgroups fit on a CU.
 template <typename T, int R, int TB>
 __device__ __forceinline__ void reg_remap(vec2_t<T> (&x)[R], T *sa, const uint32_t (&src4)[4], uint32_t t) {
     constexpr uint32_t NT = 1u << TB;
@@ -785,8 +783,7 @@ __global__ __launch_bounds__(1 << (M - RB))
 __attribute__((amdgpu_waves_per_eu(FMA && sizeof(T) == 4 ? 8 : 1))) void k_tile(vec2_t<T> *__restrict__ psi, const TileArgs a,
                                                        const TileDevOp *__restrict__ ops) {
     using V = vec2_t<T>;
-    // the remap buffer: 2^M + 2^RB reals for FP64 (one component at a time),
-    // as many amplitudes for FP32
+    // the remap buffer: one component of the block (2^M reals, padded rows)
     __shared__ __align__(16) T sa[(1 << M) + (1 << RB)];
     const uint64_t toff = thread_offset<M - RB>(a, threadIdx.x);
     // One tile per workgroup (grid-striding only past the dispatch limit):
@@ -830,8 +827,7 @@ __attribute__((amdgpu_waves_per_eu(FMA && sizeof(T) == 4 ? 8 : 1))) void k_tile_
     vec2_t<T> *__restrict__ base, const TileEntry *__restrict__ ent, const uint32_t *__restrict__ blk_ent,
     uint64_t total_blocks, uint32_t tiles_per_block, const char *__restrict__ op_buf) {
     using V = vec2_t<T>;
-    // the remap buffer: 2^M + 2^RB reals for FP64 (one component at a time),
-    // as many amplitudes for FP32
+    // the remap buffer: one component of the block (2^M reals, padded rows)
     __shared__ __align__(16) T sa[(1 << M) + (1 << RB)];
     // round robin over the XCDs (no xcd_block): work blocks of different
     // entries differ in cost, and contiguous shares per XCD measured 5-6 %

@@ -8,6 +8,8 @@ state, so every operation is one of the pure-state kernels:
     gate U on qubits q          U* on q and U on the ghosts q + n
                                 (vec(A rho B) = (A (x) B^T) vec(rho),
                                 src/apply-gate.lisp:40-65)
+    runs of 1-qubit gates       multiplied together per qubit, several qubits a
+                                tile pass (qvmhip_density_apply_kraus_run)
     Kraus list {K_j}            sum_j (K_j (x) K_j*) vec(rho): one sweep with the
                                 map's superoperator (qvmhip_density_apply_kraus,
                                 up to 3 qubits), else a pristine copy and a
