@@ -244,9 +244,9 @@ constexpr int kraus_per_read(int k) { return k == 1 ? 4 : 2; }
 constexpr int kNormBlocks = 1024;  // partials of kNormBlocks * 4 sums fit the state's reduction scratch
 static_assert(kNormBlocks * 4 <= kRedBlocks * 2, "reduction scratch");
 
-template <typename T, int K>
+template <typename T, int K, int C>
 struct KrausArgs {
-    static constexpr int D = 1 << K, C = kraus_per_read(K);
+    static constexpr int D = 1 << K;
     GroupSpec g;
     uint64_t off[D];
     T ur[C * D * D];
@@ -255,29 +255,36 @@ struct KrausArgs {
 
 // partial[C * block + j] = the block's share of sum |K_j x|^2, in FP64; the
 // products are rounded in T and summed left to right, as the gate kernels do.
-// Bound by the read; UN groups per thread are in flight.
-template <typename T, int K>
-__global__ __launch_bounds__(kBlock) void k_kraus_norms(const vec2_t<T> *__restrict__ psi, const KrausArgs<T, K> a,
+// Bound by the read; UN groups per thread are in flight.  For one qubit a
+// workgroup takes a contiguous segment of the groups, and maps of one or two
+// operators form two products, not four: 2^24 FP64 amplitudes 47.4 -> 40.3 us
+// (6.7 TB/s).  For two qubits segments gained nothing (58.9 us against 57.7), and the
+// grid strides over the groups.
+template <typename T, int K, int C, bool NTM>
+__global__ __launch_bounds__(kBlock) void k_kraus_norms(const vec2_t<T> *__restrict__ psi, const KrausArgs<T, K, C> a,
                                                         double *__restrict__ partial) {
-    constexpr int D = 1 << K, C = kraus_per_read(K), UN = K == 1 ? 4 : 2, NW = kBlock / 64;
+    constexpr int D = 1 << K, UN = K == 1 ? 4 : 2, NW = kBlock / 64;
     using V = vec2_t<T>;
     __shared__ double sm[C][NW];
     double acc[C];
 #pragma unroll
     for (int j = 0; j < C; ++j) acc[j] = 0.0;
-    const uint64_t step = (uint64_t)gridDim.x * kBlock;
-    for (uint64_t i0 = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i0 < a.g.ngroups; i0 += UN * step) {
+    // 1 qubit: a segment per workgroup (both counts are powers of two)
+    const uint64_t step = K == 1 ? kBlock : (uint64_t)gridDim.x * kBlock;
+    const uint64_t seg = K == 1 ? a.g.ngroups / gridDim.x : a.g.ngroups;
+    const uint64_t first = K == 1 ? seg * xcd_block(blockIdx.x, gridDim.x) : 0;
+    for (uint64_t i0 = (K == 1 ? 0 : (uint64_t)blockIdx.x * kBlock) + threadIdx.x; i0 < seg; i0 += UN * step) {
         V x[UN][D];
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
             const uint64_t i = i0 + u * step;
-            const uint64_t base = group_base(a.g, i < a.g.ngroups ? i : i0);
+            const uint64_t base = group_base(a.g, first + (i < seg ? i : i0));
 #pragma unroll
-            for (int d = 0; d < D; ++d) x[u][d] = psi[base + a.off[d]];
+            for (int d = 0; d < D; ++d) x[u][d] = ldg<NTM>(&psi[base + a.off[d]]);
         }
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
-            if (i0 + u * step >= a.g.ngroups) break;
+            if (i0 + u * step >= seg) break;
 #pragma unroll
             for (int j = 0; j < C; ++j)
 #pragma unroll
@@ -311,11 +318,11 @@ __global__ __launch_bounds__(kBlock) void k_kraus_norms(const vec2_t<T> *__restr
     }
 }
 
-// out[j] = |K_j psi|^2 for the first `count` (at most kraus_per_read(K)) operators.
-template <typename T, int K>
-static int kraus_norms(qvmhip_state *s, const cd *ops, uint32_t count, const uint32_t *qubits, double *out) {
-    constexpr int D = 1 << K, C = kraus_per_read(K);
-    KrausArgs<T, K> a;
+// out[j] = |K_j psi|^2 for the first `count` (at most C) operators.
+template <typename T, int K, int C>
+static int kraus_norms_c(qvmhip_state *s, const cd *ops, uint32_t count, const uint32_t *qubits, double *out) {
+    constexpr int D = 1 << K;
+    KrausArgs<T, K, C> a;
     std::memset(&a, 0, sizeof(a));
     a.g.nsorted = K;
     for (int b = 0; b < K; ++b) a.g.sorted[b] = qubits[b];
@@ -329,10 +336,21 @@ static int kraus_norms(qvmhip_state *s, const cd *ops, uint32_t count, const uin
         a.ui[e] = (T)ops[e].imag();
     }
     const uint32_t grid = (uint32_t)std::min<uint64_t>((a.g.ngroups + kBlock - 1) / kBlock, kNormBlocks);
-    hipLaunchKernelGGL((k_kraus_norms<T, K>), dim3(grid), dim3(kBlock), 0, s->stream, (const vec2_t<T> *)s->amps, a,
-                       partials_of(s, (int)grid, C));
+    double *partial = partials_of(s, (int)grid, C);
+    if (stream_accesses(s))
+        hipLaunchKernelGGL((k_kraus_norms<T, K, C, true>), dim3(grid), dim3(kBlock), 0, s->stream,
+                           (const vec2_t<T> *)s->amps, a, partial);
+    else
+        hipLaunchKernelGGL((k_kraus_norms<T, K, C, false>), dim3(grid), dim3(kBlock), 0, s->stream,
+                           (const vec2_t<T> *)s->amps, a, partial);
     QH_LAUNCH_CHECK();
     return sums_to_host(s, (int)grid, C, out, (int)count);
+}
+
+template <typename T, int K>
+static int kraus_norms(qvmhip_state *s, const cd *ops, uint32_t count, const uint32_t *qubits, double *out) {
+    return count <= 2 ? kraus_norms_c<T, K, 2>(s, ops, count, qubits, out)
+                      : kraus_norms_c<T, K, kraus_per_read(K)>(s, ops, count, qubits, out);
 }
 
 int launch_kraus_choice(qvmhip_state *s, const double *K, uint32_t count, uint32_t k, const uint32_t *qubits, double r,

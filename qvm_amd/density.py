@@ -120,7 +120,7 @@ class DensityQVM:
                 ops = self._kraus_ops(ins)
             except Exception:
                 break
-            if not ops or not 0 <= q < self.number_of_qubits or any(K.shape != (2, 2) for K in ops):
+            if not ops or not 0 <= q < self.number_of_qubits or any(getattr(K, "shape", None) != (2, 2) for K in ops):
                 break
             maps.append((ops, q))
         if len(maps) < 2:

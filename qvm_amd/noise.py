@@ -161,7 +161,7 @@ class NoisyQVM(PureStateQVM):
     def run(self) -> "NoisyQVM":
         # without noisy gates every step is the pure machine's; a subclass that
         # handles instructions itself sees each of them
-        if (self.program is None or not self.noisy_gate_definitions
+        if (self.program is None or self._compiled is not None or not self.noisy_gate_definitions
                 or type(self).transition is not NoisyQVM.transition):
             return super().run()
         code = self.program.executable_code
@@ -195,7 +195,7 @@ class NoisyQVM(PureStateQVM):
                     ops = [Q.resolve_gate_matrix(ins, self.program.gate_definitions, self.memory)]
                 except Exception:
                     break  # its own transition reports it
-            if not ops or not 0 <= q < self.number_of_qubits or any(K.shape != (2, 2) for K in ops):
+            if not ops or not 0 <= q < self.number_of_qubits or any(getattr(K, "shape", None) != (2, 2) for K in ops):
                 break
             weights = [_unitary_weight(K) for K in ops]
             if None in weights or (not noisy and abs(weights[0] - 1) > 2.0 ** -49):
