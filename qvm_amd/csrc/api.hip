@@ -50,6 +50,10 @@ int check_qubits(const qvmhip_state *s, uint32_t k, const uint32_t *qubits) {
     return QVMHIP_OK;
 }
 
+// Whether s can hold the density matrix of nq qubits.  (2 * nq == n would let
+// an nq of 2^31 + n / 2 through, whose row bits nq + q lie far outside the state.)
+bool holds_density(const qvmhip_state *s, uint32_t nq) { return s->n % 2 == 0 && nq == s->n / 2; }
+
 bool finite_matrix(const double *U, uint32_t k) {
     const size_t n = size_t(2) << (2 * k);
     for (size_t i = 0; i < n; ++i)
@@ -250,7 +254,7 @@ int qvmhip_apply_fused(qvmhip_state *s, const double *U, uint32_t k, const uint3
 int qvmhip_density_apply_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, uint32_t k,
                                const uint32_t *qubits) {
     if (!s) return fail(QVMHIP_EINVAL, "null state");
-    if (2 * nq != s->n) return fail(QVMHIP_EINVAL, "a density state of nq qubits has 2*nq qubits");
+    if (!holds_density(s, nq)) return fail(QVMHIP_EINVAL, "a density state of nq qubits has 2*nq qubits");
     if (k < 1 || k > 3 || k > nq) return fail(QVMHIP_EINVAL, "Kraus operators act on 1..3 qubits of the density state");
     int rc = check_qubits(s, k, qubits);
     if (rc) return rc;
@@ -266,7 +270,7 @@ int qvmhip_density_apply_kraus(qvmhip_state *s, uint32_t nq, const double *K, ui
 int qvmhip_density_apply_kraus_run(qvmhip_state *s, uint32_t nq, uint32_t nmaps, const uint32_t *qubits,
                                    const uint32_t *counts, const double *K) {
     if (!s) return fail(QVMHIP_EINVAL, "null state");
-    if (2 * nq != s->n) return fail(QVMHIP_EINVAL, "a density state of nq qubits has 2*nq qubits");
+    if (!holds_density(s, nq)) return fail(QVMHIP_EINVAL, "a density state of nq qubits has 2*nq qubits");
     if (!qubits || !counts || !K) return fail(QVMHIP_EINVAL, "null argument");
     const double *k = K;
     const char *bad = nullptr;
@@ -632,7 +636,7 @@ int qvmhip_accumulate(qvmhip_state *dst, const qvmhip_state *src) {
 int qvmhip_density_diagonal(qvmhip_state *s, uint32_t nq, double *out) {
     if (!s || !out) return fail(QVMHIP_EINVAL, "null argument");
     DeviceScope ds(s->device);
-    if (2 * nq != s->n) return fail(QVMHIP_EINVAL, "a density state of nq qubits has 2*nq qubits");
+    if (!holds_density(s, nq)) return fail(QVMHIP_EINVAL, "a density state of nq qubits has 2*nq qubits");
     return density_diagonal(s, nq, out);
 }
 

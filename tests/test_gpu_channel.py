@@ -76,6 +76,22 @@ def test_density_apply_kraus_refuses():
                 st.density_apply_kraus(nq, K, q)
 
 
+def test_density_calls_refuse_a_qubit_count_that_wraps():
+    """Twice 2^31 + 3 is 6 in 32 bits: the row bits of that many qubits lie
+    outside a 6-qubit state."""
+    from qvm_amd import _native as N
+    from qvm_amd.state import HipPureState
+    nq, eye = 2 ** 31 + 3, np.eye(2)
+    out = np.zeros(8)
+    with HipPureState(6, "f64") as st:
+        for call in (lambda: st.density_apply_kraus(nq, eye[None], [0]),
+                     lambda: st.density_apply_kraus_run(nq, [([eye], 0), ([eye], 1)]),
+                     lambda: N.check(N.lib().qvmhip_density_diagonal(st.handle, nq, N.dptr(out)))):
+            with pytest.raises(N.QVMHipError):
+                call()
+        assert st.amplitudes()[0] == 1
+
+
 @pytest.mark.parametrize("dtype,n,k,count", [("f64", 1, 1, 2), ("f64", 2, 2, 3), ("f64", 3, 1, 9), ("f64", 9, 1, 4),
                                              ("f64", 9, 2, 5), ("f64", 13, 1, 5), ("f32", 9, 1, 4), ("f32", 9, 2, 3)])
 def test_kraus_choice(dtype, n, k, count):
