@@ -279,14 +279,17 @@ QVMHIP_API int qvmhip_accumulate(qvmhip_state *dst, const qvmhip_state *src);
  * the density matrix vec(rho) held row-major in a 2*nq-qubit state: the Kraus
  * loop of apply-gate-to-state on density states (src/apply-gate.lisp:66-99) as
  * one sweep with the map's superoperator.  K: `count` 2^k x 2^k matrices,
- * 1 <= k <= 3; count = 1 is a unitary gate (src/apply-gate.lisp:40-65). */
+ * 1 <= k <= 3; count = 1 is a unitary gate (src/apply-gate.lisp:40-65).
+ * QVMHIP_ERANGE, with the state unchanged, when an entry of the superoperator
+ * is past the range of the state's type. */
 QVMHIP_API int qvmhip_density_apply_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, uint32_t k,
                                           const uint32_t *qubits);
 /* A run of 1-qubit Kraus maps on the density state, in order: map i acts on
  * qubits[i] (< nq) with counts[i] operators; K holds all their 2x2 matrices one
  * after another.  The same as qvmhip_density_apply_kraus per map up to rounding
  * (maps on one qubit are multiplied together, maps on different qubits share
- * sweeps).  A map that is refused leaves the maps before it applied. */
+ * sweeps).  A map that is refused leaves the maps before it applied, except
+ * that a superoperator past the range (QVMHIP_ERANGE) refuses the whole run. */
 QVMHIP_API int qvmhip_density_apply_kraus_run(qvmhip_state *s, uint32_t nq, uint32_t nmaps, const uint32_t *qubits,
                                               const uint32_t *counts, const double *K);
 /* For a 2*nq-qubit state holding vec(rho) row-major (rho[i][j] at i*2^nq + j):

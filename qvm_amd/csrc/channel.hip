@@ -28,6 +28,7 @@
 #include <cmath>
 #include <complex>
 #include <cstring>
+#include <limits>
 #include <vector>
 
 #include "qvmhip_internal.h"
@@ -58,8 +59,20 @@ static std::vector<cd> superoperator(const cd *K, uint32_t count, uint32_t k) {
     return S;
 }
 
+// Whether the state's type holds every entry.  Finite Kraus entries can have
+// products past the range (1e25 twice in FP32), where the operators applied one
+// after another still give finite amplitudes.
+static bool in_range(const qvmhip_state *s, const std::vector<cd> &A) {
+    const double top = s->dtype == QVMHIP_F64 ? std::numeric_limits<double>::max() : std::numeric_limits<float>::max();
+    return std::all_of(A.begin(), A.end(),
+                       [&](const cd &z) { return std::abs(z.real()) <= top && std::abs(z.imag()) <= top; });
+}
+
+static int past_range() { return fail(QVMHIP_ERANGE, "the map's superoperator is past the range of the state's type"); }
+
 int launch_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, uint32_t k, const uint32_t *qubits) {
     const std::vector<cd> S = superoperator(reinterpret_cast<const cd *>(K), count, k);
+    if (!in_range(s, S)) return past_range();
     uint32_t q[6];
     for (uint32_t i = 0; i < k; ++i) {
         q[i] = qubits[i];
@@ -116,10 +129,11 @@ struct TileGroup {
 int launch_kraus_run(qvmhip_state *s, uint32_t nq, uint32_t nmaps, const uint32_t *qubits, const uint32_t *counts,
                      const double *K) {
     std::vector<std::vector<cd>> S(nq);
-    bool finite = true;
+    bool fits = true;
     const cd *k = reinterpret_cast<const cd *>(K);
     for (uint32_t i = 0; i < nmaps; k += 4 * (size_t)counts[i], ++i) {
         const std::vector<cd> A = superoperator(k, counts[i], 1);
+        if (!in_range(s, A)) return past_range();
         std::vector<cd> &B = S[qubits[i]];
         if (B.empty()) {
             B = A;
@@ -132,10 +146,10 @@ int launch_kraus_run(qvmhip_state *s, uint32_t nq, uint32_t nmaps, const uint32_
                     const cd a = A[4 * r + j], b = B[4 * j + c];
                     if (a != cd(0, 0) && b != cd(0, 0)) P[4 * r + c] += a * b;
                 }
-        for (const cd &x : P) finite = finite && std::isfinite(x.real()) && std::isfinite(x.imag());
+        fits = fits && in_range(s, P);
         B.swap(P);
     }
-    if (!finite) {  // a product past the range: map by map, as given
+    if (!fits) {  // a product past the range: map by map, as given
         k = reinterpret_cast<const cd *>(K);
         for (uint32_t i = 0; i < nmaps; k += 4 * (size_t)counts[i], ++i)
             if (const int rc = launch_kraus(s, nq, reinterpret_cast<const double *>(k), counts[i], 1, qubits + i))

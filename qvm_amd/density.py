@@ -36,6 +36,7 @@ from typing import Dict, List, Optional
 
 import numpy as np
 
+from . import _native as N
 from . import gates as G
 from . import quil as Q
 from .noise import check_kraus_ops, check_povm, perturb_measurement
@@ -125,7 +126,12 @@ class DensityQVM:
             maps.append((ops, q))
         if len(maps) < 2:
             return False
-        self.state.density_apply_kraus_run(self.number_of_qubits, maps)
+        try:
+            self.state.density_apply_kraus_run(self.number_of_qubits, maps)
+        except N.QVMHipError as e:
+            if e.code == N.ERANGE:  # nothing was applied: one by one
+                return False
+            raise
         self.pc += len(maps)
         return True
 
@@ -193,8 +199,12 @@ class DensityQVM:
         if 1 <= k <= (2 if len(ops) == 1 else 3):
             # one sweep with the map's superoperator.  A 3-qubit unitary stays
             # two sweeps: its 64x64 superoperator is bound by the matrix cores
-            self.state.density_apply_kraus(self.number_of_qubits, np.stack(ops), G.nat_tuple(*quil_qubits))
-            return
+            try:
+                self.state.density_apply_kraus(self.number_of_qubits, np.stack(ops), G.nat_tuple(*quil_qubits))
+                return
+            except N.QVMHipError as e:
+                if e.code != N.ERANGE:  # products past the range: operator by operator
+                    raise
         if len(ops) == 1:
             self._apply_single(ops[0], quil_qubits)
             return

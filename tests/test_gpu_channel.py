@@ -76,6 +76,43 @@ def test_density_apply_kraus_refuses():
                 st.density_apply_kraus(nq, K, q)
 
 
+@pytest.mark.parametrize("dtype,big,small", [("f64", 1e200, 1e-300), ("f32", 1e25, 1e-30)])
+def test_density_products_past_the_range(dtype, big, small):
+    """A finite operator whose products of two entries overflow, on a state
+    that stays finite under one operator after another: a single gate, a list, a
+    run of gates, and a run whose product overflows though no map does.  Bound:
+    the gates' products are single ones, rounded four times on the way."""
+    from qvm_amd._native import ERANGE, QVMHipError
+    from qvm_amd.density import DensityQVM
+    u = 2.0 ** (-53 if dtype == "f64" else -24)
+    rho = np.arange(1, 257).reshape(16, 16) * (1 + 0.5j) * small
+    A, mid = np.diag([big, -big]), np.diag([big ** 0.5, 1])
+    S = embed(A, [1], 4)
+    qvm = DensityQVM(4, dtype=dtype)
+    text = (f"DEFGATE A:\n    {big!r}, 0\n    0, {-big!r}\n\nDEFGATE B:\n    {big ** 0.5!r}, 0\n    0, 1\n\n"
+            f"DEFGATE C:\n    {big ** -0.6!r}, 0\n    0, 1\n\n")
+    for way in ("gate", "list", "A 1\nZ 0\n", "B 1\nB 1\nC 1\nZ 0\n"):
+        want = S @ rho @ S
+        qvm.state.write_amplitudes(rho.reshape(-1))
+        if way == "gate":
+            with pytest.raises(QVMHipError) as e:
+                qvm.state.density_apply_kraus(4, A[None], [1])
+            assert e.value.code == ERANGE
+            qvm.apply_superoperator([A], [1])
+        elif way == "list":
+            qvm.apply_superoperator([A, 0 * A], [1])
+        else:
+            want = rho
+            for ins in way.split("\n")[:-1]:
+                M = {"A": A, "B": mid, "C": np.diag([big ** -0.6, 1]), "Z": np.diag([1, -1])}[ins[0]]
+                F = embed(M, [int(ins[2])], 4)
+                want = F @ want @ F
+            qvm.load_program(text + way)
+            qvm.run()
+        assert np.max(np.abs(qvm.density_matrix() - want)) <= 16 * u * np.max(np.abs(want)), way
+    qvm.close()
+
+
 def test_density_calls_refuse_a_qubit_count_that_wraps():
     """Twice 2^31 + 3 is 6 in 32 bits: the row bits of that many qubits lie
     outside a 6-qubit state."""
