@@ -40,7 +40,7 @@ from . import _native as N
 from . import gates as G
 from . import quil as Q
 from .noise import check_kraus_ops, check_povm, perturb_measurement
-from .qvm import QVMError, _UniformStream, transition_classical
+from .qvm import QVMError, _UniformStream, method_chain, transition_classical
 from .state import HipPureState
 
 
@@ -97,9 +97,8 @@ class DensityQVM:
             raise QVMError("no program loaded")
         code = self.program.executable_code
         self.pc = 0
-        # a subclass that handles instructions or maps itself sees each of them
-        fuse = (type(self).transition is DensityQVM.transition and type(self)._kraus_ops is DensityQVM._kraus_ops
-                and type(self).apply_superoperator is DensityQVM.apply_superoperator)
+        # code that handles instructions or maps itself sees each of them
+        fuse = all(method_chain(self, name) == own for name, own in _PER_GATE.items())
         while self.pc is not None and self.pc < len(code):
             if fuse and self._run_maps(code):
                 continue
@@ -278,6 +277,10 @@ class DensityQVM:
                 s.close()
         self._pristine = self._sum = None
         self.state.close()
+
+
+_PER_GATE = {name: method_chain(DensityQVM, name)
+             for name in ("transition", "_kraus_ops", "apply_superoperator", "_apply_single")}
 
 
 def make_density_qvm(num_qubits: int, **kw) -> DensityQVM:

@@ -25,7 +25,7 @@ import numpy as np
 
 from . import gates as G
 from . import quil as Q
-from .qvm import PureStateQVM, QVMError, apply_gate_to_state
+from .qvm import PureStateQVM, QVMError, apply_gate_to_state, method_chain
 from .state import HipPureState
 
 
@@ -159,10 +159,10 @@ class NoisyQVM(PureStateQVM):
         self.readout_povms[int(qubit)] = tuple(float(x) for x in povm)
 
     def run(self) -> "NoisyQVM":
-        # without noisy gates every step is the pure machine's; a subclass that
-        # handles instructions itself sees each of them
+        # without noisy gates every step is the pure machine's; code that handles
+        # instructions itself sees each of them
         if (self.program is None or self._compiled is not None or not self.noisy_gate_definitions
-                or type(self).transition is not NoisyQVM.transition):
+                or method_chain(self, "transition") != _TRANSITIONS):
             return super().run()
         code = self.program.executable_code
         self.pc = 0
@@ -267,3 +267,6 @@ class NoisyQVM(PureStateQVM):
             self._trial.close()
             self._trial = None
         super().close()
+
+
+_TRANSITIONS = method_chain(NoisyQVM, "transition")

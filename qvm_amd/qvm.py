@@ -173,6 +173,17 @@ class _UniformStream:
         return float(self._g.random())
 
 
+def method_chain(machine, name: str) -> list:
+    """Every definition of a method that a call on the machine (an instance
+    or a class) can reach, super() calls included, outermost first.  A machine
+    that applies several instructions at once compares the chain with its own:
+    an override in a subclass, a function set on the instance or a wrapper put on
+    a class shows as another chain, and then sees each instruction."""
+    own = [] if isinstance(machine, type) else [vars(machine)[name]] if name in vars(machine) else []
+    cls = machine if isinstance(machine, type) else type(machine)
+    return own + [vars(c)[name] for c in cls.__mro__ if name in vars(c)]
+
+
 class PureStateQVM:
     """pure-state-qvm (src/qvm.lisp:106-148) with an HBM-resident state."""
 

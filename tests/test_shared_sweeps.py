@@ -1,0 +1,97 @@
+"""The interpreters' shared sweeps (several instructions as one engine call)
+on a stand-in for the engine state: who still sees each instruction, and what a
+failure in the middle leaves behind."""
+import numpy as np
+import pytest
+
+from qvm_amd import density, gates as G, noise, qvm
+
+
+class StandIn:
+    """Records the engine calls of a machine."""
+
+    def __init__(self, num_qubits, dtype="f64", **kw):
+        self.num_qubits, self.dtype, self.calls = num_qubits, dtype, []
+
+    def total_probability(self):
+        return 1.0
+
+    def apply_1q_run(self, mats, qubits, normalize=False):
+        self.calls.append(("run", len(mats)))
+
+    def density_apply_kraus_run(self, nq, maps):
+        self.calls.append(("run", len(maps)))
+
+    def apply_matrix(self, U, qubits):
+        self.calls.append(("gate", 1))
+
+    def apply_kraus_choice(self, kraus_ops, qubits, r):
+        self.calls.append(("choice", 1))
+        return 0
+
+    def density_apply_kraus(self, nq, kraus_ops, qubits):
+        self.calls.append(("map", 1))
+
+    def close(self):
+        pass
+
+
+MIX = [np.sqrt(0.75) * G.gate_matrix("X"), 0.5 * G.gate_matrix("Z") @ G.gate_matrix("X")]
+TEXT = "X 0\nH 1\nX 0\nCNOT 0 1\nH 0\nX 0\n"
+
+
+@pytest.fixture
+def machine(monkeypatch):
+    for module in (qvm, noise, density):
+        monkeypatch.setattr(module, "HipPureState", StandIn)
+
+    def make(cls, rng=lambda: 0.1, text=TEXT):
+        m = cls(2, noisy_gate_definitions={("X", (0,)): MIX}, rng=rng)
+        m.load_program(text)
+        return m
+    return make
+
+
+@pytest.mark.parametrize("base", [noise.NoisyQVM, density.DensityQVM])
+def test_machines_without_hooks_share_sweeps(machine, base):
+    m = machine(base)
+    m.run()
+    assert [c for c in m.state.calls if c[0] == "run"] == [("run", 3), ("run", 2)] and m.pc == 6
+
+
+@pytest.mark.parametrize("base", [noise.NoisyQVM, density.DensityQVM])
+@pytest.mark.parametrize("way", ["subclass", "instance", "wrapped class", "wrapped base", "mixin"])
+def test_every_instruction_reaches_a_hook(machine, monkeypatch, base, way):
+    seen = []
+    own = qvm.PureStateQVM if base is noise.NoisyQVM and way in ("wrapped base", "mixin") else base
+    plain = own.transition
+
+    def hook(self, ins):
+        seen.append(ins)
+        return plain(self, ins)
+
+    cls = base
+    if way == "subclass":
+        cls = type("Sub", (base,), {"transition": hook})
+    elif way == "mixin":
+        if base is density.DensityQVM:
+            pytest.skip("no base class to mix in behind")
+        cls = type("Mixed", (base, type("Tracer", (qvm.PureStateQVM,), {"transition": hook})), {})
+    m = machine(cls)
+    if way == "instance":
+        m.transition = hook.__get__(m)
+    elif way.startswith("wrapped"):
+        monkeypatch.setattr(own, "transition", hook)
+    m.run()
+    # the pure machine's transition sees what the noisy one passes on
+    assert len(seen) == (3 if own is qvm.PureStateQVM else 6)
+    assert not [c for c in m.state.calls if c[0] == "run"]
+
+
+@pytest.mark.parametrize("name", ["_kraus_ops", "apply_superoperator"])
+def test_every_map_reaches_a_hook(machine, monkeypatch, name):
+    seen = []
+    plain = getattr(density.DensityQVM, name)
+    monkeypatch.setattr(density.DensityQVM, name, lambda self, *a: seen.append(a) or plain(self, *a))
+    machine(density.DensityQVM).run()
+    assert len(seen) == 6
