@@ -177,8 +177,9 @@ class NoisyQVM(PureStateQVM):
         sqrt(c_j) times a unitary, such as a Pauli channel after a gate), and
         advance pc.  |K_j psi|^2 is then c_j |psi|^2 whatever the state, so the
         choices need one read of the norm instead of one read per gate (24 qubits:
-        47 us, and 73 us for the gate chosen).  False, with nothing done and
-        no draw taken, when fewer than two follow each other."""
+        47 us, and 73 us for the gate chosen).  The draws are taken in the
+        program's order, before any of the run's gates is applied.  False, with
+        nothing done and no draw taken, when fewer than two follow each other."""
         run = []
         for i in range(self.pc, len(code)):
             ins = code[i]
@@ -204,25 +205,29 @@ class NoisyQVM(PureStateQVM):
         if len(run) < 2:
             return False
         norm2 = 1.0
-        normalize = any(w is not None for _, w, _ in run)
-        if normalize:
+        if any(w is not None for _, w, _ in run):
             norm2 = self.state.total_probability()
             if not 0.0 < norm2 < float("inf"):
                 return False
         mats = []
-        for ops, weights, q in run:
-            if weights is None:
-                mats.append(ops[0])
-                continue
-            r, summed = self._draw(), 0.0
-            for K, c in zip(ops, weights):
-                summed += c * norm2
-                if summed >= r:
-                    break
-            mats.append(K / np.sqrt(c))
-            norm2 = 1.0  # each noisy gate leaves a normalized state; the factor goes in at the end
-        self.state.apply_1q_run(mats, [q for _, _, q in run], normalize)
-        self.pc += len(run)
+        try:
+            for ops, weights, q in run:
+                if weights is None:
+                    mats.append(ops[0])
+                    continue
+                r, summed = self._draw(), 0.0
+                for K, c in zip(ops, weights):
+                    summed += c * norm2
+                    if summed >= r:
+                        break
+                mats.append(K / np.sqrt(c))
+                norm2 = 1.0  # each noisy gate leaves a normalized state; the factor goes in at the end
+        finally:
+            # a draw that raises leaves the gates before its own applied
+            done = run[:len(mats)]
+            if done:
+                self.state.apply_1q_run(mats, [q for _, _, q in done], any(w is not None for _, w, _ in done))
+                self.pc += len(done)
         return True
 
     def transition(self, ins):

@@ -18,6 +18,7 @@ class StandIn:
 
     def apply_1q_run(self, mats, qubits, normalize=False):
         self.calls.append(("run", len(mats)))
+        self.normalized = normalize
 
     def density_apply_kraus_run(self, nq, maps):
         self.calls.append(("run", len(maps)))
@@ -95,3 +96,15 @@ def test_every_map_reaches_a_hook(machine, monkeypatch, name):
     monkeypatch.setattr(density.DensityQVM, name, lambda self, *a: seen.append(a) or plain(self, *a))
     machine(density.DensityQVM).run()
     assert len(seen) == 6
+
+
+@pytest.mark.parametrize("good,pc,normalized", [(0, 1, False), (1, 3, True), (2, 5, True)])
+def test_a_draw_that_raises_leaves_the_gates_before_it_applied(machine, good, pc, normalized):
+    """H 0, X 0 (noisy), H 1, X 0 (noisy), H 1, X 0 (noisy): the draw of the
+    gate at pc raises."""
+    draws = iter([0.1] * good)
+    m = machine(noise.NoisyQVM, rng=lambda: next(draws), text="H 0\nX 0\nH 1\nX 0\nH 1\nX 0\n")
+    with pytest.raises(StopIteration):
+        m.run()
+    assert m.pc == pc and m.draws_used == good + 1
+    assert m.state.calls == [("run", pc)] and m.state.normalized == normalized
