@@ -130,6 +130,8 @@ class DensityQVM:
         except N.QVMHipError as e:
             if e.code == N.ERANGE:  # nothing was applied: one by one
                 return False
+            # a map that is not finite: the maps before it were applied
+            self.pc += next((i for i, (ops, _) in enumerate(maps) if not np.all(np.isfinite(ops))), 0)
             raise
         self.pc += len(maps)
         return True

@@ -104,3 +104,19 @@ def test_measure_collapse_and_measure_all():
     assert bits[0] == bit and bits[2] == bit  # collapsed qubit 0, and qubit 2 = qubit 0 (CNOT)
     assert q.draws_used <= 4
     q.close()
+
+
+@pytest.mark.parametrize("before", ["", "X 0\n", "X 0\nX 1\nH 2\n"])
+def test_a_gate_that_is_not_finite_stops_at_its_own_instruction(before):
+    """A gate whose angle is not a number is refused with pc on it and the
+    gates before it applied, alone, after one gate and after a run."""
+    from qvm_amd._native import QVMHipError
+    from qvm_amd.density import DensityQVM
+    q = DensityQVM(4)
+    q.load_program("DECLARE t REAL[1]\n" + before + "RX(t[0]) 3\nX 2\n")
+    q.memory["t"][0] = np.nan
+    with pytest.raises(QVMHipError):
+        q.run()
+    assert q.program.executable_code[q.pc].name == "RX"
+    assert (q.excited_probability(0) > 0.5) == bool(before)  # X 0 was applied
+    q.close()
