@@ -97,9 +97,14 @@ def evolve_pure_state_stochastically(state: HipPureState, trial: HipPureState, k
     2 qubits read the state once for the p_j and apply the chosen operator in
     place; wider ones set the trial buffer to each K_j psi in turn.  Returns
     the index j chosen."""
-    if 1 <= len(quil_qubits) <= 2 and len(kraus_ops):
-        ops = np.stack([np.asarray(k, dtype=np.complex128) for k in kraus_ops])
-        return state.apply_kraus_choice(ops, G.nat_tuple(*quil_qubits), r)
+    quil_qubits = list(quil_qubits)
+    D = 1 << len(quil_qubits)
+    if 2 <= D <= 4:
+        kraus_ops = list(kraus_ops)
+        ops = [np.asarray(K, dtype=np.complex128) for K in kraus_ops if np.shape(K) == (D, D)]
+        # one that does not fit the qubits is refused below, when its turn comes
+        if ops and len(ops) == len(kraus_ops):
+            return state.apply_kraus_choice(np.stack(ops), G.nat_tuple(*quil_qubits), r)
     summed = 0.0
     chosen = -1
     for j, K in enumerate(kraus_ops):

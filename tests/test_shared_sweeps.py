@@ -33,6 +33,15 @@ class StandIn:
     def density_apply_kraus(self, nq, kraus_ops, qubits):
         self.calls.append(("map", 1))
 
+    def copy_from(self, other):
+        pass
+
+    def swap_contents(self, other):
+        self.calls += other.calls
+
+    def normalize(self):
+        pass
+
     def close(self):
         pass
 
@@ -108,3 +117,14 @@ def test_a_draw_that_raises_leaves_the_gates_before_it_applied(machine, good, pc
         m.run()
     assert m.pc == pc and m.draws_used == good + 1
     assert m.state.calls == [("run", pc)] and m.state.normalized == normalized
+
+
+def test_kraus_evolution_takes_any_iterable():
+    """Operators and qubits as generators; an operator of another size behind
+    the chosen one is never reached."""
+    one, two = MIX, [np.kron(K, np.eye(2)) for K in MIX]
+    for ops, qubits, call in ((one, [0], "choice"), (two, [1, 0], "choice"), ([one[0], np.eye(4)], [0], "gate"),
+                              ([np.eye(8)], [0, 1, 2], "gate")):
+        st = StandIn(3)
+        assert noise.evolve_pure_state_stochastically(st, StandIn(3), (K for K in ops), (q for q in qubits), 0.5) == 0
+        assert st.calls == [(call, 1)]
