@@ -134,14 +134,23 @@ __global__ __launch_bounds__(kBlock) void k_prob_partial(const vec2_t<T> *__rest
 // sum over edges of <Z_a Z_b>: weight(i) = nedges - 2 * #cut edges.  The
 // amplitudes are taken 2^11 at a time; the edges come ordered by where their
 // ends lie: both below bit 11 (ll; a constant of the thread's amplitude), one
-// below (cr), both above (hh; a constant of the chunk).  The cross edges of
-// an amplitude are popcount(A(low bits) ^ B(chunk)), one bit per edge, so an
-// amplitude costs a handful of instructions instead of five per edge (30
-// qubits, ring of 30 edges, FP32: 4.4 ms of instruction issue for a 1.2 ms read).
-constexpr int kZZBits = 11;
+// below (cr), both above (hh; a constant of the chunk).  Of the cross edges with
+// low end x, d of them, s have their upper bit set in the chunk (a population
+// count of chunk bits): they cut s where bit x of an amplitude is 0 and d - s where
+// it is 1, so an amplitude costs a handful of instructions however many edges
+// there are.  Bound by the read.  28 qubits FP64, a ring / 80 / 256 random edges:
+// 0.63 ms (6.8 TB/s); edge by edge, five instructions per amplitude and edge,
+// 1.02 / 2.31 / 6.8 ms.  22 qubits, 80 edges: 32 us against 60, FP32 30 against 59.
+constexpr int kZZBits = 11, kZZGroup = 8;
 struct ZZArgs {
-    uint32_t nll, ncr, nhh, fast;  // fast: at most 32 cross edges
-    uint8_t lo[256], hi[256];      // ends of edge e, lo[e] <= hi[e]
+    uint32_t nll, nhh, planes;
+    int ne;                         // edges in all
+    int d[kZZBits];                 // cr edges with low end x
+    // their upper ends less 11, as masks: an edge given m times is in the planes
+    // of the bits of m
+    uint32_t upper[9][kZZBits];
+    uint16_t ll[256];               // ends lo | hi << 8, in groups of kZZGroup filled up with (0, 0), which nothing cuts
+    uint16_t hh[256];               // ends less 11, as in ll
 };
 
 template <typename T, bool NTM>
@@ -154,39 +163,30 @@ __global__ __launch_bounds__(kBlock) void k_zz_partial(const vec2_t<T> *__restri
     const uint64_t nchunk = (len + (1u << kZZBits) - 1) >> kZZBits;
     const uint32_t b = xcd_block(blockIdx.x, gridDim.x);
     const uint64_t per = nchunk / gridDim.x;
-    const uint32_t ne = a.nll + a.ncr + a.nhh;
-    // low bits of the thread's amplitude k (bit 0 is the place in an FP32 pair)
-    auto low = [&](int k) { return (uint32_t)H * (threadIdx.x + (uint32_t)(k / H) * kBlock) + (uint32_t)(k % H); };
+    // low bits of the thread's amplitude k: thread bits, and bits of k (bit 0
+    // is the place in an FP32 pair)
+    const uint32_t tlow = (uint32_t)H * threadIdx.x;
+    auto klow = [](int k) { return (uint32_t)(H * (k / H) * kBlock + k % H); };
     int win[U * H];
-    uint32_t A[U * H];
 #pragma unroll
-    for (int k = 0; k < U * H; ++k) {
-        win[k] = 0;
-        A[k] = 0;
+    for (int k = 0; k < U * H; ++k) win[k] = 0;
+    for (uint32_t e = 0; e < a.nll; e += kZZGroup) {
+#pragma unroll
+        for (int i = 0; i < kZZGroup; ++i) {
+            const uint32_t w = reinterpret_cast<const uint32_t *>(a.ll)[(e + i) / 2] >> (i % 2 ? 16 : 0);
+            const uint32_t x = w & 31u, y = (w >> 8) & 31u, t = ((tlow >> x) ^ (tlow >> y)) & 1u;
+#pragma unroll
+            for (int k = 0; k < U * H; ++k) win[k] += (int)(t ^ (((klow(k) >> x) ^ (klow(k) >> y)) & 1u));
+        }
     }
-    // lane l looks after edge l of the upper classes (and l + 64, ...): their
-    // bits of a chunk are one ballot
-    const uint32_t lane = threadIdx.x % kWave;
-    uint32_t cr_hi = 63, hh_lo[4], hh_hi[4];
-    if (a.fast) {
-        for (uint32_t e = 0; e < a.nll; ++e) {
-            const uint32_t x = a.lo[e], y = a.hi[e];
+    // lane l looks after edges l, l + 64, ... of hh: their bits of a chunk are
+    // one ballot
+    uint32_t hh_lo[4], hh_hi[4];
 #pragma unroll
-            for (int k = 0; k < U * H; ++k) win[k] += (int)(((low(k) >> x) ^ (low(k) >> y)) & 1u);
-        }
-        for (uint32_t e = 0; e < a.ncr; ++e) {
-            const uint32_t x = a.lo[a.nll + e];
-#pragma unroll
-            for (int k = 0; k < U * H; ++k) A[k] |= ((low(k) >> x) & 1u) << e;
-        }
-        if (lane < a.ncr) cr_hi = a.hi[a.nll + lane] - kZZBits;
-#pragma unroll
-        for (uint32_t r = 0; r < 4; ++r) {
-            const uint32_t e = lane + r * kWave;
-            const bool on = e < a.nhh;
-            hh_lo[r] = on ? a.lo[a.nll + a.ncr + e] - kZZBits : 63u;
-            hh_hi[r] = on ? a.hi[a.nll + a.ncr + e] - kZZBits : 63u;
-        }
+    for (uint32_t r = 0; r < 4; ++r) {
+        const uint32_t e = threadIdx.x % kWave + r * kWave;
+        hh_lo[r] = e < a.nhh ? a.hh[e] & 0xFFu : 63u;
+        hh_hi[r] = e < a.nhh ? a.hh[e] >> 8 : 63u;
     }
     double acc = 0.0;
     for (uint64_t c = per * b; c < per * (b + 1); ++c) {
@@ -196,23 +196,29 @@ __global__ __launch_bounds__(kBlock) void k_zz_partial(const vec2_t<T> *__restri
             const uint64_t e = ((c << kZZBits) / H) + threadIdx.x + (uint64_t)u * kBlock;
             v[u] = load_elem<T, NTM>(psi, e < len / H ? e : 0);
         }
-        uint32_t B = 0;
-        int hh = 0;
-        if (a.fast) {
-            B = (uint32_t)__ballot((c >> cr_hi) & 1u);
+        // cut: edges that every amplitude of the thread cuts, whatever its k
+        int set[kZZBits], cut = 0;
 #pragma unroll
-            for (uint32_t r = 0; r < 4; ++r)
-                if (r * kWave < a.nhh) hh += __popcll(__ballot(((c >> hh_lo[r]) ^ (c >> hh_hi[r])) & 1u));
-        }
+        for (int x = 0; x < kZZBits; ++x) set[x] = __popc((uint32_t)c & a.upper[0][x]);
+        for (uint32_t p = 1; p < a.planes; ++p)
+#pragma unroll
+            for (int x = 0; x < kZZBits; ++x) set[x] += __popc((uint32_t)c & a.upper[p][x]) << p;
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r)
+            if (r * kWave < a.nhh) cut += __popcll(__ballot(((c >> hh_lo[r]) ^ (c >> hh_hi[r])) & 1u));
+#pragma unroll
+        for (int x = 0; x < kZZBits; ++x) cut += set[x];
+#pragma unroll
+        for (int x = 0; x < kZZBits; ++x) cut += __mul24((int)((tlow >> x) & 1u), a.d[x] - 2 * set[x]);
 #pragma unroll
         for (int k = 0; k < U * H; ++k) {
-            const uint64_t x = (c << kZZBits) + (uint64_t)H * (threadIdx.x + (uint64_t)(k / H) * kBlock) + (k % H);
-            int cut = win[k] + hh + __popc(A[k] ^ B);
-            if (!a.fast) {
-                cut = 0;
-                for (uint32_t e = 0; e < ne; ++e) cut += (int)(((x >> a.lo[e]) ^ (x >> a.hi[e])) & 1u);
-            }
-            if (x < len) acc += Elem<T>::p(v[k / H], k % H) * (double)((int)ne - 2 * cut);
+            const uint64_t x = (c << kZZBits) + tlow + klow(k);
+            int n = 0;
+#pragma unroll
+            for (int y = 0; y < kZZBits; ++y)
+                if ((klow(k) >> y) & 1u) n += a.d[y] - 2 * set[y];
+            n += win[k] + cut;
+            if (x < len) acc += Elem<T>::p(v[k / H], k % H) * (double)(a.ne - 2 * n);
         }
     }
     const double t = block_sum(acc, sm);
@@ -1059,18 +1065,24 @@ int expectation_zz(qvmhip_state *s, const uint32_t *edges, uint32_t nedges, doub
     // the edges travel with the launch, ordered ll, cr, hh (see k_zz_partial)
     ZZArgs a;
     std::memset(&a, 0, sizeof(a));
-    uint32_t at = 0;
-    for (int cls = 0; cls < 3; ++cls) {
-        const uint32_t from = at;
-        for (uint32_t e = 0; e < nedges; ++e) {
-            const uint32_t lo = std::min(edges[2 * e], edges[2 * e + 1]), hi = std::max(edges[2 * e], edges[2 * e + 1]);
-            if ((hi < (uint32_t)kZZBits ? 0 : lo < (uint32_t)kZZBits ? 1 : 2) != cls) continue;
-            a.lo[at] = (uint8_t)lo;
-            a.hi[at++] = (uint8_t)hi;
+    a.ne = (int)nedges;
+    a.planes = 1;
+    for (uint32_t e = 0; e < nedges; ++e) {
+        const uint32_t lo = std::min(edges[2 * e], edges[2 * e + 1]), hi = std::max(edges[2 * e], edges[2 * e + 1]);
+        if (hi < (uint32_t)kZZBits) {
+            a.ll[a.nll++] = (uint16_t)(lo | hi << 8);
+        } else if (lo >= (uint32_t)kZZBits) {
+            a.hh[a.nhh++] = (uint16_t)((lo - kZZBits) | (hi - kZZBits) << 8);
+        } else {
+            ++a.d[lo];
+            // one more of this edge: add with carry over the planes
+            const uint32_t bit = 1u << (hi - kZZBits);
+            uint32_t p = 0;
+            for (; a.upper[p][lo] & bit; ++p) a.upper[p][lo] ^= bit;
+            a.upper[p][lo] |= bit;
+            a.planes = std::max(a.planes, p + 1);
         }
-        (cls == 0 ? a.nll : cls == 1 ? a.ncr : a.nhh) = at - from;
     }
-    a.fast = a.ncr <= 32 ? 1u : 0u;
     const uint64_t nchunk = (s->len + (1u << kZZBits) - 1) >> kZZBits;
     const uint32_t grid = (uint32_t)std::min<uint64_t>(nchunk, kRedBlocks);  // powers of two
     double *partial = partials_of(s, (int)grid, 1);

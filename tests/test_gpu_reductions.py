@@ -57,6 +57,29 @@ def test_expectation_zz(dtype, n, nedges):
 
 
 @pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("n", [11, 12, 14, 22, 24])
+def test_expectation_zz_of_basis_states(dtype, n):
+    """Every edge is +1 or -1 on a basis state, so the sum is exact: dense edge
+    lists across bit 11, one edge up to 256 times, states of several chunks per
+    workgroup."""
+    from qvm_amd import gates as G
+    from qvm_amd.state import HipPureState
+    rng = np.random.default_rng(n)
+    lists = [rng.integers(0, n, size=(256, 2)), np.array([(i % min(n, 11), n - 1 - i % (n - 10)) for i in range(200)])]
+    lists += [np.repeat([[3, n - 1]], m, axis=0) for m in (2, 7, 255, 256)]
+    lists.append(np.repeat([[0, n - 1], [n - 1, 2], [n - 2, n - 1]], [5, 130, 64], axis=0))
+    with HipPureState(n, dtype) as st:
+        for _ in range(12):
+            bits = rng.integers(0, 2, size=n)
+            st.reset_zero()
+            for q in np.flatnonzero(bits):
+                st.apply_matrix(G.gate_matrix("X"), [int(q)])
+            z = 1 - 2 * bits
+            for edges in lists:
+                assert st.expectation_zz(edges) == np.sum(z[edges[:, 0]] * z[edges[:, 1]])
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
 @pytest.mark.parametrize("n", [1, 2, 7, 9, 12])
 def test_collapse_bit_exact(dtype, n):
     """Both forms, every qubit: the kept half times the rounded factor, zeros
