@@ -341,7 +341,7 @@ class CostModel:
         cands = candidates or candidate_plans(gates, n, dtype)
         costs = {name: self.plan_cost(plan, n, dtype) for name, plan in cands.items()}
         best = min(costs, key=costs.get)
-        fixed = fixed_rule_name(dtype)
+        fixed = fixed_rule_name(dtype, n)
         if fixed in costs and costs[best] > (1.0 - self.MARGIN) * costs[fixed]:
             best = fixed
         return best, cands[best], costs
@@ -371,23 +371,26 @@ class CostModel:
         return cm
 
 
-def fixed_rule_name(dtype: str) -> str:
-    """The candidate the planner's "tiled" mode runs without a model."""
-    return f"tiled_m{P.default_tile_m(dtype)}_l{P.default_low(dtype)}"
+def fixed_rule_name(dtype: str, n: int | None = None) -> str:
+    """The candidate the planner's "tiled" mode runs without a model on n
+    qubits (without n: on a large state)."""
+    m = P.default_tile_m(dtype, n)
+    return f"tiled_m{m if n is None else min(m, n)}_l{P.default_low(dtype)}"
 
 
 def candidate_plans(gates, n: int, dtype: str) -> Dict[str, List["P.PlanItem"]]:
-    """plain; fused_k2..6; tiled_m{m}_l{low} for three tile widths and three
-    low runs (the qubit permutation into the block: the default run of one
-    128 B line and two longer ones); hybrid_m{m}: the default tile passes with
-    the gates on more than two qubits as MFMA blocks."""
+    """plain; fused_k2..6; tiled_m{m}_l{low} for three tile widths, and on
+    small states the narrow default width, each with three low runs (the qubit
+    permutation into the block: the default run of one 128 B line and two longer
+    ones); hybrid_m{m}: the tile passes of large states with the gates on more
+    than two qubits as MFMA blocks."""
     cands = {"plain": P.plan_plain(gates, n)}
     for k in (2, 3, 4, 5, 6):
         if k <= n:
             cands[f"fused_k{k}"] = P.plan_fused(gates, n, k)
     if n >= 10:
         m0, l0 = P.default_tile_m(dtype), P.default_low(dtype)
-        for m in (m0 - 1, m0, m0 + 1):
+        for m in sorted({m0 - 1, m0, m0 + 1, min(P.default_tile_m(dtype, n), n)}):
             if m > min(n, P.max_tile_m(dtype)):
                 continue
             for low in (l0, l0 + 1, l0 + 2):
@@ -430,7 +433,7 @@ def evaluate_planners(workload, learned: "CostModel", analytic: "AnalyticModel |
         t_plan = time.perf_counter() - t0
         pick = {"learned": learned.choose(gates, n, dtype, cands)[0],
                 "analytic": analytic.choose(gates, n, dtype, cands)[0],
-                "fixed_rule": fixed_rule_name(dtype)}
+                "fixed_rule": fixed_rule_name(dtype, n)}
         ref = HipPureState(n, dtype, fma_tiles=True)
         st = HipPureState(n, dtype, fma_tiles=True)
         P.execute_plan(ref, cands["plain"])

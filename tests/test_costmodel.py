@@ -53,6 +53,19 @@ def test_launch_features_and_candidates():
                 assert CM.low_run(it.qubits) >= L
 
 
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+@pytest.mark.parametrize("n", [10, 11, 12, 15, 17, 18, 19, 24])
+def test_fixed_rule_is_the_plan_of_tiled_mode(dtype, n, monkeypatch):
+    """The rule's candidate exists and is what compile_gates(mode="tiled")
+    runs, on small states too, where its tiles are narrower."""
+    from types import SimpleNamespace
+    gates = CI.layered(n, 2, seed=n)
+    monkeypatch.setattr(P, "build_program", lambda state, plan, use_graph=True: None)
+    own = P.compile_gates(SimpleNamespace(num_qubits=n, dtype=dtype), gates, mode="tiled", merge_1q=True).plan
+    cand = CM.candidate_plans(gates, n, dtype)[CM.fixed_rule_name(dtype, n)]
+    assert [(it.kind, it.qubits, it.gates) for it in own] == [(it.kind, it.qubits, it.gates) for it in cand]
+
+
 def test_hybrid_plan_runs_wide_gates_on_the_matrix_cores():
     n = 14
     gates = CI.dense_blocks(n, 2, 5, seed=3)
