@@ -95,8 +95,8 @@ def evolve_pure_state_stochastically(state: HipPureState, trial: HipPureState, k
     sampling with the draw r: p_j = |K_j psi|^2 is added to a running sum until
     the sum reaches r; K_j psi, renormalised, becomes the state.  Maps on 1 or
     2 qubits read the state once for the p_j and apply the chosen operator in
-    place; wider ones set the trial buffer to each K_j psi in turn.  Returns
-    the index j chosen."""
+    place; wider ones set the trial buffer (a state of the same size, or a
+    function that gives one) to each K_j psi in turn.  Returns the index j chosen."""
     quil_qubits = list(quil_qubits)
     D = 1 << len(quil_qubits)
     if 2 <= D <= 4:
@@ -105,6 +105,8 @@ def evolve_pure_state_stochastically(state: HipPureState, trial: HipPureState, k
         # one that does not fit the qubits is refused below, when its turn comes
         if ops and len(ops) == len(kraus_ops):
             return state.apply_kraus_choice(np.stack(ops), G.nat_tuple(*quil_qubits), r)
+    if callable(trial):
+        trial = trial()
     summed = 0.0
     chosen = -1
     for j, K in enumerate(kraus_ops):
@@ -148,7 +150,8 @@ class NoisyQVM(PureStateQVM):
             self.set_readout_povm(q, povm)
 
     def _trial_state(self) -> HipPureState:
-        # check-allocate-computation-space: the trial buffer is made on first need
+        # check-allocate-computation-space: the trial buffer is made on first need,
+        # which maps on 1 and 2 qubits do not have (16 GiB at 30 qubits)
         if self._trial is None:
             self._trial = HipPureState(self.number_of_qubits, dtype=self.state.dtype)
         return self._trial
@@ -156,7 +159,6 @@ class NoisyQVM(PureStateQVM):
     def set_noisy_gate(self, gate_name: str, qubits, kraus_ops) -> None:
         ops = [np.asarray(k, dtype=np.complex128) for k in kraus_ops]
         check_kraus_ops(ops)
-        self._trial_state()
         self.noisy_gate_definitions[(gate_name.upper(), tuple(int(q) for q in qubits))] = ops
 
     def set_readout_povm(self, qubit: int, povm) -> None:
@@ -246,7 +248,7 @@ class NoisyQVM(PureStateQVM):
                     raise QVMError("noisy gate definitions apply to static gates only")
                 if ops[0].shape[0] != 1 << len(ins.qubits):
                     raise QVMError(f"Kraus operators of {ins.name} do not match its qubit count")
-                evolve_pure_state_stochastically(self.state, self._trial_state(), ops, ins.qubits, self._draw())
+                evolve_pure_state_stochastically(self.state, self._trial_state, ops, ins.qubits, self._draw())
                 return self.pc + 1
             return super().transition(ins)
         if isinstance(ins, Q.Measure):

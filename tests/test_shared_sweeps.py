@@ -9,8 +9,10 @@ from qvm_amd import density, gates as G, noise, qvm
 
 class StandIn:
     """Records the engine calls of a machine."""
+    made = 0
 
     def __init__(self, num_qubits, dtype="f64", **kw):
+        StandIn.made += 1
         self.num_qubits, self.dtype, self.calls = num_qubits, dtype, []
 
     def total_probability(self):
@@ -128,3 +130,19 @@ def test_kraus_evolution_takes_any_iterable():
         st = StandIn(3)
         assert noise.evolve_pure_state_stochastically(st, StandIn(3), (K for K in ops), (q for q in qubits), 0.5) == 0
         assert st.calls == [(call, 1)]
+
+
+def test_the_second_statevector_is_made_for_wide_maps_only(machine):
+    """Noisy gates on 1 and 2 qubits, alone and in runs, work in place; the
+    first one on 3 qubits makes the trial buffer, the next one finds it."""
+    StandIn.made = 0
+    m = machine(noise.NoisyQVM)
+    m.set_noisy_gate("CNOT", [0, 1], [G.gate_matrix("CNOT")])
+    m.run()
+    assert ("choice", 1) in m.state.calls and StandIn.made == 1
+    wide = noise.NoisyQVM(3, noisy_gate_definitions={("CCNOT", (0, 1, 2)): [G.gate_matrix("CCNOT")]})
+    assert StandIn.made == 2
+    wide.load_program("CCNOT 0 1 2\nCCNOT 0 1 2\n")
+    wide.run()
+    assert StandIn.made == 3
+    wide.close()
