@@ -191,11 +191,13 @@ int launch_kraus_run(qvmhip_state *s, uint32_t nq, uint32_t nmaps, const uint32_
 // A run of 1-qubit gates on a pure state (a sweep of 73 us each at 2^24 FP64
 // amplitudes), multiplied together per qubit and applied up to eleven qubits a
 // pass.  normalize, for unitary gates: the state ends with norm 1; its norm is
-// read before the last pass, whose first matrix takes the factor.
+// read before the last pass, whose first matrix takes the factor.  A norm that
+// cannot be divided by is found there too: the run is finished without the factor
+// and reported, as by gate after gate and a normalization that is refused.
 int launch_1q_run(qvmhip_state *s, uint32_t count, const uint32_t *qubits, const double *U, bool normalize) {
     std::vector<std::vector<cd>> S(s->n);
     const cd *u = reinterpret_cast<const cd *>(U);
-    bool finite = true;
+    bool fits = true;
     for (uint32_t i = 0; i < count; ++i, u += 4) {
         std::vector<cd> &B = S[qubits[i]];
         if (B.empty()) {
@@ -204,28 +206,41 @@ int launch_1q_run(qvmhip_state *s, uint32_t count, const uint32_t *qubits, const
         }
         const cd P[4] = {u[0] * B[0] + u[1] * B[2], u[0] * B[1] + u[1] * B[3], u[2] * B[0] + u[3] * B[2],
                          u[2] * B[1] + u[3] * B[3]};
-        for (const cd &x : P) finite = finite && std::isfinite(x.real()) && std::isfinite(x.imag());
         B.assign(P, P + 4);
+        fits = fits && in_range(s, B);
     }
-    if (!finite) return fail(QVMHIP_ERANGE, "the product of the run's gates is not finite");
     std::vector<uint32_t> on;
     for (uint32_t q = 0; q < s->n; ++q)
         if (!S[q].empty()) on.push_back(q);
+    bool normalized = true;
     auto scale = [&](std::vector<cd> &A) -> int {
         double n2 = 0;
         if (const int rc = reduce_norm2(s, &n2)) return rc;
         const double len = std::sqrt(n2);
-        if (!(len > 0) || !std::isfinite(len)) return fail(QVMHIP_ERANGE, "cannot normalize a zero/non-finite state");
-        for (cd &x : A) x *= 1.0 / len;
+        normalized = len > 0 && std::isfinite(len);
+        for (cd &x : A) x *= normalized ? 1.0 / len : 1.0;
         return QVMHIP_OK;
     };
+    auto done = [&] {
+        return normalized ? QVMHIP_OK : fail(QVMHIP_ERANGE, "cannot normalize a zero/non-finite state");
+    };
+    if (!fits) {  // a product past the range: gate by gate, as given
+        u = reinterpret_cast<const cd *>(U);
+        for (uint32_t i = 0; i < count; ++i, u += 4) {
+            std::vector<cd> A(u, u + 4);
+            if (normalize && i + 1 == count)
+                if (const int rc = scale(A)) return rc;
+            if (const int rc = launch_gate(s, reinterpret_cast<const double *>(A.data()), 1, qubits + i, 0)) return rc;
+        }
+        return done();
+    }
     if (on.size() < 2 || s->n < 8) {
         for (uint32_t q : on) {
             if (normalize && q == on.back())
                 if (const int rc = scale(S[q])) return rc;
             if (const int rc = launch_gate(s, reinterpret_cast<const double *>(S[q].data()), 1, &q, 0)) return rc;
         }
-        return QVMHIP_OK;
+        return done();
     }
     for (size_t i = 0; i < on.size();) {
         TileGroup g(s, on, i, 0);
@@ -247,7 +262,7 @@ int launch_1q_run(qvmhip_state *s, uint32_t count, const uint32_t *qubits, const
         }
         if (const int rc = launch_tile_pass_async(s, g.m, g.tq, (uint32_t)ops.size(), ops.data())) return rc;
     }
-    return QVMHIP_OK;
+    return done();
 }
 
 // Operators per read: every one adds 2^k complex products per amplitude.  Four

@@ -137,7 +137,8 @@ class HipPureState:
     def apply_1q_run(self, mats, qubits, normalize: bool = False) -> None:
         """The 1-qubit gates mats[i] on qubits[i], in order, as apply_matrix one
         after another up to rounding, in shared sweeps; ``normalize`` (for
-        unitary gates) also divides the state by its norm."""
+        unitary gates) also divides the state by its norm, and raises with the
+        gates applied when that is zero or not finite."""
         U, q = N.cmat(mats), N.u32arr(qubits)
         if U.shape != (len(q), 2, 2):
             raise ValueError(f"matrices of shape {U.shape} for {len(q)} 1-qubit gates")

@@ -295,6 +295,43 @@ def test_noisy_runs_match_one_by_one(dtype, n):
         assert abs(np.linalg.norm(a) - 1) <= (4 * n + 10) * 8 * u
 
 
+@pytest.mark.parametrize("n", [1, 5, 9, 13])
+def test_1q_run_whose_norm_is_not_finite_is_applied_whole(n):
+    """Amplitudes of 1e200 have no finite norm: the run reports it, after one
+    gate, in sweeps, in one pass and in two, with every gate applied.  Bound: two
+    roundings of the entry and one of the sum per gate."""
+    from qvm_amd import _native as N
+    from qvm_amd.state import HipPureState
+    H = G.gate_matrix("H")
+    with HipPureState(n) as st:
+        psi = np.zeros(1 << n, dtype=np.complex128)
+        psi[0] = 1e200
+        st.write_amplitudes(psi)
+        with pytest.raises(N.QVMHipError) as e:
+            st.apply_1q_run([H] * n, list(range(n)), normalize=True)
+        assert e.value.code == N.ERANGE
+        want = 1e200 * 2.0 ** (-n / 2)
+        assert np.max(np.abs(st.amplitudes() - want)) <= 3 * n * 2.0 ** -53 * want
+
+
+@pytest.mark.parametrize("dtype,big,small", [("f64", 1e200, 1e-300), ("f32", 1e25, 1e-30)])
+@pytest.mark.parametrize("n", [3, 9])
+def test_1q_run_whose_product_overflows(dtype, big, small, n):
+    """Two gates on one qubit whose product is past the range go gate by
+    gate: the same bits as apply_matrix."""
+    from qvm_amd.state import HipPureState
+    mats = [np.diag([big, 1]), G.gate_matrix("H"), np.diag([big, 1j]), np.diag([1 / big, 1])]
+    qubits = [n - 1, 0, n - 1, n - 1]
+    psi = np.arange(1, (1 << n) + 1) * (1 - 2j) * small
+    with HipPureState(n, dtype) as st, HipPureState(n, dtype) as ref:
+        st.write_amplitudes(psi)
+        ref.write_amplitudes(psi)
+        st.apply_1q_run(mats, qubits)
+        for U, q in zip(mats, qubits):
+            ref.apply_matrix(U, [q])
+        assert np.all(np.isfinite(ref.amplitudes())) and np.array_equal(st.amplitudes(), ref.amplitudes())
+
+
 def test_noisy_run_takes_no_draw_for_a_gate_it_does_not_cover():
     """Damping only, a plain matrix that is not unitary, a modifier on a noisy gate."""
     from qvm_amd.noise import NoisyQVM
