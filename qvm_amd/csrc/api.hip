@@ -247,7 +247,7 @@ int qvmhip_apply_fused(qvmhip_state *s, const double *U, uint32_t k, const uint3
     // upload to the matrix slot's second half (first half: ops / dense)
     const std::vector<char> A = fused_operand(s->dtype, U, k, qubits);
     void *dst = (char *)s->mat + kFusedMatOffset;
-    QH_CHECK(hipMemcpyAsync(dst, A.data(), A.size(), hipMemcpyHostToDevice, s->stream));
+    if (const int up = upload_operand(s, dst, A.data(), A.size())) return up;
     return launch_fused_dense(s, dst, k, qubits);
 }
 

@@ -85,7 +85,7 @@ int launch_kraus(qvmhip_state *s, uint32_t nq, const double *K, uint32_t count, 
     if (k == 1 || !gate_is_dense(m, 2 * k, q)) return launch_gate(s, m, 2 * k, q, 0);
     const std::vector<char> A = fused_operand(s->dtype, m, 2 * k, q);
     void *dst = (char *)s->mat + kFusedMatOffset;
-    QH_CHECK(hipMemcpyAsync(dst, A.data(), A.size(), hipMemcpyHostToDevice, s->stream));
+    if (const int rc = upload_operand(s, dst, A.data(), A.size())) return rc;
     return launch_fused_dense(s, dst, 2 * k, q);
 }
 
@@ -183,7 +183,7 @@ int launch_kraus_run(qvmhip_state *s, uint32_t nq, uint32_t nmaps, const uint32_
             }
             ops.push_back(op);
         }
-        if (const int rc = launch_tile_pass_async(s, g.m, g.tq, (uint32_t)ops.size(), ops.data())) return rc;
+        if (const int rc = launch_tile_pass(s, g.m, g.tq, (uint32_t)ops.size(), ops.data())) return rc;
     }
     return QVMHIP_OK;
 }
@@ -260,7 +260,7 @@ int launch_1q_run(qvmhip_state *s, uint32_t count, const uint32_t *qubits, const
             }
             ops.push_back(op);
         }
-        if (const int rc = launch_tile_pass_async(s, g.m, g.tq, (uint32_t)ops.size(), ops.data())) return rc;
+        if (const int rc = launch_tile_pass(s, g.m, g.tq, (uint32_t)ops.size(), ops.data())) return rc;
     }
     return done();
 }

@@ -898,8 +898,7 @@ int run_dense_big(qvmhip_state *s, const GateSplit &gs) {
             host[c * D + r] = (T)gs.V[r * D + c].real();
             host[D * D + c * D + r] = (T)gs.V[r * D + c].imag();
         }
-    QH_CHECK(hipMemcpyAsync(s->mat, host.data(), host.size() * sizeof(T), hipMemcpyHostToDevice,
-                            s->stream));
+    if (const int rc = upload_operand(s, s->mat, host.data(), host.size() * sizeof(T))) return rc;
     const uint64_t gpb = kBlock / D;
     const uint64_t nbatch = (g.ngroups + gpb - 1) / gpb;
     const uint32_t grid = (uint32_t)std::min<uint64_t>(nbatch, 256 * 16);

@@ -1607,31 +1607,8 @@ int launch_tile_code(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, c
                                   : run_tile_m<float>(s, m, tile_qubits, dev, cut);
 }
 
-int launch_tile_pass(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, uint32_t nops,
-                     const qvmhip_tile_op *ops) {
-    const TileCode code = compile_tile_ops(s->dtype, (s->flags & QVMHIP_FLAG_FMA_TILES) != 0, m, ops, nops);
-    // Operands go through the matrix slot's first half (64 KiB, some 800
-    // ops); longer lists get a temporary buffer released after the stream
-    // drains.  The copy is ordered on the stream after every earlier reader.
-    void *dev = s->mat, *tmp = nullptr;
-    if (code.bytes.size() > kFusedMatOffset) {
-        QH_CHECK(hipMalloc(&tmp, code.bytes.size()));
-        dev = tmp;
-    }
-    hipError_t e = hipMemcpyAsync(dev, code.bytes.data(), code.bytes.size(), hipMemcpyHostToDevice, s->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);  // code is a host temporary
-    const int rc = e == hipSuccess ? launch_tile_code(s, m, tile_qubits, dev, code.cut)
-                                   : fail(QVMHIP_EDEVICE, std::string("tile ops upload: ") + hipGetErrorString(e));
-    if (tmp) {
-        (void)hipStreamSynchronize(s->stream);
-        (void)hipFree(tmp);
-    }
-    return rc;
-}
-
-// An op list travels to the state's operand slot in the arguments of small
-// launches, which are copied when they are enqueued: no host buffer has to
-// outlive the call, and the host does not wait.
+// A short op list travels to the state's operand slot in the arguments of
+// small launches, which are copied when they are enqueued.
 struct OpChunk {
     uint4 w[192];
 };
@@ -1639,19 +1616,37 @@ __global__ __launch_bounds__(192) void k_put_ops(uint4 *__restrict__ dst, const 
     if (threadIdx.x < n) dst[threadIdx.x] = c.w[threadIdx.x];
 }
 
-int launch_tile_pass_async(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, uint32_t nops,
-                           const qvmhip_tile_op *ops) {
+int launch_tile_pass(qvmhip_state *s, uint32_t m, const uint32_t *tile_qubits, uint32_t nops,
+                     const qvmhip_tile_op *ops) {
     const TileCode code = compile_tile_ops(s->dtype, (s->flags & QVMHIP_FLAG_FMA_TILES) != 0, m, ops, nops);
-    if (code.bytes.size() > kFusedMatOffset) return launch_tile_pass(s, m, tile_qubits, nops, ops);
-    for (size_t off = 0; off < code.bytes.size(); off += sizeof(OpChunk)) {
-        const size_t n = std::min(sizeof(OpChunk), code.bytes.size() - off);  // slots: a multiple of 16 bytes
-        OpChunk c;
-        std::memcpy(&c, code.bytes.data() + off, n);
-        hipLaunchKernelGGL(k_put_ops, dim3(1), dim3(192), 0, s->stream, (uint4 *)((char *)s->mat + off), c,
-                           (uint32_t)(n / 16));
-        QH_LAUNCH_CHECK();
+    // Operands go through the matrix slot's first half (64 KiB, some 800
+    // ops), ordered on the stream after every earlier reader: up to two chunks
+    // (6 KiB, some 75 ops) by launches, which cost 3 us each where a copy costs
+    // 10; longer lists get a temporary buffer released after the stream drains.
+    const size_t bytes = code.bytes.size();
+    if (bytes <= 2 * sizeof(OpChunk)) {
+        for (size_t off = 0; off < bytes; off += sizeof(OpChunk)) {
+            const size_t n = std::min(sizeof(OpChunk), bytes - off);  // slots: a multiple of 16 bytes
+            OpChunk c;
+            std::memcpy(&c, code.bytes.data() + off, n);
+            hipLaunchKernelGGL(k_put_ops, dim3(1), dim3(192), 0, s->stream, (uint4 *)((char *)s->mat + off), c,
+                               (uint32_t)(n / 16));
+            QH_LAUNCH_CHECK();
+        }
+        return launch_tile_code(s, m, tile_qubits, s->mat, code.cut);
     }
-    return launch_tile_code(s, m, tile_qubits, s->mat, code.cut);
+    void *dev = s->mat, *tmp = nullptr;
+    if (bytes > kFusedMatOffset) {
+        QH_CHECK(hipMalloc(&tmp, bytes));
+        dev = tmp;
+    }
+    int rc = upload_operand(s, dev, code.bytes.data(), bytes);
+    if (!rc) rc = launch_tile_code(s, m, tile_qubits, dev, code.cut);
+    if (tmp) {
+        (void)hipStreamSynchronize(s->stream);
+        (void)hipFree(tmp);
+    }
+    return rc;
 }
 
 size_t tile_entry_bytes() { return sizeof(TileEntry); }
