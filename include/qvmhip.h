@@ -181,8 +181,8 @@ QVMHIP_API int qvmhip_norm(qvmhip_state *s, double *out);
  * (src/apply-gate.lisp:16-39). */
 QVMHIP_API int qvmhip_total_probability(qvmhip_state *s, double *out);
 /* A run of 1-qubit gates, gate i with the 2x2 matrix U + 8*i on qubits[i], in
- * order: qvmhip_apply_matrix per gate up to rounding (gates on one qubit are
- * multiplied together, gates on different qubits share sweeps).  normalize != 0,
+ * order: qvmhip_apply_matrix per gate up to rounding, on finite amplitudes (gates
+ * on one qubit are multiplied together, gates on different qubits share sweeps).  normalize != 0,
  * for unitary gates: the state is also divided by its norm; when that is zero or
  * not finite, QVMHIP_ERANGE, with the gates applied. */
 QVMHIP_API int qvmhip_apply_1q_run(qvmhip_state *s, uint32_t count, const uint32_t *qubits, const double *U,

@@ -266,9 +266,11 @@ int launch_1q_run(qvmhip_state *s, uint32_t count, const uint32_t *qubits, const
 }
 
 // Operators per read: every one adds 2^k complex products per amplitude.  Four
-// 1-qubit or two 2-qubit operators stay under the time of the read (2^24 FP64
-// amplitudes: 4 x 18 or 2 x 30 FP64 operations per amplitude, about 30 us of
-// issue against 45 us).
+// 1-qubit operators stay under the time of the read (2^24 FP64 amplitudes: 4 x 18
+// FP64 operations per amplitude, about 30 us of issue against 45 us).  Two 2-qubit
+// ones do not: their 64 FP64 coefficients do not fit the scalar registers (115
+// spills, 106 VGPRs, four waves per SIMD), and the read takes 57 us where the
+// 1-qubit form takes 40.
 constexpr int kraus_per_read(int k) { return k == 1 ? 4 : 2; }
 constexpr int kNormBlocks = 1024;  // partials of kNormBlocks * 4 sums fit the state's reduction scratch
 static_assert(kNormBlocks * 4 <= kRedBlocks * 2, "reduction scratch");

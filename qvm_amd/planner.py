@@ -320,8 +320,8 @@ def _kind_1q(U: np.ndarray) -> str:
 
 
 # Relative cost of one tile op per kind in FMA passes, from per-op timings at
-# n = 30 (FP64: general U3 0.27-0.29 ms, RX 0.12-0.14, RZ 0 on a register bit
-# and 0.19 on a lane bit).
+# n = 30 (us, FP64 / FP32: general U3 220 / 120, RX and H 110 / 56, RZ 0 on a
+# register bit and 174 / 74 on a lane bit).
 _COST_1Q = {"diag": 0.8, "reduced": 1.0, "general": 2.2}
 
 
@@ -331,9 +331,9 @@ def _merge_runs_1q(gates: List[Gate]) -> List[Gate]:
     keeping them apart: RX then RZ stay two ops (a reduced op and a
     diagonal, which the FMA scheduler folds into the register diagonals)
     instead of one general op, while runs of general gates become one.
-    Measured at n = 30 (FMA passes, ms): layered-40 FP64 759.7 merged / 728.2
-    kept apart, FP32 442.8 / 398.2; random 60 % U3 / 40 % CNOT-CZ FP64 230.0 /
-    286.5, FP32 121.8 / 159.6."""
+    Measured at n = 30 (FMA passes, ms): layered-40 FP64 563.7 merged / 520.5
+    kept apart, FP32 285.1 / 262.5; random 60 % U3 / 40 % CNOT-CZ FP64 169.3 /
+    207.3, FP32 82.3 / 104.5."""
     # pending[q] = index in `merged` of the open 1-qubit run on q; a gate on
     # q with more qubits closes the run.
     merged: List[Gate] = []
