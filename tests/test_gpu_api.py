@@ -216,3 +216,26 @@ def test_noisy_qvm_gates_and_readout():
     with pytest.raises(Exception):
         q.set_noisy_gate("H", [1], [np.eye(2) * 0.5])
     q.close()
+
+
+@pytest.mark.parametrize("dtype,over", [("f64", 2.0 ** -52), ("f64", 2.0 ** -41), ("f32", 2.0 ** -23), ("f32", 2.0 ** -12)])
+def test_a_probability_a_few_roundings_above_one_is_one(dtype, over):
+    """A qubit that is certainly 1 on a state whose norm rounding left above 1
+    is measured; a state that is not normalized stays refused."""
+    from qvm_amd import _native as N
+    from qvm_amd.qvm import make_qvm
+    q = make_qvm(3, dtype=dtype, rng=lambda: 0.75)
+    q.load_program("DECLARE ro BIT[2]\nMEASURE 1 ro[1]\nMEASURE 0 ro[0]\nX 1\nRESET 1\n")
+    for amp, ok in ((1 + over, True), (1.5, False)):
+        psi = np.zeros(8, dtype=np.complex128)
+        psi[2] = amp
+        q.set_amplitudes(psi)
+        assert q.state.prob_excited(1) > 1
+        if ok:
+            q.run()
+            assert list(q.memory["ro"]) == [0, 1]
+        else:
+            with pytest.raises(N.QVMHipError) as e:
+                q.run()
+            assert e.value.code == N.ERANGE and q.pc == 0
+    q.close()
